@@ -86,7 +86,8 @@ __device__ __forceinline__ void boids_pair(const float4 p, const float4 q, const
   // vec / squaredDist: sq lies in (1e-8, radiusSq] with radiusSq <= 2^30 (checked on the
   // host), so the short division applies unless a numerator is a nonzero value under 2^-90
   const float y = rcp_refined(sq);
-  float qx = div_short(vx, sq, y), qy = div_short(vy, sq, y), qz = div_short(vz, sq, y);
+  float qx = div_unsigned_zero(vx, sq, y), qy = div_unsigned_zero(vy, sq, y),
+        qz = div_unsigned_zero(vz, sq, y);
   const bool general = !c.shortDiv || tiny_numerator3(vx, vy, vz);
   if (__builtin_amdgcn_ballot_w64(general) != 0) {
     rare_path();
@@ -394,7 +395,8 @@ __device__ __forceinline__ void boids_pair_quad(bool v, const float4 p, const fl
   const float vx = p.x - q.x, vy = p.y - q.y, vz = p.z - q.z;
   const float sq = vx * vx + vy * vy + vz * vz;
   const float y = rcp_refined(sq);
-  float qx = div_short(vx, sq, y), qy = div_short(vy, sq, y), qz = div_short(vz, sq, y);
+  float qx = div_unsigned_zero(vx, sq, y), qy = div_unsigned_zero(vy, sq, y),
+        qz = div_unsigned_zero(vz, sq, y);
   const bool general = !c.shortDiv || tiny_numerator3(vx, vy, vz);
   if (__builtin_amdgcn_ballot_w64(general) != 0) {
     rare_path();

@@ -102,38 +102,40 @@ __device__ __forceinline__ float4 grad_spiky_r(float4 vec, float r, const PbfCon
 // length(vec) from d2 = dot4(vec, vec): sqrt_cr returns sqrtf's bits for every d2 >= 0.
 __device__ __forceinline__ float len_of(float d2) { return sqrt_cr(d2); }
 
-__device__ __forceinline__ bool tiny_numerator4(float a, float b, float c, float d)
+// The length and spiky gradient of a pair: r = sqrtf(vv) for vv = dot4(vec, vec) and g =
+// grad_spiky_r(vec, r, c), a zero component of g in either sign.  The short correctly rounded
+// root and quotients serve pairs with kFloatEps < r < h under the shortMath bit (with t = 1 -
+// step(h, r) = 1 the factor t is an exact identity) and d2 = 0; the w lane, whose positions
+// carry w = 0, is +-0 and its own quotient.  The other lanes (nonzero vv under 2^-52, a
+// nonzero numerator under 2^-90, a root whose significand is all ones, r >= h, NaN) take the
+// general expressions.
+constexpr uint32_t kNearVv = 0x25800000u;  // 2^-52
+struct CldPair {
+  float r;
+  float4 g;
+};
+__device__ __forceinline__ CldPair cld_pair(float4 vec, float vv, const PbfConsts& c)
 {
-  return tiny_numerator3(a, b, c) || num_key(d) < (kDivNumMin << 1) - 2u;
-}
-
-// grad_spiky_r with the short correctly rounded division where its operand ranges hold
-// (the shortMath bit: kFloatEps < r < h, every numerator +-0 or not tiny): the four
-// quotients by r share one refined reciprocal.  With t = 1 - step(h, r) = 1 the factor t
-// is an exact identity.  Other lanes take the general expression.
-__device__ __forceinline__ float4 grad_spiky_fast(float4 vec, float r, const PbfConsts& c)
-{
-  const bool in = (c.shortMath & kShortSqrtGrad) != 0 && r < c.h;
-  float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  float4 n = g;
-  bool general = !in;
-  if (in) {
-    const float p2 = (c.h - r) * (c.h - r);
-    n = make_float4(((vec.x * c.spiky) * -3.0f) * p2, ((vec.y * c.spiky) * -3.0f) * p2,
-                    ((vec.z * c.spiky) * -3.0f) * p2, ((vec.w * c.spiky) * -3.0f) * p2);
-    const float yr = rcp_refined(r);
-    const bool on = r > kFloatEps;
-    if (on)
-      g = make_float4(div_short(n.x, r, yr), div_short(n.y, r, yr), div_short(n.z, r, yr),
-                      div_short(n.w, r, yr));
-    general = on && tiny_numerator4(n.x, n.y, n.z, n.w);
-  }
+  const Root q = root_short(vv);
+  CldPair o;
+  o.r = q.r;
+  const float p2 = (c.h - q.r) * (c.h - q.r);
+  const float4 n = make_float4(((vec.x * c.spiky) * -3.0f) * p2, ((vec.y * c.spiky) * -3.0f) * p2,
+                               ((vec.z * c.spiky) * -3.0f) * p2, ((vec.w * c.spiky) * -3.0f) * p2);
+  const float y = root_rcp(q);
+  o.g = make_float4(div_unsigned_zero(n.x, q.r, y), div_unsigned_zero(n.y, q.r, y),
+                    div_unsigned_zero(n.z, q.r, y), n.w);
+  const bool general = !((c.shortMath & kShortSqrtGrad) != 0 && q.r < c.h) |
+                       (__float_as_uint(vv) - 1u < kNearVv - 1u) | tiny_numerator3(n.x, n.y, n.z) |
+                       ones_significand(q.r);
   if (__builtin_amdgcn_ballot_w64(general) != 0) {
     rare_path();
-    if (general)
-      g = in ? div4s(n, r) : grad_spiky_r(vec, r, c);
+    if (general) {
+      o.r = __builtin_sqrtf(vv);
+      o.g = grad_spiky_r(vec, o.r, c);
+    }
   }
-  return g;
+  return o;
 }
 
 // clouds.cl:106-114 given w = poly6(vec) (poly6L(artPressureRadius * h) is folded into
@@ -142,7 +144,7 @@ __device__ __forceinline__ float art_pressure_w(float w, float ywdq, const PbfCo
 {
   if (c.p.isArtPressureEnabled == 0)
     return 0.0f;
-  const float q = (c.shortMath & kShortArtDiv) ? div_short(w, c.wdq, ywdq) : w / c.wdq;
+  const float q = (c.shortMath & kShortArtDiv) ? div_unsigned_zero(w, c.wdq, ywdq) : w / c.wdq;
   return -c.p.artPressureCoeff * pown(q, c.p.artPressureExp);
 }
 
@@ -818,7 +820,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_temp_lambda(const float4* __r
   cld_walk_record(i, pos, posP, se, c.f.g, lds, list, [&](uint32_t e) { return tempP[e]; }, keep, [&](uint32_t, float te, float4 vec) {
     const float dTemp = temp - te;
     const float vv = dot4(vec, vec);
-    const float4 grad = grad_spiky_fast(vec, len_of(vv), c.f);
+    const float4 grad = cld_pair(vec, vv, c.f).g;
     const float vg = dot4(vec, grad);
     laplacian = laplacian + dTemp * vg / (vv + kFloatEps);
     const float derivativeTemp = vg / (vv * rho0 + kFloatEps);
@@ -853,7 +855,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_temp_correct(const float4* __
                   [&](uint32_t e) { return lambdaT[e]; }, keep, [&](uint32_t, float le, float4 vec) {
     const float l = lambdaI + le;
     const float vv = dot4(vec, vec);
-    const float4 grad = grad_spiky_fast(vec, len_of(vv), c.f);
+    const float4 grad = cld_pair(vec, vv, c.f).g;
     const float derivativeTemp = dot4(vec, grad) / (vv * rho0 + kFloatEps);
     corr = corr + l * derivativeTemp;
   });
@@ -879,9 +881,9 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_density_lambda(const float4* 
   __shared__ CldLds lds;
   const auto keep = [&](int, float4 vec) { return !negligible(vec, c.f); };
   cld_walk_record(i, pos, pred, se, c.f.g, lds, list, [](uint32_t) { return 0; }, keep, [&](uint32_t, int, float4 vec) {
-    const float r = len_of(dot4(vec, vec));
-    fluidDensity = fluidDensity + poly6_r(r, c.f);
-    const float4 grad = grad_spiky_fast(vec, r, c.f);
+    const CldPair q = cld_pair(vec, dot4(vec, vec), c.f);
+    fluidDensity = fluidDensity + poly6_r(q.r, c.f);
+    const float4 grad = q.g;
     sumGradCi = add4(sumGradCi, grad);
     sumSqGradC = sumSqGradC + dot4(grad, grad);
   });
@@ -916,9 +918,9 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_correct(const float4* __restr
   };
   cld_walk_replay(i, pos, pred, se, c.f.g, lds, list, useList && bit && !(*flags & bit),
                   [&](uint32_t e) { return lambda[e]; }, keep, [&](uint32_t, float le, float4 vec) {
-    const float r = len_of(dot4(vec, vec));
-    const float s = lambdaI + le + art_pressure_w(poly6_r(r, c.f), ywdq, c.f);
-    corr = add4(corr, muls4(s, grad_spiky_fast(vec, r, c.f)));
+    const CldPair q = cld_pair(vec, dot4(vec, vec), c.f);
+    const float s = lambdaI + le + art_pressure_w(poly6_r(q.r, c.f), ywdq, c.f);
+    corr = add4(corr, muls4(s, q.g));
   });
   cld_correct_out(i, pos, corr, predOut, totCorr, vel, c);
 }
@@ -955,7 +957,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_vorticity(const float4* __res
   const auto keep = [&](float4 ve, float4 vec) { return !(negligible(vec, c.f) & finite4(sub4(ve, velocity))); };
   cld_walk_record(i, pos, pred, se, c.f.g, lds, list, [&](uint32_t e) { return vel[e]; }, keep, [&](uint32_t, float4 ve, float4 vec) {
     const float4 dv = sub4(ve, velocity);
-    w = add4(w, cross4(dv, grad_spiky_fast(vec, len_of(dot4(vec, vec)), c.f)));
+    w = add4(w, cross4(dv, cld_pair(vec, dot4(vec, vec), c.f).g));
   });
   vort[i] = w;
   cld_flag(cld_safe(w), flags, kFlagVort);
@@ -985,7 +987,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_confinement(const float4* __r
   cld_walk_replay(i, pos, pred, se, c.f.g, lds, list, useList && !(*flags & kFlagVort),
                   [&](uint32_t e) { return vort[e]; }, keep, [&](uint32_t, float4 we, float4 vec) {
     const float lw = len_of(dot4(we, we));
-    nn = add4(nn, muls4(lw, grad_spiky_fast(vec, len_of(dot4(vec, vec)), c.f)));
+    nn = add4(nn, muls4(lw, cld_pair(vec, dot4(vec, vec), c.f).g));
   });
   const float4 vo = cld_confinement_out(i, nn, vorticity, vel, velOut, c);
   cld_flag(cld_safe(vo), flags, kFlagVelTmp);
@@ -1062,7 +1064,7 @@ struct CqTempLambda {
   {
     const float dTemp = temp - te;
     const float vv = dot4(vec, vec);
-    const float4 grad = grad_spiky_fast(vec, len_of(vv), c.f);
+    const float4 grad = cld_pair(vec, vv, c.f).g;
     const float vg = dot4(vec, grad);
     const float lapTerm = dTemp * vg / (vv + kFloatEps);
     const float derivativeTemp = vg / (vv * rho0 + kFloatEps);
@@ -1086,7 +1088,7 @@ struct CqTempCorrect {
   {
     const float l = lambdaI + le;
     const float vv = dot4(vec, vec);
-    const float4 grad = grad_spiky_fast(vec, len_of(vv), c.f);
+    const float4 grad = cld_pair(vec, vv, c.f).g;
     const float derivativeTemp = dot4(vec, grad) / (vv * rho0 + kFloatEps);
     corr = quad_add(corr, v ? l * derivativeTemp : 0.0f);
   }
@@ -1101,9 +1103,9 @@ struct CqDensity {
   __device__ __forceinline__ bool keep(int, float4 vec) const { return !negligible(vec, c.f); }
   __device__ __forceinline__ void add(bool v, int, float4 vec)
   {
-    const float r = len_of(dot4(vec, vec));
-    const float w = poly6_r(r, c.f);
-    const float4 grad = grad_spiky_fast(vec, r, c.f);
+    const CldPair q = cld_pair(vec, dot4(vec, vec), c.f);
+    const float w = poly6_r(q.r, c.f);
+    const float4 grad = q.g;
     const float sq = dot4(grad, grad);
     fluidDensity = quad_add(fluidDensity, v ? w : 0.0f);
     sumGradCi = quad_add4(sumGradCi, v, grad);
@@ -1123,9 +1125,9 @@ struct CqCorrect {
   }
   __device__ __forceinline__ void add(bool v, float le, float4 vec)
   {
-    const float r = len_of(dot4(vec, vec));
-    const float s = lambdaI + le + art_pressure_w(poly6_r(r, c.f), ywdq, c.f);
-    corr = quad_add4(corr, v, muls4(s, grad_spiky_fast(vec, r, c.f)));
+    const CldPair q = cld_pair(vec, dot4(vec, vec), c.f);
+    const float s = lambdaI + le + art_pressure_w(poly6_r(q.r, c.f), ywdq, c.f);
+    corr = quad_add4(corr, v, muls4(s, q.g));
   }
 };
 
@@ -1142,7 +1144,7 @@ struct CqVorticity {
   __device__ __forceinline__ void add(bool v, float4 ve, float4 vec)
   {
     const float4 dv = sub4(ve, velocity);
-    w = quad_add4(w, v, cross4(dv, grad_spiky_fast(vec, len_of(dot4(vec, vec)), c.f)));
+    w = quad_add4(w, v, cross4(dv, cld_pair(vec, dot4(vec, vec), c.f).g));
   }
 };
 
@@ -1158,7 +1160,7 @@ struct CqConfinement {
   __device__ __forceinline__ void add(bool v, float4 we, float4 vec)
   {
     const float lw = len_of(dot4(we, we));
-    nn = quad_add4(nn, v, muls4(lw, grad_spiky_fast(vec, len_of(dot4(vec, vec)), c.f)));
+    nn = quad_add4(nn, v, muls4(lw, cld_pair(vec, dot4(vec, vec), c.f).g));
   }
 };
 

@@ -532,29 +532,46 @@ __device__ __forceinline__ float poly6_in(float r, const PbfConsts& c)
   return c.poly6 * cube(c.hh - r * r);
 }
 
-// gradSpiky for kFloatEps < r < h, as grad_spiky(dx, dy, dz, r, 1, c); yr = rcp_refined(r).
-// Lanes with a nonzero numerator under 2^-90 take the general division.
-__device__ __forceinline__ Grad grad_spiky_in(float dx, float dy, float dz, float r, float yr,
+// The distance and spiky gradient of a pair, for kShortSqrtGrad: r = sqrtf(d2) and g = gradSpiky
+// (as grad_spiky(dx, dy, dz, r, 1, c), +-0 for r <= kFloatEps) where `in` (r < h).  With the
+// rooted reciprocal, one remainder correction a quotient and one test for all rare operands a
+// pair's root, reciprocal and quotients take about 20 issue slots fewer than with separate
+// v_sqrt and v_rcp forms.  The general forms serve lanes with a nonzero d2 under 2^-52 (which
+// covers 0 < r <= kFloatEps and the roots' own 2^-96), a nonzero numerator under 2^-90, or a
+// root whose significand is all ones; d2 = 0 gives numerators +-0 and quotients +-0.
+constexpr uint32_t kNearD2 = 0x25800000u;  // 2^-52
+struct PairGrad {
+  float r;
+  bool in;
+  Grad g;
+};
+__device__ __forceinline__ PairGrad pair_grad(float dx, float dy, float dz, float d2,
                                               const PbfConsts& c)
 {
-  const float p2 = (c.h - r) * (c.h - r);
+  const Root q = root_short(d2);
+  PairGrad o;
+  o.r = q.r;
+  const float p2 = (c.h - q.r) * (c.h - q.r);
   const float nx = ((dx * c.spiky) * -3.0f) * p2;
   const float ny = ((dy * c.spiky) * -3.0f) * p2;
   const float nz = ((dz * c.spiky) * -3.0f) * p2;
-  Grad g;
-  g.x = div_short(nx, r, yr);
-  g.y = div_short(ny, r, yr);
-  g.z = div_short(nz, r, yr);
-  const bool general = tiny_numerator3(nx, ny, nz);
+  const float y = root_rcp(q);
+  o.g.x = div_unsigned_zero(nx, q.r, y);
+  o.g.y = div_unsigned_zero(ny, q.r, y);
+  o.g.z = div_unsigned_zero(nz, q.r, y);
+  const bool general = (__float_as_uint(d2) - 1u < kNearD2 - 1u) | tiny_numerator3(nx, ny, nz) |
+                       ones_significand(q.r);
   if (__builtin_amdgcn_ballot_w64(general) != 0) {
     rare_path();
     if (general) {
-      g.x = nx / r;
-      g.y = ny / r;
-      g.z = nz / r;
+      o.r = __builtin_sqrtf(d2);
+      o.g = Grad{ 0.0f, 0.0f, 0.0f };
+      if (o.r > kFloatEps)
+        o.g = grad_spiky(dx, dy, dz, o.r, 1.0f, c);
     }
   }
-  return g;
+  o.in = o.r < c.h;
+  return o;
 }
 
 // pown for the exponent of the dam-break parameters without the loop.
@@ -570,7 +587,7 @@ __device__ __forceinline__ float art_pressure_in(float w, float ywdq, const PbfC
 {
   if (c.p.isArtPressureEnabled == 0)
     return 0.0f;
-  const float q = (c.shortMath & kShortArtDiv) ? div_short(w, c.wdq, ywdq) : w / c.wdq;
+  const float q = (c.shortMath & kShortArtDiv) ? div_unsigned_zero(w, c.wdq, ywdq) : w / c.wdq;
   return -c.p.artPressureCoeff * pown_art(q, c.p.artPressureExp);
 }
 
@@ -646,25 +663,27 @@ __device__ __forceinline__ void density_lambda_body(uint32_t i, const float4* __
   const bool fast = (c.shortMath & kShortSqrtGrad) != 0;
   walk27<CL, (MODE & (kNbRecord | kNbReplay))>(p, pred, se, c, [](uint32_t) { return 0; },
              [&](uint32_t, int, float dx, float dy, float dz, float d2) {
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
-    if (fast && r < c.h) {
-      // gradient zero (and nothing added) for r <= kFloatEps; adding +0 changes no sum
-      dens = dens + poly6_in(r, c);
-      if (MODE & kFeatures)
-        count += 1.0f;
-      if (!(MODE & kDensOnly)) {
-        Grad g = grad_spiky_in(dx, dy, dz, r, rcp_refined(r), c);
-        const bool on = r > kFloatEps;
-        g.x = on ? g.x : 0.0f;
-        g.y = on ? g.y : 0.0f;
-        g.z = on ? g.z : 0.0f;
-        sgx = sgx + g.x;
-        sgy = sgy + g.y;
-        sgz = sgz + g.z;
-        ssq = ssq + (g.x * g.x + g.y * g.y + g.z * g.z);
+    if ((MODE & kDensOnly) && fast) {
+      const float r = sqrt_cr(d2);
+      if (r < c.h) {
+        dens = dens + poly6_in(r, c);
+        return;
       }
-      return;
+    } else if (fast) {
+      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
+      if (q.in) {
+        dens = dens + poly6_in(q.r, c);
+        if (MODE & kFeatures)
+          count += 1.0f;
+        // gradient +-0 for r <= kFloatEps (the reference adds nothing): no sum changes
+        sgx = sgx + q.g.x;
+        sgy = sgy + q.g.y;
+        sgz = sgz + q.g.z;
+        ssq = ssq + (q.g.x * q.g.x + q.g.y * q.g.y + q.g.z * q.g.z);
+        return;
+      }
     }
+    const float r = __builtin_sqrtf(d2);
     const float t = r < c.h ? 1.0f : 0.0f;
     dens = dens + poly6(r, t, c);
     if (MODE & kFeatures)
@@ -800,17 +819,17 @@ __device__ __forceinline__ void correct_body(uint32_t i, const float4* __restric
   const float ywdq = (c.shortMath & kShortArtDiv) ? rcp_refined(c.wdq) : 0.0f;
   walk27<CL, (MODE & (kNbRecord | kNbReplay))>(p, pred, se, c, [&](uint32_t e) { return lambda[e]; },
              [&](uint32_t, float le, float dx, float dy, float dz, float d2) {
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
-    if (fast && r < c.h) {
-      const float s = li + le + art_pressure_in(poly6_in(r, c), ywdq, c);
-      // r <= kFloatEps: gradSpiky is the zero vector
-      const Grad g = grad_spiky_in(dx, dy, dz, r, rcp_refined(r), c);
-      const bool on = r > kFloatEps;
-      cx = cx + s * (on ? g.x : 0.0f);
-      cy = cy + s * (on ? g.y : 0.0f);
-      cz = cz + s * (on ? g.z : 0.0f);
-      return;
+    if (fast) {
+      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
+      if (q.in) {
+        const float s = li + le + art_pressure_in(poly6_in(q.r, c), ywdq, c);
+        cx = cx + s * q.g.x;
+        cy = cy + s * q.g.y;
+        cz = cz + s * q.g.z;
+        return;
+      }
     }
+    const float r = __builtin_sqrtf(d2);
     const float t = r < c.h ? 1.0f : 0.0f;
     const float s = li + le + art_pressure(poly6(r, t, c), c);
     if (r > kFloatEps) {
@@ -1192,18 +1211,21 @@ struct QuadDensity {
   {
     const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
     const float d2 = dx * dx + dy * dy + dz * dz;
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
-    float w, gx = 0.0f, gy = 0.0f, gz = 0.0f, sq = 0.0f;
-    if (fast && r < c.h) {
-      w = poly6_in(r, c);
-      const Grad g = grad_spiky_in(dx, dy, dz, r, rcp_refined(r), c);
-      const bool on = r > kFloatEps;
-      gx = on ? g.x : 0.0f;
-      gy = on ? g.y : 0.0f;
-      gz = on ? g.z : 0.0f;
+    float w = 0.0f, gx = 0.0f, gy = 0.0f, gz = 0.0f, sq = 0.0f;
+    bool done = false;
+    if (fast) {
+      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
+      done = q.in;
+      w = poly6_in(q.r, c);
+      gx = q.g.x;
+      gy = q.g.y;
+      gz = q.g.z;
       sq = gx * gx + gy * gy + gz * gz;
-    } else {
+    }
+    if (!done) {
+      const float r = __builtin_sqrtf(d2);
       const float t = r < c.h ? 1.0f : 0.0f;
+      gx = gy = gz = sq = 0.0f;
       w = poly6(r, t, c);
       if (r > kFloatEps) {  // else the reference adds no gradient: +0 here
         const Grad g = grad_spiky(dx, dy, dz, r, t, c);
@@ -1233,16 +1255,18 @@ struct QuadCorrect {
   {
     const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
     const float d2 = dx * dx + dy * dy + dz * dz;
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
-    float tx, ty, tz;
-    if (fast && r < c.h) {
-      const float s = li + le + art_pressure_in(poly6_in(r, c), ywdq, c);
-      const Grad g = grad_spiky_in(dx, dy, dz, r, rcp_refined(r), c);
-      const bool on = r > kFloatEps;
-      tx = s * (on ? g.x : 0.0f);
-      ty = s * (on ? g.y : 0.0f);
-      tz = s * (on ? g.z : 0.0f);
-    } else {
+    float tx = 0.0f, ty = 0.0f, tz = 0.0f;
+    bool done = false;
+    if (fast) {
+      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
+      done = q.in;
+      const float s = li + le + art_pressure_in(poly6_in(q.r, c), ywdq, c);
+      tx = s * q.g.x;
+      ty = s * q.g.y;
+      tz = s * q.g.z;
+    }
+    if (!done) {
+      const float r = __builtin_sqrtf(d2);
       const float t = r < c.h ? 1.0f : 0.0f;
       const float s = li + le + art_pressure(poly6(r, t, c), c);
       if (r > kFloatEps) {
@@ -1392,17 +1416,19 @@ __device__ __forceinline__ void vorticity_body(uint32_t i, const float4* __restr
   const bool fast = (c.shortMath & kShortSqrtGrad) != 0;
   walk27<false, NB>(p, pred, se, c, [&](uint32_t e) { return vel[e]; },
          [&](uint32_t, const float4 ve, float dx, float dy, float dz, float d2) {
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
-    if (fast && r < c.h) {
-      // nothing is added for r <= kFloatEps
-      const Grad g = grad_spiky_in(dx, dy, dz, r, rcp_refined(r), c);
-      const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
-      const bool on = r > kFloatEps;
-      wx = on ? wx + (ay * g.z - az * g.y) : wx;
-      wy = on ? wy + (az * g.x - ax * g.z) : wy;
-      wz = on ? wz + (ax * g.y - ay * g.x) : wz;
-      return;
+    if (fast) {
+      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
+      if (q.in) {
+        const Grad g = q.g;
+        const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
+        const bool on = q.r > kFloatEps;  // else nothing is added, whatever the velocities
+        wx = on ? wx + (ay * g.z - az * g.y) : wx;
+        wy = on ? wy + (az * g.x - ax * g.z) : wy;
+        wz = on ? wz + (ax * g.y - ay * g.x) : wz;
+        return;
+      }
     }
+    const float r = __builtin_sqrtf(d2);
     if (r > kFloatEps) {
       const float t = r < c.h ? 1.0f : 0.0f;
       const Grad g = grad_spiky(dx, dy, dz, r, t, c);
@@ -1467,16 +1493,17 @@ __device__ __forceinline__ void confinement_body(uint32_t i, const float4* __res
   const bool fast = (c.shortMath & kShortSqrtGrad) != 0;
   walk27<false, NB>(p, pred, se, c, [&](uint32_t e) { return vort[e].w; },
          [&](uint32_t, float l, float dx, float dy, float dz, float d2) {
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
-    if (fast && r < c.h) {
-      // nothing is added for r <= kFloatEps
-      const Grad g = grad_spiky_in(dx, dy, dz, r, rcp_refined(r), c);
-      const bool on = r > kFloatEps;
-      nx = on ? nx + l * g.x : nx;
-      ny = on ? ny + l * g.y : ny;
-      nz = on ? nz + l * g.z : nz;
-      return;
+    if (fast) {
+      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
+      if (q.in) {
+        const bool on = q.r > kFloatEps;  // else nothing is added, whatever l
+        nx = on ? nx + l * q.g.x : nx;
+        ny = on ? ny + l * q.g.y : ny;
+        nz = on ? nz + l * q.g.z : nz;
+        return;
+      }
     }
+    const float r = __builtin_sqrtf(d2);
     if (r > kFloatEps) {
       const float t = r < c.h ? 1.0f : 0.0f;
       const Grad g = grad_spiky(dx, dy, dz, r, t, c);
@@ -1564,23 +1591,28 @@ struct QuadVorticity {
   {
     const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
     const float d2 = dx * dx + dy * dy + dz * dz;
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
     float tx = 0.0f, ty = 0.0f, tz = 0.0f;
-    if (fast && r < c.h) {
-      // nothing is added for r <= kFloatEps
-      const Grad g = grad_spiky_in(dx, dy, dz, r, rcp_refined(r), c);
-      const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
-      const bool on = r > kFloatEps;
+    const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
+    bool done = false;
+    if (fast) {
+      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
+      const Grad g = q.g;
+      done = q.in;
+      const bool on = q.r > kFloatEps;  // else nothing is added, whatever the velocities
       tx = on ? ay * g.z - az * g.y : 0.0f;
       ty = on ? az * g.x - ax * g.z : 0.0f;
       tz = on ? ax * g.y - ay * g.x : 0.0f;
-    } else if (r > kFloatEps) {
+    }
+    if (!done) {
+      const float r = __builtin_sqrtf(d2);
       const float t = r < c.h ? 1.0f : 0.0f;
-      const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-      const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
-      tx = ay * g.z - az * g.y;
-      ty = az * g.x - ax * g.z;
-      tz = ax * g.y - ay * g.x;
+      tx = ty = tz = 0.0f;
+      if (r > kFloatEps) {
+        const Grad g = grad_spiky(dx, dy, dz, r, t, c);
+        tx = ay * g.z - az * g.y;
+        ty = az * g.x - ax * g.z;
+        tz = ax * g.y - ay * g.x;
+      }
     }
     wx = quad_add(wx, v ? tx : 0.0f);
     wy = quad_add(wy, v ? ty : 0.0f);
@@ -1599,21 +1631,26 @@ struct QuadConfinement {
   {
     const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
     const float d2 = dx * dx + dy * dy + dz * dz;
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
     float tx = 0.0f, ty = 0.0f, tz = 0.0f;
-    if (fast && r < c.h) {
-      // nothing is added for r <= kFloatEps
-      const Grad g = grad_spiky_in(dx, dy, dz, r, rcp_refined(r), c);
-      const bool on = r > kFloatEps;
-      tx = on ? l * g.x : 0.0f;
-      ty = on ? l * g.y : 0.0f;
-      tz = on ? l * g.z : 0.0f;
-    } else if (r > kFloatEps) {
+    bool done = false;
+    if (fast) {
+      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
+      done = q.in;
+      const bool on = q.r > kFloatEps;  // else nothing is added, whatever l
+      tx = on ? l * q.g.x : 0.0f;
+      ty = on ? l * q.g.y : 0.0f;
+      tz = on ? l * q.g.z : 0.0f;
+    }
+    if (!done) {
+      const float r = __builtin_sqrtf(d2);
       const float t = r < c.h ? 1.0f : 0.0f;
-      const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-      tx = l * g.x;
-      ty = l * g.y;
-      tz = l * g.z;
+      tx = ty = tz = 0.0f;
+      if (r > kFloatEps) {
+        const Grad g = grad_spiky(dx, dy, dz, r, t, c);
+        tx = l * g.x;
+        ty = l * g.y;
+        tz = l * g.z;
+      }
     }
     nx = quad_add(nx, v ? tx : 0.0f);
     ny = quad_add(ny, v ? ty : 0.0f);

@@ -5,24 +5,30 @@
 // general sequences that handle every input: a square root pre-scales arguments below
 // 2^-96 by 2^32 and patches +-0 / +inf afterwards (v_cmp_class); a division range-reduces
 // both operands with v_div_scale, post-scales in v_div_fmas and patches special cases in
-// v_div_fixup.  Inside the ranges below those steps are identities, and what is left is
-// the same instruction sequence written out here, so these functions return the same bits
-// as sqrtf / '/' (checked on the GPU against the compiled general forms: every float for
-// the square root, every pair of significands for the division; rtp_selfcheck_*):
+// v_div_fixup.  Inside the ranges below the following shorter sequences return the same bits
+// (checked on the GPU against the compiled general forms: every float for the square root and
+// its reciprocal, every pair of significands for the division; rtp_selfcheck_*):
 //
-//   square root (result s0 = v_sqrt_f32(x) corrected by one ulp either way from the
-//   signs of the residuals x - s*(s -+ ulp)), for x = +-0, x >= 2^-96, +inf or NaN;
+//   square root: y = v_rsq_f32(x), s0 = x*y, s = s0 + (x - s0*s0)*(y/2), for x = 0 (y is
+//   taken of 2^-96 there), x >= 2^-96 or NaN;
 //
-//   division n / d for d > 0 (Newton-Raphson reciprocal refinement followed by two
-//   remainder corrections, the FMA division of Markstein, IBM J. Res. Dev. 34(1), 1990):
-//     y0 = rcp(d), y = y0 + (1 - d*y0)*y0,
-//     q0 = n*y, q1 = q0 + (n - d*q0)*y, q = q1 + (n - d*q1)*y,
-//   the sign taken from n as v_div_fixup does, for d in [2^-40, 2^40] and n = +-0 or
-//   |n| in [2^-90, 2^50] with |n|/d in [2^-120, 2^90]: operands and quotient normal, the
-//   remainders multiples of 2^(e(n) - 46) >= 2^-136 and so exact even where they are
-//   denormal, and exponent differences below the 96 at which v_div_scale starts scaling.
+//   reciprocal of a divisor d > 0 in [2^-40, 2^40]: y0 = rcp(d), y = y0 + (1 - d*y0)*y0,
+//   which is the correctly rounded 1/d for every significand.  The same step from y0 =
+//   v_rsq_f32(x) gives the correctly rounded reciprocal of s = sqrtf(x) except where the
+//   significand of s is all ones (there the step's tie goes the wrong way);
+//
+//   division n / d by such a reciprocal: q0 = n*y, q = q0 + (n - d*q0)*y (Markstein, IBM J.
+//   Res. Dev. 34(1), 1990: one remainder correction is enough when y is the correctly
+//   rounded reciprocal), for d in [2^-40, 2^40] and n = +-0 or |n| in [2^-90, 2^50] with
+//   |n|/d in [2^-120, 2^90]: operands and quotient normal, the remainder a multiple of
+//   2^(e(n) - 46) >= 2^-136 and so exact even where it is denormal, and exponent differences
+//   below the 96 at which v_div_scale starts scaling.
 //
 // The reciprocal y depends on d alone, so divisions by one divisor share it.
+//
+// Issue slots of one lane's pair (a quarter-rate v_rsq, v_rcp or v_sqrt counts four): square
+// root, reciprocal and three quotients 44 with v_sqrt and its two one-ulp residual tests, a
+// v_rcp and two remainder corrections a quotient, 24 in these forms.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -41,29 +47,45 @@ __device__ __forceinline__ void rare_path()
   asm volatile("");
 }
 
-// sqrt_short(x) == sqrtf(x) for x = +-0, x >= 2^-96, +inf, NaN.
-__device__ __forceinline__ float sqrt_short(float x)
+// A square root and the raw estimate of its reciprocal.
+struct Root {
+  float r;  // sqrtf(x) for x = 0, x >= 2^-96 or NaN (NaN for +inf)
+  float y;  // v_rsq_f32(max(x, 2^-96))
+};
+
+__device__ __forceinline__ Root root_short(float x)
 {
-  float s = __builtin_amdgcn_sqrtf(x);
-  const uint32_t sb = __float_as_uint(s);
-  const float sd = __uint_as_float(sb - 1u), su = __uint_as_float(sb + 1u);
-  const float rd = __builtin_fmaf(-sd, s, x), ru = __builtin_fmaf(-su, s, x);
-  s = rd <= 0.0f ? sd : s;
-  s = ru > 0.0f ? su : s;
-  return s;
+  // x >= 0 or NaN: the unsigned order of the bits is the order of the values
+  const float y = __builtin_amdgcn_rsqf(__uint_as_float(max(__float_as_uint(x), kSqrtShortMin)));
+  const float s = x * y, h = 0.5f * y;
+  return Root{ __builtin_fmaf(__builtin_fmaf(-s, s, x), h, s), y };
 }
 
-// sqrtf(x) for x >= 0: the short form, and the general one for lanes with 0 < x < 2^-96.
+// sqrtf(x) for x >= 0: the short form, and the general one for lanes with 0 < x < 2^-96 or
+// x = +inf.
 __device__ __forceinline__ float sqrt_cr(float x)
 {
-  float s = sqrt_short(x);
-  const bool general = __float_as_uint(x) - 1u < kSqrtShortMin - 1u;
+  float s = root_short(x).r;
+  const uint32_t b = __float_as_uint(x);
+  const bool general = (b - 1u < kSqrtShortMin - 1u) | (b == 0x7f800000u);
   if (__builtin_amdgcn_ballot_w64(general) != 0) {
     rare_path();
     if (general)
       s = __builtin_sqrtf(x);
   }
   return s;
+}
+
+// The reciprocal of a root r = root_short(x).r from its estimate, for x >= 2^-96; wrong in
+// the last bit where ones_significand(r).
+__device__ __forceinline__ float root_rcp(Root q)
+{
+  return __builtin_fmaf(__builtin_fmaf(-q.r, q.y, 1.0f), q.y, q.y);
+}
+
+__device__ __forceinline__ bool ones_significand(float r)
+{
+  return (__float_as_uint(r) | 0xff800000u) == 0xffffffffu;
 }
 
 // Refined reciprocal of a divisor d in [2^-40, 2^40].
@@ -75,14 +97,18 @@ __device__ __forceinline__ float rcp_refined(float d)
 }
 
 // n / d for d in [2^-40, 2^40] (y = rcp_refined(d)) and n = +-0 or |n| in [2^-90, 2^50]
-// with |n|/d in [2^-120, 2^90].
+// with |n|/d in [2^-120, 2^90]; a zero quotient may have either sign (no sum that starts at
+// +0 can tell).
+__device__ __forceinline__ float div_unsigned_zero(float n, float d, float y)
+{
+  const float q = n * y;
+  return __builtin_fmaf(__builtin_fmaf(-d, q, n), y, q);
+}
+
+// ... with the sign of n, as v_div_fixup gives it.
 __device__ __forceinline__ float div_short(float n, float d, float y)
 {
-  const float q0 = n * y;
-  const float r0 = __builtin_fmaf(-d, q0, n);
-  const float q1 = __builtin_fmaf(r0, y, q0);
-  const float r1 = __builtin_fmaf(-d, q1, n);
-  const float q = __builtin_fmaf(r1, y, q1);
+  const float q = div_unsigned_zero(n, d, y);
   return __uint_as_float((__float_as_uint(q) & 0x7fffffffu) | (__float_as_uint(n) & 0x80000000u));
 }
 

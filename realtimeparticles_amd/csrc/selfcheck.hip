@@ -28,8 +28,9 @@ __device__ __noinline__ float div_general(float n, float d)
   return n / d;
 }
 
-// Every bit pattern x in [lo, hi): sqrt_cr(x) against sqrtf(x).  first[0] keeps the smallest
-// mismatching pattern.
+// Every bit pattern x in [lo, hi): sqrt_cr(x) against sqrtf(x), and for finite x >= 2^-52
+// root_rcp against the reciprocal of sqrtf(x) unless its significand is all ones.  first[0]
+// keeps the smallest mismatching pattern.
 __global__ __launch_bounds__(256) void k_check_sqrt(uint32_t lo, uint32_t hi,
                                                     unsigned long long* bad, uint32_t* first)
 {
@@ -37,7 +38,9 @@ __global__ __launch_bounds__(256) void k_check_sqrt(uint32_t lo, uint32_t hi,
   uint32_t nbad = 0;
   for (uint64_t b = (uint64_t)lo + blockIdx.x * blockDim.x + threadIdx.x; b < hi; b += stride) {
     const float x = __uint_as_float((uint32_t)b);
-    if (!same(sqrt_cr(x), sqrt_general(x))) {
+    const float r = sqrt_general(x);
+    const bool rcp = b >= 0x25800000u && b < 0x7f800000u && !ones_significand(r);
+    if (!same(sqrt_cr(x), r) || (rcp && !same(root_rcp(root_short(x)), div_general(1.0f, r)))) {
       ++nbad;
       atomicMin(first, (uint32_t)b);
     }
