@@ -167,6 +167,7 @@ struct rtp_mlp {
   float* m1 = nullptr;    // Adam moments
   float* m2 = nullptr;
   float* loss = nullptr;
+  float* partial = nullptr;  // the training kernel's partial gradients
   short* w1t = nullptr;
   short* w2t = nullptr;
   short* w2 = nullptr;
@@ -197,7 +198,7 @@ struct rtp_mlp {
   {
     if (stream)
       (void)hipStreamSynchronize(stream);
-    for (float** b : { &p, &grad, &m1, &m2, &loss, &dFeat, &dTarget, &dOut })
+    for (float** b : { &p, &grad, &m1, &m2, &loss, &partial, &dFeat, &dTarget, &dOut })
       dev_free(*b);
     dev_free(w1t);
     dev_free(w2t);
@@ -1720,7 +1721,9 @@ int rtp_mlp_create(int device, uint32_t seed, rtp_mlp** out)
   }
   if ((rc = dev_alloc(&h->p, kMlpParams)) || (rc = dev_alloc(&h->grad, kMlpParams)) ||
       (rc = dev_alloc(&h->m1, kMlpParams)) || (rc = dev_alloc(&h->m2, kMlpParams)) ||
-      (rc = dev_alloc(&h->loss, 4)) || (rc = dev_alloc(&h->w1t, 64 * 16)) ||
+      (rc = dev_alloc(&h->loss, 4)) ||
+      (rc = dev_alloc(&h->partial, (size_t)kMlpMaxBlocks * kMlpPartial)) ||
+      (rc = dev_alloc(&h->w1t, 64 * 16)) ||
       (rc = dev_alloc(&h->w2t, 64 * 64)) || (rc = dev_alloc(&h->w2, 64 * 64))) {
     h->release();
     delete h;
@@ -1776,7 +1779,6 @@ int rtp_mlp_set_params(rtp_mlp* h, const float* params, uint32_t count)
   RTP_REQUIRE(count == (uint32_t)kMlpParams, "parameter count must be rtp_mlp_param_count()");
   RTP_HIP_TRY(hipSetDevice(h->device));
   RTP_HIP_TRY(hipMemcpyAsync(h->p, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice, h->stream));
-  launch_zero(h->grad, kMlpParams, h->stream);
   launch_zero(h->m1, kMlpParams, h->stream);
   launch_zero(h->m2, kMlpParams, h->stream);
   launch_mlp_pack(h->p, h->dev, h->stream);
@@ -1835,13 +1837,11 @@ int rtp_mlp_gradients(rtp_mlp* h, const float* feat, const float* target, uint32
     return rc;
   RTP_HIP_TRY(hipMemcpyAsync(h->dFeat, feat, sizeof(float) * 8 * n, hipMemcpyHostToDevice, h->stream));
   RTP_HIP_TRY(hipMemcpyAsync(h->dTarget, target, sizeof(float) * n, hipMemcpyHostToDevice, h->stream));
-  launch_zero(h->grad, kMlpParams, h->stream);
-  launch_zero(h->loss, 1, h->stream);
-  launch_mlp_train(h->dFeat, h->dTarget, nullptr, n, h->dev, h->grad, h->loss, h->stream);
+  launch_mlp_train(h->dFeat, h->dTarget, nullptr, n, h->dev, h->partial, h->stream);
+  launch_mlp_sum(h->partial, n, h->grad, h->loss, h->stream);
   RTP_HIP_TRY(hipGetLastError());
   RTP_HIP_TRY(hipMemcpyAsync(grad, h->grad, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost, h->stream));
   RTP_HIP_TRY(hipMemcpyAsync(loss, h->loss, sizeof(float), hipMemcpyDeviceToHost, h->stream));
-  launch_zero(h->grad, kMlpParams, h->stream);
   RTP_HIP_TRY(hipStreamSynchronize(h->stream));
   *loss /= (float)n;
   return RTP_OK;
@@ -1882,9 +1882,8 @@ int rtp_mlp_train(rtp_mlp* h, const float* feat, const float* target, uint32_t n
     launch_zero(h->loss, 1, h->stream);
     for (uint32_t b0 = 0; b0 < n; b0 += batch) {
       const uint32_t rows = std::min(batch, n - b0);
-      launch_mlp_train(h->dFeat, h->dTarget, h->dPerm + b0, rows, h->dev, h->grad, h->loss, h->stream);
-      launch_mlp_adam(h->p, h->grad, h->m1, h->m2, lr, ++h->step, h->dev, h->stream);
-      launch_mlp_pack(h->p, h->dev, h->stream);
+      launch_mlp_train(h->dFeat, h->dTarget, h->dPerm + b0, rows, h->dev, h->partial, h->stream);
+      launch_mlp_update(h->partial, rows, h->p, h->m1, h->m2, h->loss, lr, ++h->step, h->dev, h->stream);
     }
     RTP_HIP_TRY(hipGetLastError());
     if (epochLoss) {

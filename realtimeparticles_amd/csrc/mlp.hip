@@ -2,10 +2,11 @@
 // activations on the matrix cores (v_mfma_f32_16x16x16_bf16) with FP32 accumulation.
 // No reference counterpart: it predicts a particle's initial lambda for the PBF solver.
 //
-// One wave owns 64 rows (particles or training samples).  Layers 1 and 2 are 4 x 4 tiles
-// of 16 x 16 outputs per wave; the 64 -> 1 head and the elementwise work run on the VALU.
-// Activations are staged through LDS to turn the accumulator layout into the next layer's
-// operand layout.
+// A wave works on tiles of 16 rows (particles or training samples), transposed: the weights
+// are the A operand and the rows the columns of B, so a layer's result has the layout of
+// the next layer's B operand (a lane keeps its row and four consecutive hidden units) and
+// activations go from layer to layer in registers.  The 64 -> 1 head and the elementwise
+// work run on the VALU.
 //
 // Operand layout of v_mfma_f32_16x16x16_bf16 (lane l, j = 0..3):
 //   A (16 x 16, M x K): A[l % 16][4 * (l / 16) + j]
@@ -30,8 +31,6 @@ __device__ __forceinline__ short f2bf(float f)
   return (short)(u >> 16);
 }
 
-__device__ __forceinline__ float bf2f(short b) { return __uint_as_float(((uint32_t)(uint16_t)b) << 16); }
-
 constexpr float kGeluA = 0.7978845608028654f;  // sqrt(2 / pi)
 constexpr float kGeluB = 0.044715f;
 
@@ -41,7 +40,7 @@ constexpr float kGeluB = 0.044715f;
 __device__ __forceinline__ float sigmoid2u(float z)
 {
   const float u = kGeluA * (z + kGeluB * (z * z) * z);
-  return __builtin_amdgcn_rcpf(1.0f + __expf(-2.0f * u));
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(u * (-2.0f * 1.44269504f)));
 }
 
 __device__ __forceinline__ float gelu(float z) { return z * sigmoid2u(z); }
@@ -61,300 +60,352 @@ __device__ __forceinline__ f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c)
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
 }
 
-struct WaveLds {
-  short X[64][16];   // normalised inputs (bf16, k padded to 16 with zeros)
-  short H1[64][64];  // layer-1 activations (bf16)
+// Four floats rounded to bf16 (nearest even, as f2bf).
+__device__ __forceinline__ bf16x4 to_bf16(f32x4 v)
+{
+  typedef __bf16 bfv4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(bf16x4, __builtin_convertvector(v, bfv4));
+}
+
+// GELU and its derivative of four pre-activations (gelu, gelu_grad).
+__device__ __forceinline__ f32x4 gelu4(f32x4 z)
+{
+  return f32x4{ gelu(z[0]), gelu(z[1]), gelu(z[2]), gelu(z[3]) };
+}
+__device__ __forceinline__ f32x4 gelu_grad4(f32x4 z)
+{
+  return f32x4{ gelu_grad(z[0]), gelu_grad(z[1]), gelu_grad(z[2]), gelu_grad(z[3]) };
+}
+
+// The lane's part of a row's standardised inputs as layer 1's B operand: inputs 4 lq + j for
+// lq < 2; inputs 8..15 of the padded layer are zero, an invalid row standardises zeros.
+struct InputScale {
+  f32x4 mu, inv;
+  __device__ __forceinline__ InputScale(const MlpDev& m, uint32_t lq)
+  {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      mu[j] = lq == 1u ? m.mu[4 + j] : m.mu[j];
+      inv[j] = lq == 1u ? m.invSigma[4 + j] : m.invSigma[j];
+    }
+  }
+  __device__ __forceinline__ bf16x4 operator()(const float* __restrict__ feat, uint32_t src, bool valid,
+                                               uint32_t lq) const
+  {
+    f32x4 x = { 0.0f, 0.0f, 0.0f, 0.0f };
+    if (lq < 2u) {
+      if (valid)  // feat rows are 32-byte aligned
+        x = *reinterpret_cast<const f32x4*>(feat + (size_t)src * 8 + 4 * lq);
+      x = (x - mu) * inv;
+    }
+    return to_bf16(x);
+  }
 };
 
-// Inputs of the wave's 64 rows into LDS; returns whether this lane's row exists.
-__device__ __forceinline__ bool load_inputs(const float* __restrict__ feat, uint32_t row0, uint32_t n,
-                                            const MlpDev& m, short (*X)[16], const uint32_t* perm)
+// The head of a row from this lane's y[j] = sum over t of gelu(z2) w3 at hidden units 16 t + 4 lq
+// + j: the sums of lanes lq ^ 2, lq ^ 1, then j ^ 2, j ^ 1.
+__device__ __forceinline__ float head_sum(f32x4 y)
 {
-  const uint32_t l = threadIdx.x;
-  const uint32_t r = row0 + l;
-  const bool valid = r < n;
-  const uint32_t src = valid ? (perm ? perm[r] : r) : 0u;
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const float x = valid ? feat[(size_t)src * 8 + k] : 0.0f;
-    X[l][k] = f2bf((x - m.mu[k]) * m.invSigma[k]);
-    X[l][8 + k] = 0;
+  for (int j = 0; j < 4; ++j) {
+    y[j] += __shfl_xor(y[j], 32, 64);
+    y[j] += __shfl_xor(y[j], 16, 64);
   }
-  return valid;
+  return (y[0] + y[2]) + (y[1] + y[3]);
 }
 
-// Layer 1 for the wave: z1 = x W1 + b1, writing GELU(z1) (bf16) to H1 and optionally z1.
-__device__ __forceinline__ void layer1(const MlpDev& m, short (*X)[16], short (*H1)[64], float (*Z1)[64])
+// Inference: each wave keeps its lanes' weights in registers and runs two tiles of 16 rows at
+// a time (two independent chains) in a grid-stride loop.  Bound by issue: 128 GELUs a row, two
+// quarter-rate transcendentals each.
+constexpr uint32_t kFwdTiles = 2;
+__global__ __launch_bounds__(256) void k_mlp_forward(const float* __restrict__ feat, uint32_t n, MlpDev m,
+                                                     float* __restrict__ out)
 {
-  const uint32_t l = threadIdx.x, lr = l % 16u, lq = l / 16u;
-  float b1[4];
+  const uint32_t l = threadIdx.x & 63u, lr = l % 16u, lq = l / 16u;
+  const InputScale inputs(m, lq);
+  bf16x4 w1[4], w2[4][4];
+  f32x4 b1[4], b2[4], w3[4];
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
-    b1[nt] = m.p[kMlpB1 + nt * 16 + lr];
-  for (int mt = 0; mt < 4; ++mt)
+  for (int u = 0; u < 4; ++u) {
+    w1[u] = ld4(m.w1t + (u * 16 + lr) * 16 + 4 * lq);
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-      acc = mfma(ld4(&X[mt * 16 + lr][4 * lq]), ld4(m.w1t + (nt * 16 + lr) * 16 + 4 * lq), acc);
+    for (int t = 0; t < 4; ++t)
+      w2[u][t] = ld4(m.w2t + (u * 16 + lr) * 64 + t * 16 + 4 * lq);
+    const float* at = m.p + u * 16 + 4 * lq;  // the offsets are multiples of four floats
+    b1[u] = *reinterpret_cast<const f32x4*>(at + kMlpB1);
+    b2[u] = *reinterpret_cast<const f32x4*>(at + kMlpB2);
+    w3[u] = *reinterpret_cast<const f32x4*>(at + kMlpW3);
+  }
+  const float b3 = m.p[kMlpB3];
+  const uint32_t rows = 16u * kFwdTiles, waves = gridDim.x * 4u;
+  const uint32_t groups = (n + rows - 1u) / rows;
+  for (uint32_t g = blockIdx.x * 4u + (threadIdx.x >> 6); g < groups; g += waves) {
+    const uint32_t row0 = g * rows;
+    bf16x4 h[kFwdTiles][4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int row = mt * 16 + 4 * lq + j, col = nt * 16 + lr;
-        const float z = acc[j] + b1[nt];
-        if (Z1)
-          Z1[row][col] = z;
-        H1[row][col] = f2bf(gelu(z));
+    for (uint32_t k = 0; k < kFwdTiles; ++k) {
+      const uint32_t r = row0 + k * 16u + lr;
+      const bf16x4 x = inputs(feat, r, r < n, lq);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const f32x4 z = mfma(w1[t], x, f32x4{ 0.0f, 0.0f, 0.0f, 0.0f });
+        h[k][t] = to_bf16(gelu4(z + b1[t]));
       }
     }
-}
-
-// Layer 2 tile (mt, nt): z2 = h1 W2 + b2 for rows mt*16.., columns nt*16..
-__device__ __forceinline__ f32x4 layer2_tile(const MlpDev& m, short (*H1)[64], int mt, int nt)
-{
-  const uint32_t l = threadIdx.x, lr = l % 16u, lq = l / 16u;
-  f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-  for (int kt = 0; kt < 4; ++kt)
-    acc = mfma(ld4(&H1[mt * 16 + lr][kt * 16 + 4 * lq]), ld4(m.w2t + (nt * 16 + lr) * 64 + kt * 16 + 4 * lq), acc);
-  return acc;
+    for (uint32_t k = 0; k < kFwdTiles; ++k) {
+      f32x4 y = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        f32x4 z = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          z = mfma(w2[u][t], h[k][t], z);
+        y += gelu4(z + b2[u]) * w3[u];
+      }
+      const float v = head_sum(y) + b3;
+      const uint32_t r = row0 + k * 16u + lr;
+      if (lq == 0 && r < n)
+        out[r] = v * m.outScale;
+    }
+  }
 }
 
-// Sum over the 16 lanes that share l / 16.
-__device__ __forceinline__ float sum16(float v)
+// Q[row][c] held as lane (row = lr, c = 4 lq + j) -> lane (c = lr, row = 4 lq + j): a product
+// with the identity, exact (one term of each sum is not zero).
+__device__ __forceinline__ bf16x4 transpose16(bf16x4 q, bf16x4 identity)
 {
-  v += __shfl_xor(v, 8, 64);
-  v += __shfl_xor(v, 4, 64);
-  v += __shfl_xor(v, 2, 64);
-  v += __shfl_xor(v, 1, 64);
+  return to_bf16(mfma(q, identity, f32x4{ 0.0f, 0.0f, 0.0f, 0.0f }));
+}
+
+// Forward + backward of the mean squared error over a batch.  A wave carries a tile of 16
+// rows from the inputs to the last gradient in registers (the two products that contract
+// over rows read tiles transposed by transpose16) and adds up every gradient over its tiles;
+// a workgroup's waves put their sums side by side in LDS, and the workgroup writes their sum as
+// one partial gradient (its squared errors as entry kMlpParams), which k_mlp_update or
+// k_mlp_sum adds up in order, so a batch's gradient repeats bit for bit.  Bound by the one wave
+// a SIMD that the sums leave room for (300 registers).  65,536 rows: 27 us, and 5 us for
+// k_mlp_update; a 64-row wave with its tile in 58 KB of LDS (two waves a CU) and 4.9 M atomics
+// on 4,801 words took 78 us, and 10 us for the step and the operand copies apart.
+constexpr uint32_t kTrainWaves = 4;
+constexpr uint32_t kW1Pitch = 20, kW2Pitch = 68;  // shorts per row in LDS: 16 rows' 8-byte reads on distinct banks
+__global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train(const float* __restrict__ feat,
+                                                                const float* __restrict__ target,
+                                                                const uint32_t* __restrict__ perm,
+                                                                uint32_t n, float invBatch, MlpDev m,
+                                                                float* __restrict__ partial)
+{
+  __shared__ __align__(16) short sw1[64 * kW1Pitch], sw2t[64 * kW2Pitch], sw2[64 * kW2Pitch];
+  __shared__ __align__(16) float sb1[64], sb2[64], sw3[64];
+  __shared__ float sums[kTrainWaves][kMlpPartial];
+  const uint32_t l = threadIdx.x & 63u, lr = l % 16u, lq = l / 16u, w = threadIdx.x >> 6;
+  for (uint32_t i = 4u * threadIdx.x; i < 64u * 64u; i += 4u * blockDim.x) {
+    const uint32_t at = (i >> 6) * kW2Pitch + (i & 63u);
+    *reinterpret_cast<bf16x4*>(sw2t + at) = ld4(m.w2t + i);
+    *reinterpret_cast<bf16x4*>(sw2 + at) = ld4(m.w2 + i);
+  }
+  if (4u * threadIdx.x < 64u * 16u) {
+    const uint32_t i = 4u * threadIdx.x;
+    *reinterpret_cast<bf16x4*>(sw1 + (i >> 4) * kW1Pitch + (i & 15u)) = ld4(m.w1t + i);
+  }
+  if (threadIdx.x < 64u) {
+    sb1[threadIdx.x] = m.p[kMlpB1 + threadIdx.x];
+    sb2[threadIdx.x] = m.p[kMlpB2 + threadIdx.x];
+    sw3[threadIdx.x] = m.p[kMlpW3 + threadIdx.x];
+  }
+  __syncthreads();
+  const f32x4 zero = { 0.0f, 0.0f, 0.0f, 0.0f };
+  const InputScale inputs(m, lq);
+  const float b3 = m.p[kMlpB3];
+  const auto four = [&](const float* p, int t) { return *reinterpret_cast<const f32x4*>(p + t * 16 + 4 * lq); };
+  bf16x4 identity;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    identity[j] = 4u * lq + j == lr ? (short)0x3f80 : (short)0;
+  f32x4 dW2[4][4], dW1[4], db1[4], db2[4], dw3[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    dW1[t] = db1[t] = db2[t] = dw3[t] = zero;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      dW2[t][u] = zero;
+  }
+  float db3 = 0.0f, se = 0.0f;
+  const uint32_t tiles = (n + 15u) / 16u;
+  for (uint32_t tile = blockIdx.x * kTrainWaves + w; tile < tiles; tile += gridDim.x * kTrainWaves) {
+    // the weights stay in LDS: hoisted out of the loop they would spill the gradient sums
+    asm volatile("" ::: "memory");
+    const uint32_t row = tile * 16u + lr;
+    const bool valid = row < n;
+    const uint32_t src = valid ? (perm ? perm[row] : row) : 0u;
+    const float goal = valid ? target[src] / m.outScale : 0.0f;
+    const bf16x4 x = inputs(feat, src, valid, lq);
+    bf16x4 h[4], d2[4];
+    f32x4 g1[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const f32x4 z = mfma(ld4(sw1 + (t * 16 + lr) * kW1Pitch + 4 * lq), x, zero) + four(sb1, t);
+      h[t] = to_bf16(gelu4(z));
+      g1[t] = gelu_grad4(z);
+    }
+    f32x4 a2[4], g2[4], y = zero;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      f32x4 z = zero;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        z = mfma(ld4(sw2t + (u * 16 + lr) * kW2Pitch + t * 16 + 4 * lq), h[t], z);
+      z += four(sb2, u);
+      a2[u] = gelu4(z);
+      g2[u] = gelu_grad4(z);
+      y += a2[u] * four(sw3, u);
+    }
+    const float e = valid ? head_sum(y) + b3 - goal : 0.0f;
+    const float dy = 2.0f * e * invBatch;
+    if (lq == 0) {  // the four lanes of a row hold the same error
+      se += e * e;
+      db3 += dy;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const f32x4 dz = (dy * four(sw3, u)) * g2[u];
+      dw3[u] += a2[u] * dy;
+      db2[u] += dz;
+      d2[u] = to_bf16(dz);
+    }
+      bf16x4 hT[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      hT[t] = transpose16(h[t], identity);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const bf16x4 dT = transpose16(d2[u], identity);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)  // dW2[k][n] = sum over rows of h1[row][k] dz2[row][n]
+        dW2[t][u] = mfma(hT[t], dT, dW2[t][u]);
+    }
+    const bf16x4 xT = transpose16(x, identity);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      f32x4 dh = zero;  // dh1[k][row] = sum over n of W2[k][n] dz2[row][n]
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        dh = mfma(ld4(sw2 + (t * 16 + lr) * kW2Pitch + u * 16 + 4 * lq), d2[u], dh);
+      const f32x4 dz = dh * g1[t];
+      db1[t] += dz;
+      // dW1[k][n] = sum over rows of x[row][k] dz1[row][n]
+      dW1[t] = mfma(xT, transpose16(to_bf16(dz), identity), dW1[t]);
+    }
+  }
+  // sums over the tile's rows
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        db1[t][j] += __shfl_xor(db1[t][j], o, 64);
+        db2[t][j] += __shfl_xor(db2[t][j], o, 64);
+        dw3[t][j] += __shfl_xor(dw3[t][j], o, 64);
+      }
+    se += __shfl_xor(se, o, 64);
+    db3 += __shfl_xor(db3, o, 64);
+  }
+  float* const own = sums[w];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t k = t * 16 + 4 * lq + j;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        own[kMlpW2 + k * 64 + u * 16 + lr] = dW2[t][u][j];
+      if (lq < 2)
+        own[kMlpW1 + (4 * lq + j) * 64 + t * 16 + lr] = dW1[t][j];
+      if (lr == 0) {
+        own[kMlpB1 + k] = db1[t][j];
+        own[kMlpB2 + k] = db2[t][j];
+        own[kMlpW3 + k] = dw3[t][j];
+      }
+    }
+  if (l == 0) {
+    own[kMlpB3] = db3;
+    own[kMlpParams] = se;
+  }
+  __syncthreads();
+  float* const mine = partial + (size_t)blockIdx.x * kMlpPartial;
+  for (uint32_t i = threadIdx.x; i <= (uint32_t)kMlpParams; i += blockDim.x) {
+    float v = sums[0][i];
+#pragma unroll
+    for (uint32_t k = 1; k < kTrainWaves; ++k)
+      v += sums[k][i];
+    mine[i] = v;
+  }
+}
+
+// Sum of entry i of `blocks` partial gradients, 16 slices of a 1024-thread block at a time in
+// a fixed order; threads of slice 0 hold it (64 entries per block).
+constexpr uint32_t kSumSlices = 16;
+__device__ __forceinline__ float sum_partials(const float* __restrict__ partial, uint32_t blocks,
+                                              uint32_t i)
+{
+  __shared__ float s[kSumSlices][64];
+  const uint32_t c = threadIdx.x & 63u, slice = threadIdx.x >> 6;
+  float v = 0.0f;
+#pragma unroll 4
+  for (uint32_t b = slice; b < blocks; b += kSumSlices)
+    v += partial[(size_t)b * kMlpPartial + i];
+  s[slice][c] = v;
+  __syncthreads();
+  if (slice == 0)
+    for (uint32_t k = 1; k < kSumSlices; ++k)
+      v += s[k][c];
   return v;
 }
 
-// Inference: each wave keeps its lanes' weight operands (W1, W2 fragments, biases, head)
-// in registers and runs 64-row tiles in a grid-stride loop.
-__global__ __launch_bounds__(64) void k_mlp_forward(const float* __restrict__ feat, uint32_t n, MlpDev m,
-                                                    float* __restrict__ out)
+// The batch's gradient and squared-error sum.
+__global__ __launch_bounds__(64 * kSumSlices) void k_mlp_sum(const float* __restrict__ partial, uint32_t blocks,
+                                                             float* __restrict__ grad, float* __restrict__ loss)
 {
-  __shared__ WaveLds s;
-  const uint32_t l = threadIdx.x, lr = l % 16u, lq = l / 16u;
-  bf16x4 w1f[4], w2f[4][4];
-  float b1[4], b2[4], w3[4];
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    w1f[nt] = ld4(m.w1t + (nt * 16 + lr) * 16 + 4 * lq);
-#pragma unroll
-    for (int kt = 0; kt < 4; ++kt)
-      w2f[nt][kt] = ld4(m.w2t + (nt * 16 + lr) * 64 + kt * 16 + 4 * lq);
-    b1[nt] = m.p[kMlpB1 + nt * 16 + lr];
-    b2[nt] = m.p[kMlpB2 + nt * 16 + lr];
-    w3[nt] = m.p[kMlpW3 + nt * 16 + lr];
-  }
-  const float b3 = m.p[kMlpB3];
-  for (uint32_t row0 = blockIdx.x * 64u; row0 < n; row0 += gridDim.x * 64u) {
-    (void)load_inputs(feat, row0, n, m, s.X, nullptr);
-    __syncthreads();
-    for (int mt = 0; mt < 4; ++mt) {
-      const bf16x4 xa = ld4(&s.X[mt * 16 + lr][4 * lq]);
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-        acc = mfma(xa, w1f[nt], acc);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          s.H1[mt * 16 + 4 * lq + j][nt * 16 + lr] = f2bf(gelu(acc[j] + b1[nt]));
-      }
-    }
-    __syncthreads();
-    for (int mt = 0; mt < 4; ++mt) {
-      bf16x4 ha[4];
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt)
-        ha[kt] = ld4(&s.H1[mt * 16 + lr][kt * 16 + 4 * lq]);
-      float y[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-#pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-          acc = mfma(ha[kt], w2f[nt][kt], acc);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          y[j] += gelu(acc[j] + b2[nt]) * w3[nt];
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float v = sum16(y[j]);
-        const uint32_t r = row0 + mt * 16 + 4 * lq + j;
-        if (lr == 0 && r < n)
-          out[r] = (v + b3) * m.outScale;
-      }
-    }
-    __syncthreads();  // the next tile overwrites X and H1
-  }
-}
-
-// Forward + backward of the mean squared error over a batch; gradients are added to grad
-// (the parameter layout above) and the squared-error sum to loss.
-struct TrainLds {
-  short X[64][16];
-  short H1[64][64];
-  float Z1[64][64];
-  float Z2[64][64];
-  float DZ[64][64];  // dz2, then dz1
-  float Y[64];
-  float DY[64];
-};
-
-__global__ __launch_bounds__(64) void k_mlp_train(const float* __restrict__ feat,
-                                                  const float* __restrict__ target,
-                                                  const uint32_t* __restrict__ perm, uint32_t n,
-                                                  float invBatch, MlpDev m, float* __restrict__ grad,
-                                                  float* __restrict__ loss)
-{
-  __shared__ TrainLds s;
-  const uint32_t l = threadIdx.x, lr = l % 16u, lq = l / 16u;
-  const uint32_t row0 = blockIdx.x * 64u;
-  const bool valid = load_inputs(feat, row0, n, m, s.X, perm);
-  __syncthreads();
-  layer1(m, s.X, s.H1, s.Z1);
-  __syncthreads();
-  // layer 2 and the head
-  for (int mt = 0; mt < 4; ++mt) {
-    float y[4] = { 0.0f, 0.0f, 0.0f, 0.0f };
-    for (int nt = 0; nt < 4; ++nt) {
-      const f32x4 acc = layer2_tile(m, s.H1, mt, nt);
-      const int col = nt * 16 + lr;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float z = acc[j] + m.p[kMlpB2 + col];
-        s.Z2[mt * 16 + 4 * lq + j][col] = z;
-        y[j] += gelu(z) * m.p[kMlpW3 + col];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float v = sum16(y[j]);
-      if (lr == 0)
-        s.Y[mt * 16 + 4 * lq + j] = v + m.p[kMlpB3];
-    }
-  }
-  __syncthreads();
-  // d loss / d y for this lane's row
-  {
-    const uint32_t r = row0 + l;
-    const float t = valid ? target[perm ? perm[r] : r] / m.outScale : 0.0f;
-    const float e = valid ? s.Y[l] - t : 0.0f;
-    s.DY[l] = 2.0f * e * invBatch;
-    float se = e * e, db3 = 2.0f * e * invBatch;
-    for (int o = 32; o > 0; o >>= 1) {
-      se += __shfl_xor(se, o, 64);
-      db3 += __shfl_xor(db3, o, 64);
-    }
-    if (l == 0) {
-      atomicAdd(loss, se);
-      atomicAdd(grad + kMlpB3, db3);
-    }
-  }
-  __syncthreads();
-  // head and layer-2 activation: lane l owns hidden unit l
-  {
-    float dw3 = 0.0f, db2 = 0.0f;
-    const float w3 = m.p[kMlpW3 + l];
-    for (int r = 0; r < 64; ++r) {
-      const float z = s.Z2[r][l];
-      const float dy = s.DY[r];
-      dw3 += gelu(z) * dy;
-      const float dz = dy * w3 * gelu_grad(z);
-      s.DZ[r][l] = dz;
-      db2 += dz;
-    }
-    atomicAdd(grad + kMlpW3 + l, dw3);
-    atomicAdd(grad + kMlpB2 + l, db2);
-  }
-  __syncthreads();
-  // dW2[k][n] = sum_rows h1[row][k] dz2[row][n]   (M = k, N = n, K = rows)
-  for (int mt = 0; mt < 4; ++mt)
-    for (int nt = 0; nt < 4; ++nt) {
-      f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-      for (int kt = 0; kt < 4; ++kt) {
-        bf16x4 a, b;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int row = kt * 16 + 4 * lq + j;
-          a[j] = s.H1[row][mt * 16 + lr];
-          b[j] = f2bf(s.DZ[row][nt * 16 + lr]);
-        }
-        acc = mfma(a, b, acc);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        atomicAdd(grad + kMlpW2 + (mt * 16 + 4 * lq + j) * 64 + nt * 16 + lr, acc[j]);
-    }
-  // dh1[row][k] = sum_n dz2[row][n] W2[k][n]   (M = rows, N = k, K = n) -> dz1
-  float dz1[4][4][4];
-  for (int mt = 0; mt < 4; ++mt)
-    for (int nt = 0; nt < 4; ++nt) {
-      f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-      for (int kt = 0; kt < 4; ++kt) {
-        bf16x4 a;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          a[j] = f2bf(s.DZ[mt * 16 + lr][kt * 16 + 4 * lq + j]);
-        acc = mfma(a, ld4(m.w2 + (nt * 16 + lr) * 64 + kt * 16 + 4 * lq), acc);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        dz1[mt][nt][j] = acc[j] * gelu_grad(s.Z1[mt * 16 + 4 * lq + j][nt * 16 + lr]);
-    }
-  __syncthreads();  // every lane has read dz2
-  for (int mt = 0; mt < 4; ++mt)
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        s.DZ[mt * 16 + 4 * lq + j][nt * 16 + lr] = dz1[mt][nt][j];
-  __syncthreads();
-  {
-    float db1 = 0.0f;
-    for (int r = 0; r < 64; ++r)
-      db1 += s.DZ[r][l];
-    atomicAdd(grad + kMlpB1 + l, db1);
-  }
-  // dW1[k][n] = sum_rows x[row][k] dz1[row][n]   (M = k padded to 16, N = n, K = rows)
-  for (int nt = 0; nt < 4; ++nt) {
-    f32x4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-    for (int kt = 0; kt < 4; ++kt) {
-      bf16x4 a, b;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int row = kt * 16 + 4 * lq + j;
-        a[j] = s.X[row][lr];
-        b[j] = f2bf(s.DZ[row][nt * 16 + lr]);
-      }
-      acc = mfma(a, b, acc);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int k = 4 * lq + j;
-      if (k < 8)
-        atomicAdd(grad + kMlpW1 + k * 64 + nt * 16 + lr, acc[j]);
-    }
-  }
-}
-
-// Adam on the fp32 master parameters, then the bf16 operand copies; clears the gradient.
-__global__ __launch_bounds__(256) void k_mlp_adam(float* __restrict__ p, float* __restrict__ grad,
-                                                  float* __restrict__ m1, float* __restrict__ m2,
-                                                  float lr, float b1, float b2, float eps, float c1,
-                                                  float c2, MlpDev m)
-{
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (uint32_t)kMlpParams)
+  const uint32_t i = blockIdx.x * 64u + (threadIdx.x & 63u);  // kMlpPartial covers every i
+  const float g = sum_partials(partial, blocks, i);
+  if (threadIdx.x >= 64u)
     return;
-  const float g = grad[i];
-  grad[i] = 0.0f;
+  if (i < (uint32_t)kMlpParams)
+    grad[i] = g;
+  else if (i == (uint32_t)kMlpParams)
+    loss[0] = g;
+}
+
+// Adam on the fp32 master parameters with the summed gradient, the bf16 operand copies of the
+// parameters it moved, and the batch's squared errors added to loss: one launch.
+__global__ __launch_bounds__(64 * kSumSlices) void k_mlp_update(const float* __restrict__ partial,
+                                                                uint32_t blocks, float* __restrict__ p,
+                                                                float* __restrict__ m1, float* __restrict__ m2,
+                                                                float* __restrict__ loss, float lr, float b1,
+                                                                float b2, float eps, float c1, float c2, MlpDev m)
+{
+  const uint32_t i = blockIdx.x * 64u + (threadIdx.x & 63u);
+  const float g = sum_partials(partial, blocks, i);
+  if (threadIdx.x >= 64u || i > (uint32_t)kMlpParams)
+    return;
+  if (i == (uint32_t)kMlpParams) {
+    loss[0] += g;
+    return;
+  }
   const float a = b1 * m1[i] + (1.0f - b1) * g;
   const float v = b2 * m2[i] + (1.0f - b2) * g * g;
   m1[i] = a;
   m2[i] = v;
-  p[i] -= lr * (a / c1) / (sqrtf(v / c2) + eps);
+  const float q = p[i] - lr * (a / c1) / (sqrtf(v / c2) + eps);
+  p[i] = q;
+  if (i < (uint32_t)kMlpB1) {
+    m.w1tMut[(i % 64u) * 16u + i / 64u] = f2bf(q);
+  } else if (i >= (uint32_t)kMlpW2 && i < (uint32_t)kMlpB2) {
+    const uint32_t k = (i - kMlpW2) / 64u, u = (i - kMlpW2) % 64u;
+    m.w2tMut[u * 64u + k] = f2bf(q);
+    m.w2Mut[k * 64u + u] = f2bf(q);
+  }
 }
 
 // Rebuild the operand copies from the master parameters.
@@ -394,26 +445,45 @@ void launch_mlp_forward(const float* feat, uint32_t n, const MlpDev& m, float* o
 {
   if (n == 0)
     return;
-  const uint32_t tiles = blocks_for(n, 64);
-  hipLaunchKernelGGL(k_mlp_forward, dim3(tiles < 4096u ? tiles : 4096u), dim3(64), 0, s, feat, n, m, out);
+  // at most four workgroups a CU: a wave's weights are loaded once for all its rows
+  const uint32_t blocks = blocks_for(n, 16u * kFwdTiles * 4u);
+  hipLaunchKernelGGL(k_mlp_forward, dim3(blocks < 1024u ? blocks : 1024u), dim3(256), 0, s, feat, n, m, out);
+}
+
+// One workgroup a CU at most, so the partial gradients stay few; small batches spread their
+// tiles over as many workgroups as have four.
+static uint32_t train_blocks(uint32_t n)
+{
+  const uint32_t b = blocks_for(n, 16u * kTrainWaves);
+  return b < kMlpMaxBlocks ? b : kMlpMaxBlocks;
 }
 
 void launch_mlp_train(const float* feat, const float* target, const uint32_t* perm, uint32_t n,
-                      const MlpDev& m, float* grad, float* loss, hipStream_t s)
+                      const MlpDev& m, float* partial, hipStream_t s)
 {
   if (n == 0)
     return;
-  hipLaunchKernelGGL(k_mlp_train, dim3(blocks_for(n, 64)), dim3(64), 0, s, feat, target, perm, n,
-                     1.0f / (float)n, m, grad, loss);
+  hipLaunchKernelGGL(k_mlp_train, dim3(train_blocks(n)), dim3(64 * kTrainWaves), 0, s, feat, target,
+                     perm, n, 1.0f / (float)n, m, partial);
 }
 
-void launch_mlp_adam(float* p, float* grad, float* m1, float* m2, float lr, int step,
-                     const MlpDev& m, hipStream_t s)
+void launch_mlp_sum(const float* partial, uint32_t n, float* grad, float* loss, hipStream_t s)
 {
+  if (n == 0)
+    return;
+  hipLaunchKernelGGL(k_mlp_sum, dim3(kMlpPartial / 64), dim3(64 * kSumSlices), 0, s, partial,
+                     train_blocks(n), grad, loss);
+}
+
+void launch_mlp_update(const float* partial, uint32_t n, float* p, float* m1, float* m2, float* loss,
+                       float lr, int step, const MlpDev& m, hipStream_t s)
+{
+  if (n == 0)
+    return;
   const float b1 = 0.9f, b2 = 0.999f;
   const float c1 = 1.0f - powf(b1, (float)step), c2 = 1.0f - powf(b2, (float)step);
-  hipLaunchKernelGGL(k_mlp_adam, dim3(blocks_for(kMlpParams, 256)), dim3(256), 0, s, p, grad, m1,
-                     m2, lr, b1, b2, 1e-8f, c1, c2, m);
+  hipLaunchKernelGGL(k_mlp_update, dim3(kMlpPartial / 64), dim3(64 * kSumSlices), 0, s, partial,
+                     train_blocks(n), p, m1, m2, loss, lr, b1, b2, 1e-8f, c1, c2, m);
 }
 
 void launch_mlp_pack(const float* p, const MlpDev& m, hipStream_t s)

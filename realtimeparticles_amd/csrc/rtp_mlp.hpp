@@ -32,10 +32,18 @@ struct MlpDev {
 };
 
 void launch_mlp_forward(const float* feat, uint32_t n, const MlpDev& m, float* out, hipStream_t s);
+// Partial gradients of a batch: one per workgroup of the training kernel, kMlpPartial floats
+// each (the gradient in the parameter layout, the squared-error sum, padding).
+constexpr uint32_t kMlpMaxBlocks = 256;
+constexpr uint32_t kMlpPartial = (kMlpParams + 1 + 63) / 64 * 64;
+// Forward and backward of n rows into partial (kMlpMaxBlocks x kMlpPartial floats) ...
 void launch_mlp_train(const float* feat, const float* target, const uint32_t* perm, uint32_t n,
-                      const MlpDev& m, float* grad, float* loss, hipStream_t s);
-void launch_mlp_adam(float* p, float* grad, float* m1, float* m2, float lr, int step,
-                     const MlpDev& m, hipStream_t s);
+                      const MlpDev& m, float* partial, hipStream_t s);
+// ... then the batch's gradient and squared-error sum, or an Adam step with it (and the
+// squared errors added to loss).
+void launch_mlp_sum(const float* partial, uint32_t n, float* grad, float* loss, hipStream_t s);
+void launch_mlp_update(const float* partial, uint32_t n, float* p, float* m1, float* m2, float* loss,
+                       float lr, int step, const MlpDev& m, hipStream_t s);
 void launch_mlp_pack(const float* p, const MlpDev& m, hipStream_t s);
 void launch_zero(float* p, uint32_t n, hipStream_t s);
 void launch_affine_perm(uint32_t* perm, uint32_t n, uint32_t a, uint32_t c, hipStream_t s);
