@@ -382,7 +382,7 @@ int rtp_batch_create(int device, const rtp_batch_scene* sc, uint32_t count, rtp_
   h->nbThreads = N + 255u * (uint32_t)h->scenes.size();
   if ((rc = dev_alloc(&h->pos[0], N)) || (rc = dev_alloc(&h->pos[1], N)) ||
       (rc = dev_alloc(&h->vel[0], N)) || (rc = dev_alloc(&h->vel[1], N)) ||
-      (rc = dev_alloc(&h->pred[0], N)) || (rc = dev_alloc(&h->pred[1], N)) ||
+      (rc = dev_alloc(&h->pred[0], N + kPosPad)) || (rc = dev_alloc(&h->pred[1], N + kPosPad)) ||
       (rc = dev_alloc(&h->vort, N)) || (rc = dev_alloc(&h->velTmp, N)) ||
       (rc = dev_alloc(&h->density, N)) || (rc = dev_alloc(&h->lambda, N)) ||
       (rc = dev_alloc(&h->key[0], N)) || (rc = dev_alloc(&h->key[1], N)) ||

@@ -875,8 +875,8 @@ int rtp_fluids_create(const rtp_model_desc* d, rtp_fluids** out)
   const uint32_t maxN = d->maxNbParticles;
   if ((rc = h->grid.alloc(maxN)) || (rc = dev_alloc(&h->pos[0], maxN)) ||
       (rc = dev_alloc(&h->pos[1], maxN)) || (rc = dev_alloc(&h->vel[0], maxN)) ||
-      (rc = dev_alloc(&h->vel[1], maxN)) || (rc = dev_alloc(&h->pred[0], maxN)) ||
-      (rc = dev_alloc(&h->pred[1], maxN)) || (rc = dev_alloc(&h->vort, maxN)) ||
+      (rc = dev_alloc(&h->vel[1], maxN)) || (rc = dev_alloc(&h->pred[0], maxN + kPosPad)) ||
+      (rc = dev_alloc(&h->pred[1], maxN + kPosPad)) || (rc = dev_alloc(&h->vort, maxN)) ||
       (rc = dev_alloc(&h->velTmp, maxN)) || (rc = dev_alloc(&h->density, maxN)) ||
       (rc = dev_alloc(&h->lambda, maxN)) || (rc = dev_alloc(&h->metric, kMetricFloats)) ||
       (rc = dev_alloc(&h->feat, (size_t)maxN * 8)) ||

@@ -40,134 +40,157 @@ __device__ __forceinline__ float4 clamp_pos(float4 q, const PbfConsts& c)
                      clampf(q.z, c.lo[2], c.hi[2]), 0.0f);
 }
 
-// Position e; with CL the boundary clamp is applied on the way in, which gives a pass the
-// positions the reference clamps in place at the start of a Jacobi iteration.
-template <bool CL>
-__device__ __forceinline__ float4 ldp(const float4* __restrict__ pred, uint32_t e, const PbfConsts& c)
-{
-  const float4 q = pred[e];
-  return CL ? clamp_pos(q, c) : q;
-}
-
-// The same for a neighbour, whose w lane (always 0) no distance reads: 12 bytes instead of 16.
-template <bool CL>
-__device__ __forceinline__ float4 ldn(const float4* __restrict__ pred, uint32_t e, const PbfConsts& c)
+// Position e of a neighbour, whose w lane (always 0) no distance reads: 12 bytes instead of 16.
+__device__ __forceinline__ float4 ldn(const float4* __restrict__ pred, uint32_t e)
 {
   const float* f = reinterpret_cast<const float*>(pred + e);
-  const float4 q = make_float4(f[0], f[1], f[2], 0.0f);
-  return CL ? clamp_pos(q, c) : q;
+  return make_float4(f[0], f[1], f[2], 0.0f);
 }
 
-// A lane's survivor queue: entries slot[0], slot[stride], ... up to cap entries, the next
-// free one at wp.  Candidates are written unconditionally and kept by advancing wp, and the
-// queue is drained whenever fewer than four entries are free (wp > room4), so a group of
-// four candidates always fits.
+// A lane's survivor queue: entries slot[0], slot[64], ... (a wave's lanes side by side, so the
+// entries of one lane lie at constant distances), the next free one at wp.  Candidates are
+// written unconditionally and kept by advancing wp, and the queue is drained whenever a lane has
+// fewer than four free entries (wp > room4), so a group of four candidates always fits.
+constexpr uint32_t kQueueStride = 64;
+using LdsWord = __attribute__((address_space(3))) uint32_t;  // 32-bit pointers
 struct LaneQueue {
-  uint32_t* slot;   // this lane's first entry
-  uint32_t* wp;     // next free entry
-  uint32_t* room4;  // last position of wp that leaves four free entries
-  uint32_t stride;  // threads per block
+  LdsWord* slot;   // this lane's first entry
+  LdsWord* wp;     // next free entry
+  LdsWord* room4;  // last position of wp that leaves four free entries
 };
 
-// A pass's per-neighbour work: ld(e) loads what the body needs of neighbour e besides its
-// position (issued one survivor ahead), f(e, x, dx, dy, dz, d2) is the body.
-template <class L, class F>
-struct Body {
-  L& ld;
-  F& f;
+// What a walk does with the survivors besides running the body: nothing, or keep their indices
+// (ListRecorder below).
+struct NoRecorder {
+  bool odd = false;
+  __device__ __forceinline__ void granule(const uint32_t*) {}
+  __device__ __forceinline__ void rest(const uint32_t*, uint32_t) {}
 };
 
-// One survivor's body: the reference's d2 (unfused) and the pass's work.
-template <class B, class X>
-__device__ __forceinline__ void body_at(const float4 p, uint32_t e, const float4 o, const X& x,
-                                        B& b)
-{
-  const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-  const float d2 = dx * dx + dy * dy + dz * dz;
-  b.f(e, x, dx, dy, dz, d2);
-}
-
-// Process the lane's queued survivors in order, loading survivor k+1 while computing k.
-// Unrolled by two over two register sets, so no survivor's data is copied from one set to
-// the other between bodies.
-template <bool CL, class B>
+// Runs the body on the lane's queued survivors four at a time, in order: four indices, four
+// positions and the pass's data in flight together, then four bodies in a row without a loop
+// or a copy between them.  The up to three left over move to the front of the queue.
+//
+// Bound by VALU issue (78% of the density pass's cycles on the 1,048,576-particle dam break) and
+// the L1's address rate (72%).  With two register sets alternating, a branch out of each body and
+// two remainder forms in place, a survivor took about 97 VALU instructions, 25 of them copies,
+// and the drain was inlined 15 times; now 67, and three copies.  Density pass 203 -> 196 us
+// literal, 202 -> 197 us stable (968,375 particles), 120 -> 101 us over 24 uneven scenes.
+template <class B, class R>
 __device__ __forceinline__ void drain(LaneQueue& q, const float4 p, const float4* __restrict__ pred,
-                                      const PbfConsts& c, B& b)
+                                      B& b, R& rec)
 {
-  const uint32_t* rp = q.slot;
-  if (rp != q.wp) {
-    uint32_t e0 = *rp;
-    float4 o0 = ldn<CL>(pred, e0, c);
-    auto x0 = b.ld(e0);
-    for (;;) {
-      rp += q.stride;
-      bool more = rp != q.wp;
-      const uint32_t e1 = *(more ? rp : q.slot);  // in bounds either way
-      const float4 o1 = ldn<CL>(pred, e1, c);
-      const auto x1 = b.ld(e1);
-      body_at(p, e0, o0, x0, b);
-      if (!more)
-        break;
-      rp += q.stride;
-      more = rp != q.wp;
-      e0 = *(more ? rp : q.slot);
-      o0 = ldn<CL>(pred, e0, c);
-      x0 = b.ld(e0);
-      body_at(p, e1, o1, x1, b);
-      if (!more)
-        break;
+  const LdsWord* rp = q.slot;
+  while (rp + 4u * kQueueStride <= q.wp) {
+    uint32_t e[4];
+    float4 o[4];
+    typename B::Data x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      e[j] = rp[j * kQueueStride];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      o[j] = ldn(pred, e[j]);
+      x[j] = b.ld(e[j]);
     }
+    rec.granule(e);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      b.add(b.template term<true>(p, o[j], x[j], rec.odd));
+    rp += 4u * kQueueStride;
   }
-  q.wp = q.slot;
+  LdsWord* wp = q.slot;
+#pragma unroll
+  for (int j = 0; j < 3; ++j)
+    if (rp < q.wp) {
+      *wp = *rp;
+      rp += kQueueStride;
+      wp += kQueueStride;
+    }
+  asm("" : "+v"(wp));
+  q.wp = wp;
 }
 
-// Queue candidate e unless its contribution is provably +-0 (r >= h from the squared
-// distance); very far (d2 >= kFarD2) and NaN distances are queued for the exact
-// expressions.  The test uses the fused squared distance against bounds widened by 2^-20
-// relative, so it never skips what the unfused one keeps; the few extra candidates it
-// keeps contribute exact zeros, which leave every sum (started at +0) unchanged.
-template <bool CL>
-__device__ __forceinline__ void offer(LaneQueue& q, const float4 p, const float4 o, uint32_t e,
-                                      const PbfConsts& c)
+// ... and on the rest of them, after the walk (fewer than four once drained).
+template <class B, class R>
+__device__ __forceinline__ void drain_rest(LaneQueue& q, const float4 p,
+                                           const float4* __restrict__ pred, B& b, R& rec)
+{
+  drain(q, p, pred, b, rec);
+  const uint32_t m = (uint32_t)(q.wp - q.slot) / kQueueStride;
+  uint32_t e[3] = {};
+  float4 o[3];
+  typename B::Data x[3];
+#pragma unroll
+  for (uint32_t j = 0; j < 3u; ++j)
+    if (j < m) {
+      e[j] = q.slot[j * kQueueStride];
+      o[j] = ldn(pred, e[j]);
+      x[j] = b.ld(e[j]);
+    }
+  rec.rest(e, m);
+#pragma unroll
+  for (uint32_t j = 0; j < 3u; ++j)
+    if (j < m)
+      b.add(b.template term<true>(p, o[j], x[j], rec.odd));
+}
+
+// Whether candidate o may contribute to p: false only if its contribution is provably +-0 (r >= h
+// from the squared distance); very far (d2 >= kFarD2) and NaN distances stay for the exact
+// expressions.  The test takes the fused squared distance less a bound 2^-20 above the exact one
+// (its sum of three fused terms is off by at most 3 half ulps of the larger of the two, the
+// unfused distance by 4), so it never drops what the unfused one keeps; the few extra candidates
+// contribute exact zeros, which leave every sum (started at +0) unchanged.  One unsigned
+// comparison of the bits covers both ends: a negative difference (the sign bit), one at least
+// as large as the far bound, infinity and NaN all lie at or above farBits.
+__device__ __forceinline__ bool near_or_far(const float4 p, const float4 o, const PbfConsts& c)
 {
   const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-  const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-  const bool keep = !(d2 >= c.cullFused && d2 < c.farFused);
-  *q.wp = e;
-  q.wp += keep ? q.stride : 0u;
+  const float t = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, -c.cullFused)));
+  return __float_as_uint(t) >= c.farBits;
 }
 
-// When any lane of the wave is short of room, every active lane drains: a drain costs the
-// wave one body per entry of its fullest lane, so draining the others with it is free
-// progress.  Drain timing does not change any lane's order of survivors.
-template <bool CL, class B>
-__device__ __forceinline__ void make_room(LaneQueue& q, const float4 p,
-                                          const float4* __restrict__ pred, const PbfConsts& c, B& b)
+__device__ __forceinline__ void push(LaneQueue& q, bool keep, uint32_t e)
 {
-  if (__builtin_amdgcn_ballot_w64(q.wp > q.room4) != 0)
-    drain<CL>(q, p, pred, c, b);
+  *q.wp = e;
+  q.wp += keep ? kQueueStride : 0u;
 }
 
-// Candidates lo..hi (inclusive) in index order, four loads in flight at a time.
-template <bool CL, class B>
+// Candidates lo..hi (inclusive) in index order, four loads in flight at a time.  Every lane of
+// the walk runs the loop until the longest range of the wave is done (its own candidates only
+// while it has some), so that all of them drain together: when any lane is short of room the
+// others' entries ride along with the fullest lane's.  Drain timing does not change any lane's
+// order of survivors.  The last group may read up to three positions past hi (the buffers have
+// them, kPosPad); they are not kept.
+template <class B, class R, class LD>
 __device__ __forceinline__ void scan_range(uint32_t lo, uint32_t hi, LaneQueue& q, const float4 p,
                                            const float4* __restrict__ pred, const PbfConsts& c,
-                                           B& b)
+                                           B& b, R& rec, LD&& at)
 {
+  if (__builtin_amdgcn_ballot_w64(lo <= hi) == 0)
+    return;
   uint32_t e = lo;
-  for (; e + 3u <= hi; e += 4u) {
-    const float4* g = pred + e;
-    const float4 o0 = ldn<CL>(g, 0u, c), o1 = ldn<CL>(g, 1u, c), o2 = ldn<CL>(g, 2u, c),
-                 o3 = ldn<CL>(g, 3u, c);
-    offer<CL>(q, p, o0, e, c);
-    offer<CL>(q, p, o1, e + 1u, c);
-    offer<CL>(q, p, o2, e + 2u, c);
-    offer<CL>(q, p, o3, e + 3u, c);
-    make_room<CL>(q, p, pred, c, b);
-  }
-  for (; e <= hi; ++e)
-    offer<CL>(q, p, ldn<CL>(pred, e, c), e, c);
-  make_room<CL>(q, p, pred, c, b);
+  do {
+    if (e <= hi) {
+      const uint32_t left = hi - e;
+      float4 o[4];
+      at(e, o);
+      bool k0 = near_or_far(p, o[0], c), k1 = near_or_far(p, o[1], c),
+           k2 = near_or_far(p, o[2], c), k3 = near_or_far(p, o[3], c);
+      if (__builtin_amdgcn_ballot_w64(left < 3u) != 0) {
+        k1 &= left >= 1u;
+        k2 &= left >= 2u;
+        k3 &= left >= 3u;
+      }
+      push(q, k0, e);
+      push(q, k1, e + 1u);
+      push(q, k2, e + 2u);
+      push(q, k3, e + 3u);
+    }
+    e += 4u;
+    if (__builtin_amdgcn_ballot_w64(q.wp > q.room4) != 0)
+      drain(q, p, pred, b, rec);
+  } while (__builtin_amdgcn_ballot_w64(e <= hi) != 0);
 }
 
 // ------------------------------------------------------------------ wave tiles in LDS
@@ -187,7 +210,7 @@ constexpr uint32_t kWaves = kMaxBlock / 64;
 // What a neighbour walk works with besides the particle arrays: its lane's survivor queue
 // in LDS and, optionally, the wave's tile.  The kernel owns (and sizes) both.
 struct WalkCtx {
-  uint32_t* qslot = nullptr;               // this lane's queue column
+  LdsWord* qslot = nullptr;                // this lane's queue: its first entry
   uint32_t qcap = 0;
   bool on = false;                         // a tile is staged
   int32_t x0 = 0, y0 = 0, nx = 0, ny = 0;  // staged columns: [x0, x0+nx) x [y0, y0+ny)
@@ -222,8 +245,7 @@ __device__ __forceinline__ int32_t wave_max(int32_t v)
 }
 
 // Stage the wave's tile.  Every lane of the wave must call this (with its own position p,
-// clamped on load when CL, as the pass will see it); positions are staged the same way.
-template <bool CL>
+// as the pass will see it).
 __device__ __forceinline__ void build_tile(const float4 p, const float4* __restrict__ pred,
                                            const uint2* __restrict__ se, const PbfConsts& c,
                                            TileLds& lds, WalkCtx& T)
@@ -295,7 +317,7 @@ __device__ __forceinline__ void build_tile(const float4 p, const float4* __restr
   for (int32_t k = 0; k < ncol; ++k) {
     const uint32_t g0 = __shfl(first, k, 64), sz = __shfl(size, k, 64), o = __shfl(off, k, 64);
     for (uint32_t t = lane; t < sz; t += 64u) {
-      const float4 q = ldp<CL>(pred, g0 + t, c);
+      const float4 q = pred[g0 + t];
       lds.x[w][o + t] = q.x;
       lds.y[w][o + t] = q.y;
       lds.z[w][o + t] = q.z;
@@ -310,47 +332,35 @@ __device__ __forceinline__ void build_tile(const float4 p, const float4* __restr
   T.z = lds.z[w];
 }
 
-// Candidates lo..hi read from the tile; the staged entry of candidate e is e - shift.
-template <bool CL, class B>
-__device__ __forceinline__ void scan_tile(uint32_t lo, uint32_t hi, uint32_t shift,
-                                          const WalkCtx& T, LaneQueue& q, const float4 p,
-                                          const float4* __restrict__ pred, const PbfConsts& c,
-                                          B& b)
-{
-  uint32_t e = lo;
-  for (; e + 3u <= hi; e += 4u) {
-    const uint32_t t = e - shift;
-    const float4 o0 = make_float4(T.x[t], T.y[t], T.z[t], 0.0f);
-    const float4 o1 = make_float4(T.x[t + 1u], T.y[t + 1u], T.z[t + 1u], 0.0f);
-    const float4 o2 = make_float4(T.x[t + 2u], T.y[t + 2u], T.z[t + 2u], 0.0f);
-    const float4 o3 = make_float4(T.x[t + 3u], T.y[t + 3u], T.z[t + 3u], 0.0f);
-    offer<CL>(q, p, o0, e, c);
-    offer<CL>(q, p, o1, e + 1u, c);
-    offer<CL>(q, p, o2, e + 2u, c);
-    offer<CL>(q, p, o3, e + 3u, c);
-    make_room<CL>(q, p, pred, c, b);
-  }
-  for (; e <= hi; ++e) {
-    const uint32_t t = e - shift;
-    offer<CL>(q, p, make_float4(T.x[t], T.y[t], T.z[t], 0.0f), e, c);
-  }
-  make_room<CL>(q, p, pred, c, b);
-}
-
-// One index range of column (nx, ny): from the tile when staged, else from global memory.
-template <bool CL, class B>
+// One index range of column (nx, ny): from the tile when the lanes' ranges are staged, else from
+// global memory.  The staged entry of candidate e is e - T.lo[k] + T.off[k].
+template <class B, class R>
 __device__ __forceinline__ void scan_any(uint32_t lo, uint32_t hi, const WalkCtx& T, int32_t k,
                                          LaneQueue& q, const float4 p,
                                          const float4* __restrict__ pred, const PbfConsts& c,
-                                         B& b)
+                                         B& b, R& rec)
 {
-  if (lo > hi)
-    return;
-  if (k >= 0 && lo >= T.lo[k] && hi <= T.hi[k]) {
-    scan_tile<CL>(lo, hi, T.lo[k] - T.off[k], T, q, p, pred, c, b);
-    return;
+  if (T.on) {
+    const bool staged = lo <= hi && k >= 0 && lo >= T.lo[k] && hi <= T.hi[k];
+    const uint32_t shift = staged ? T.lo[k] - T.off[k] : 0u;
+    scan_range(staged ? lo : 1u, staged ? hi : 0u, q, p, pred, c, b, rec, [&](uint32_t e, float4* o) {
+#pragma unroll
+      for (uint32_t j = 0; j < 4u; ++j) {
+        const uint32_t t = min(e + j, hi) - shift;
+        o[j] = make_float4(T.x[t], T.y[t], T.z[t], 0.0f);
+      }
+    });
+    if (staged) {
+      lo = 1u;
+      hi = 0u;
+    }
   }
-  scan_range<CL>(lo, hi, q, p, pred, c, b);
+  scan_range(lo, hi, q, p, pred, c, b, rec, [&](uint32_t e, float4* o) {
+    const float4* g = pred + e;
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j)
+      o[j] = ldn(g, j);
+  });
 }
 
 // Visit the candidates of particle position p in the reference's order: 27 cells, x
@@ -358,14 +368,13 @@ __device__ __forceinline__ void scan_any(uint32_t lo, uint32_t hi, const WalkCtx
 // The three cells of one z-column are scanned as a single index range whenever the cell
 // table shows their non-empty ranges are back to back (always, unless a cell was capped or
 // the column wraps) -- the same candidates in the same order with one loop instead of three.
-// The queue is drained after every x-slab of nine cells.
-template <bool CL, class L, class F>
+template <class B, class R>
 __device__ __forceinline__ void walk_cells(const float4 p, const float4* __restrict__ pred,
-                                           const uint2* __restrict__ se, const PbfConsts& c,
-                                           L& ld, F& f, const WalkCtx& T)
+                                           const uint2* __restrict__ se, const PbfConsts& c, B& b,
+                                           R& rec, const WalkCtx& T)
 {
-  Body<L, F> b{ ld, f };
-  LaneQueue q{ T.qslot, T.qslot, T.qslot + (T.qcap - 4u) * blockDim.x, blockDim.x };
+  LaneQueue q{ T.qslot, T.qslot, T.qslot + (T.qcap - 4u) * kQueueStride };
+  asm("" : "+v"(q.wp));  // a pointer of its own, not slot plus an offset (an addition a push)
   uint32_t cx, cy, cz;
   cell3d(p, c.g, cx, cy, cz);
   const int32_t rx = c.g.res[0], ry = c.g.res[1], rz = c.g.res[2];
@@ -400,98 +409,116 @@ __device__ __forceinline__ void walk_cells(const float4 p, const float4* __restr
         if (dxc >= 0 && dxc < T.nx && dyc >= 0 && dyc < T.ny)
           k = dxc * T.ny + dyc;
       }
-      if (ok) {
-        scan_any<CL>(lo, hi, T, k, q, p, pred, c, b);
-      } else {
-        scan_any<CL>(ca.x, ca.y, T, k, q, p, pred, c, b);
-        scan_any<CL>(cb.x, cb.y, T, k, q, p, pred, c, b);
-        scan_any<CL>(cd.x, cd.y, T, k, q, p, pred, c, b);
+      // one range, or three in the lanes whose ranges are not back to back
+      uint2 r = ok ? make_uint2(lo, hi) : ca;
+      for (int m = 0;; ++m) {
+        scan_any(r.x, r.y, T, k, q, p, pred, c, b, rec);
+        if (m == 2 || __builtin_amdgcn_ballot_w64(!ok) == 0)
+          break;
+        r = ok ? make_uint2(1u, 0u) : (m == 0 ? cb : cd);
       }
     }
-    drain<CL>(q, p, pred, c, b);
   }
+  drain_rest(q, p, pred, b, rec);
 }
 
-// Run a recorded survivor list: the same body calls, in the same order, as the walk that
-// recorded it.  Entry k + 1's granule, position and pass data are loaded while entry k is
-// computed (a new granule every fourth entry).  Unrolled by two: odd entries are lanes y or
-// w of the current granule, even ones lanes x (of the next granule) or z, and the two
-// register sets alternate, so nothing is copied between bodies.
-template <bool CL, class B>
+// Keeps a walk's survivors as the thread's list: granules of four as they are drained.
+struct ListRecorder {
+  bool odd = false;
+  uint4* gp;
+  uint4* end;
+  uint32_t stride;
+  uint32_t cnt = 0;
+  __device__ __forceinline__ void granule(const uint32_t* e)
+  {
+    if (gp != end) {
+      *gp = make_uint4(e[0], e[1], e[2], e[3]);
+      gp += stride;
+    }
+    cnt += 4u;
+  }
+  __device__ __forceinline__ void rest(const uint32_t* e, uint32_t m)
+  {
+    if (m != 0u && gp != end)
+      *gp = make_uint4(e[0], e[1], e[2], 0u);
+    cnt += m;
+  }
+};
+
+// Run a recorded survivor list: the same terms, in the same order, as the walk that recorded
+// it.  A granule's four positions and their data are loaded together, the next granule while
+// their bodies run.  The list's last granule may hold fewer than four.  Bound by the L1's address
+// rate and latency; four loads at a time instead of one ahead, and terms without checks, took
+// the 968,375-particle scene's correction from 91 to 79 us, confinement from 119 to 94 and XSPH
+// from 117 to 88 us.
+template <bool CK, class B>
 __device__ __forceinline__ void replay(const uint4* __restrict__ gp, uint32_t stride, uint32_t cnt,
-                                       const float4 p, const float4* __restrict__ pred,
-                                       const PbfConsts& c, B& b)
+                                       const float4 p, const float4* __restrict__ pred, B& b)
 {
+  bool odd = false;
   if (cnt == 0)
     return;
   uint4 v = *gp;
-  uint32_t e0 = v.x;
-  float4 o0 = ldn<CL>(pred, e0, c);
-  auto x0 = b.ld(e0);
-  for (uint32_t k = 1;; k += 2u) {
-    bool more = k < cnt;
-    const uint32_t e1 = !more ? e0 : ((k & 2u) ? v.w : v.y);
-    const float4 o1 = ldn<CL>(pred, e1, c);
-    const auto x1 = b.ld(e1);
-    body_at(p, e0, o0, x0, b);
-    if (!more)
-      break;
-    const uint32_t k2 = k + 1u;
-    more = k2 < cnt;
-    if (more && (k2 & 3u) == 0u) {
+  for (; cnt >= 4u; cnt -= 4u) {
+    const uint32_t e[4] = { v.x, v.y, v.z, v.w };
+    float4 o[4];
+    typename B::Data x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      o[j] = ldn(pred, e[j]);
+      x[j] = b.ld(e[j]);
+    }
+    if (cnt > 4u) {
       gp += stride;
       v = *gp;
     }
-    e0 = !more ? e1 : ((k2 & 2u) ? v.z : v.x);
-    o0 = ldn<CL>(pred, e0, c);
-    x0 = b.ld(e0);
-    body_at(p, e1, o1, x1, b);
-    if (!more)
-      break;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      b.add(b.template term<CK>(p, o[j], x[j], odd));
   }
+  const uint32_t e[3] = { v.x, v.y, v.z };
+  float4 o[3];
+  typename B::Data x[3];
+#pragma unroll
+  for (uint32_t j = 0; j < 3u; ++j)
+    if (j < cnt) {
+      o[j] = ldn(pred, e[j]);
+      x[j] = b.ld(e[j]);
+    }
+#pragma unroll
+  for (uint32_t j = 0; j < 3u; ++j)
+    if (j < cnt)
+      b.add(b.template term<CK>(p, o[j], x[j], odd));
 }
 
 // The neighbour walk of one particle: walk_cells, or (NB == kNbRecord) walk_cells recording
-// every survivor the body runs on into the thread's list, or (NB == kNbReplay) the thread's
-// recorded list when it holds all of them.
-template <bool CL = false, int NB = 0, class L, class F>
+// every survivor into the thread's list, or (NB == kNbReplay) the thread's recorded list when it
+// holds all of them -- with unchecked terms unless the recording met a pair that needs the
+// checks (kNbOdd): the replayed pairs are the recorded ones, at the same positions.
+template <int NB = 0, class B>
 __device__ __forceinline__ void walk27(const float4 p, const float4* __restrict__ pred,
-                                       const uint2* __restrict__ se, const PbfConsts& c, L&& ld,
-                                       F&& f, const WalkCtx& T)
+                                       const uint2* __restrict__ se, const PbfConsts& c, B& b,
+                                       const WalkCtx& T)
 {
   if constexpr (NB == kNbReplay) {
-    const uint32_t cnt = T.nb.count[T.slot];
-    if (cnt <= kNbCap) {
-      Body<L, F> b{ ld, f };
-      replay<CL>(T.nb.list + T.slot, T.nb.stride, cnt, p, pred, c, b);
+    const uint32_t word = T.nb.count[T.slot], cnt = word & ~kNbOdd;
+    if (word <= kNbCap) {
+      replay<false>(T.nb.list + T.slot, T.nb.stride, cnt, p, pred, b);
       return;
     }
-    walk_cells<CL>(p, pred, se, c, ld, f, T);
-  } else if constexpr (NB == kNbRecord) {
-    uint4* gp = T.nb.list + T.slot;
-    uint4* const end = gp + (size_t)(kNbCap / 4u) * T.nb.stride;
-    const uint32_t stride = T.nb.stride;
-    uint32_t cnt = 0, r0 = 0, r1 = 0, r2 = 0, r3 = 0;  // the last four survivors, oldest first
-    auto fr = [&](uint32_t e, auto x, float dx, float dy, float dz, float d2) {
-      r0 = r1;
-      r1 = r2;
-      r2 = r3;
-      r3 = e;
-      ++cnt;
-      if ((cnt & 3u) == 0u && gp != end) {
-        *gp = make_uint4(r0, r1, r2, r3);
-        gp += stride;
-      }
-      f(e, x, dx, dy, dz, d2);
-    };
-    walk_cells<CL>(p, pred, se, c, ld, fr, T);
-    const uint32_t m = cnt & 3u;  // survivors of the last, partial granule
-    if (m != 0u && gp != end)
-      *gp = m == 1u ? make_uint4(r3, 0u, 0u, 0u)
-                    : (m == 2u ? make_uint4(r2, r3, 0u, 0u) : make_uint4(r1, r2, r3, 0u));
-    T.nb.count[T.slot] = cnt;
+    if (cnt <= kNbCap) {
+      replay<true>(T.nb.list + T.slot, T.nb.stride, cnt, p, pred, b);
+      return;
+    }
+  }
+  if constexpr (NB == kNbRecord) {
+    uint4* const gp = T.nb.list + T.slot;
+    ListRecorder rec{ false, gp, gp + (size_t)(kNbCap / 4u) * T.nb.stride, T.nb.stride };
+    walk_cells(p, pred, se, c, b, rec, T);
+    T.nb.count[T.slot] = rec.cnt | (rec.odd ? kNbOdd : 0u);
   } else {
-    walk_cells<CL>(p, pred, se, c, ld, f, T);
+    NoRecorder rec;
+    walk_cells(p, pred, se, c, b, rec, T);
   }
 }
 
@@ -532,46 +559,83 @@ __device__ __forceinline__ float poly6_in(float r, const PbfConsts& c)
   return c.poly6 * cube(c.hh - r * r);
 }
 
-// The distance and spiky gradient of a pair, for kShortSqrtGrad: r = sqrtf(d2) and g = gradSpiky
-// (as grad_spiky(dx, dy, dz, r, 1, c), +-0 for r <= kFloatEps) where `in` (r < h).  With the
-// rooted reciprocal, one remainder correction a quotient and one test for all rare operands a
-// pair's root, reciprocal and quotients take about 20 issue slots fewer than with separate
-// v_sqrt and v_rcp forms.  The general forms serve lanes with a nonzero d2 under 2^-52 (which
-// covers 0 < r <= kFloatEps and the roots' own 2^-96), a nonzero numerator under 2^-90, or a
-// root whose significand is all ones; d2 = 0 gives numerators +-0 and quotients +-0.
-constexpr uint32_t kNearD2 = 0x25800000u;  // 2^-52
-struct PairGrad {
-  float r;
-  bool in;
+// A pair in the short correctly rounded forms: its squared distance, r = sqrtf(d2) and spiky
+// gradient g (grad_spiky(dx, dy, dz, r, 1, c); +-0 for d2 = 0, whose numerators are +-0).  The
+// reciprocal of the root comes from the same estimate and the quotients take one remainder
+// correction, about 20 issue slots fewer than with separate v_sqrt and v_rcp forms.  Right
+// except where where_pair_odd says.
+struct Pair {
+  float d2, r;
+  float nx, ny, nz;  // numerators of g
   Grad g;
 };
-__device__ __forceinline__ PairGrad pair_grad(float dx, float dy, float dz, float d2,
-                                              const PbfConsts& c)
+__device__ __forceinline__ Pair pair_short(const float4 p, const float4 o, const PbfConsts& c)
 {
-  const Root q = root_short(d2);
-  PairGrad o;
-  o.r = q.r;
+  const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
+  Pair k;
+  k.d2 = dx * dx + dy * dy + dz * dz;
+  const Root q = root_short(k.d2);
+  k.r = q.r;
   const float p2 = (c.h - q.r) * (c.h - q.r);
-  const float nx = ((dx * c.spiky) * -3.0f) * p2;
-  const float ny = ((dy * c.spiky) * -3.0f) * p2;
-  const float nz = ((dz * c.spiky) * -3.0f) * p2;
+  k.nx = ((dx * c.spiky) * -3.0f) * p2;
+  k.ny = ((dy * c.spiky) * -3.0f) * p2;
+  k.nz = ((dz * c.spiky) * -3.0f) * p2;
   const float y = root_rcp(q);
-  o.g.x = div_unsigned_zero(nx, q.r, y);
-  o.g.y = div_unsigned_zero(ny, q.r, y);
-  o.g.z = div_unsigned_zero(nz, q.r, y);
-  const bool general = (__float_as_uint(d2) - 1u < kNearD2 - 1u) | tiny_numerator3(nx, ny, nz) |
-                       ones_significand(q.r);
-  if (__builtin_amdgcn_ballot_w64(general) != 0) {
+  k.g.x = div_unsigned_zero(k.nx, q.r, y);
+  k.g.y = div_unsigned_zero(k.ny, q.r, y);
+  k.g.z = div_unsigned_zero(k.nz, q.r, y);
+  return k;
+}
+
+// f() in the lanes whose pair needs the reference's expressions instead: r >= h or NaN (weight 0, NaN when
+// very far), a parameter set without the short forms, a nonzero d2 under 2^-52 (which covers
+// 0 < r <= kFloatEps and the roots' own 2^-96), a nonzero numerator under 2^-90, or a root whose
+// significand is all ones.  Nearly no wave has such a lane, so six instructions decide first
+// whether one may: the low half of the root for its significand, and the smallest numerator
+// against d2 * 2^-38 (at least 2^-90 beyond the near bound, and 0 for a particle's pair with
+// itself, whose numerators are 0), which a pair with one equal coordinate does not pass.
+constexpr uint32_t kNearD2 = 0x25800000u;  // 2^-52
+template <class F>
+__device__ __forceinline__ void where_pair_odd(const Pair& k, bool fast, const PbfConsts& c,
+                                               bool& any, F&& f)
+{
+  const bool near = __float_as_uint(k.d2) - 1u < kNearD2 - 1u;
+  const bool out = !(k.r < c.h);
+  const float m = __builtin_fminf(__builtin_fminf(__builtin_fabsf(k.nx), __builtin_fabsf(k.ny)),
+                                  __builtin_fabsf(k.nz));
+  const bool low = (uint16_t)__float_as_uint(k.r) == 0xffffu;
+  // a ballot each: ored as scalars, one VALU comparison a test
+  if ((__builtin_amdgcn_ballot_w64(near) | __builtin_amdgcn_ballot_w64(out) |
+       __builtin_amdgcn_ballot_w64(m < k.d2 * 0x1p-38f) | __builtin_amdgcn_ballot_w64(low)) != 0 ||
+      !fast) {
     rare_path();
-    if (general) {
-      o.r = __builtin_sqrtf(d2);
-      o.g = Grad{ 0.0f, 0.0f, 0.0f };
-      if (o.r > kFloatEps)
-        o.g = grad_spiky(dx, dy, dz, o.r, 1.0f, c);
+    if (near | out | !fast | tiny_numerator3(k.nx, k.ny, k.nz) | ones_significand(k.r)) {
+      any = true;
+      f();
     }
   }
-  o.in = o.r < c.h;
-  return o;
+}
+
+// The squared distance and r = sqrtf(d2) of a pair in the short form, right unless r >= h
+// or NaN, without short forms, or for a nonzero d2 under 2^-52 (f() in those lanes).
+__device__ __forceinline__ float dist_sq(const float4 p, const float4 o)
+{
+  const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
+  return dx * dx + dy * dy + dz * dz;
+}
+template <class F>
+__device__ __forceinline__ void where_root_odd(float d2, float r, bool fast, const PbfConsts& c,
+                                               bool& any, F&& f)
+{
+  const bool near = __float_as_uint(d2) - 1u < kNearD2 - 1u;
+  const bool out = !(r < c.h);
+  if ((__builtin_amdgcn_ballot_w64(near) | __builtin_amdgcn_ballot_w64(out)) != 0 || !fast) {
+    rare_path();
+    if (near | out | !fast) {
+      any = true;
+      f();
+    }
+  }
 }
 
 // pown for the exponent of the dam-break parameters without the loop.
@@ -598,11 +662,17 @@ __device__ __forceinline__ uint32_t particle_index(int remap)
 
 // ---------------------------------------------------------------------------- kernels
 
+// A lane's first queue entry: each wave has depth x 64 consecutive words.
+__device__ __forceinline__ LdsWord* queue_slot(uint32_t* queue, uint32_t depth)
+{
+  return (LdsWord*)queue + (threadIdx.x >> 6) * depth * kQueueStride + (threadIdx.x & 63u);
+}
+
 // The survivor queue of an untiled neighbour pass.
 #define RTP_PLAIN_CTX(DEPTH)                                 \
   extern __shared__ uint32_t rtpQueue[];                     \
   WalkCtx W;                                                 \
-  W.qslot = &rtpQueue[threadIdx.x];                          \
+  W.qslot = queue_slot(rtpQueue, DEPTH);                     \
   W.qcap = (DEPTH);
 // ... and the survivor lists of thread t (a plain pass's t and po).
 #define RTP_NB_CTX \
@@ -648,7 +718,79 @@ __global__ __launch_bounds__(256) void k_predict(const float4* __restrict__ pos,
 //   kFeatures : also write the 8 warm-start features of the particle
 //   kAccum    : add lambda into la.lamAcc (teacher runs), or start it when la.accumInit
 //   kDensOnly : density only, into `density` (the post-correction residual pass)
-//   kClampIn  : clamp positions on load (first fallback iteration)
+struct DensityBody {
+  using Data = int;
+  struct Term {
+    float w, gx, gy, gz, sq;
+    float t;  // 1 for r < h
+  };
+  const PbfConsts& c;
+  bool fast;
+  float dens = 0.0f, sgx = 0.0f, sgy = 0.0f, sgz = 0.0f, ssq = 0.0f, count = 0.0f;
+  __device__ __forceinline__ int ld(uint32_t) const { return 0; }
+  // CK: with the checks (a replayed list may be known not to need them, walk27)
+  template <bool CK>
+  __device__ __forceinline__ Term term(const float4 p, const float4 o, int, bool& odd) const
+  {
+    // the gradient is +-0 for r <= kFloatEps (the reference adds nothing): no sum changes
+    const Pair k = pair_short(p, o, c);
+    Term u{ poly6_in(k.r, c), k.g.x, k.g.y, k.g.z,
+            k.g.x * k.g.x + k.g.y * k.g.y + k.g.z * k.g.z, 1.0f };
+    if (CK)
+      where_pair_odd(k, fast, c, odd, [&]() {
+        const float r = __builtin_sqrtf(k.d2);
+        const float t = r < c.h ? 1.0f : 0.0f;
+        Grad g{ 0.0f, 0.0f, 0.0f };
+        if (r > kFloatEps)
+          g = grad_spiky(p.x - o.x, p.y - o.y, p.z - o.z, r, t, c);
+        u = Term{ poly6(r, t, c), g.x, g.y, g.z, g.x * g.x + g.y * g.y + g.z * g.z, t };
+      });
+    return u;
+  }
+  __device__ __forceinline__ void add(const Term& u)
+  {
+    dens = dens + u.w;
+    sgx = sgx + u.gx;
+    sgy = sgy + u.gy;
+    sgz = sgz + u.gz;
+    ssq = ssq + u.sq;
+    count += u.t;
+  }
+  __device__ __forceinline__ void quad(bool v, const Term& u)
+  {
+    dens = quad_add(dens, v ? u.w : 0.0f);
+    sgx = quad_add(sgx, v ? u.gx : 0.0f);
+    sgy = quad_add(sgy, v ? u.gy : 0.0f);
+    sgz = quad_add(sgz, v ? u.gz : 0.0f);
+    ssq = quad_add(ssq, v ? u.sq : 0.0f);
+  }
+};
+
+// The density alone (kDensOnly).
+struct DensityOnlyBody {
+  using Data = int;
+  struct Term {
+    float w;
+  };
+  const PbfConsts& c;
+  bool fast;
+  float dens = 0.0f;
+  __device__ __forceinline__ int ld(uint32_t) const { return 0; }
+  template <bool CK>
+  __device__ __forceinline__ Term term(const float4 p, const float4 o, int, bool& odd) const
+  {
+    const float d2 = dist_sq(p, o), rs = root_short(d2).r;
+    Term u{ poly6_in(rs, c) };
+    if (CK)
+      where_root_odd(d2, rs, fast, c, odd, [&]() {
+        const float r = __builtin_sqrtf(d2);
+        u.w = poly6(r, r < c.h ? 1.0f : 0.0f, c);
+      });
+    return u;
+  }
+  __device__ __forceinline__ void add(const Term& u) { dens = dens + u.w; }
+};
+
 template <int MODE>
 __device__ __forceinline__ void density_lambda_body(uint32_t i, const float4* __restrict__ pred,
                                                     const uint2* __restrict__ se,
@@ -657,48 +799,18 @@ __device__ __forceinline__ void density_lambda_body(uint32_t i, const float4* __
                                                     const PbfConsts& c, const LearnArgs& la,
                                                     const WalkCtx& T)
 {
-  constexpr bool CL = (MODE & kClampIn) != 0;
-  const float4 p = ldp<CL>(pred, i, c);
-  float dens = 0.0f, sgx = 0.0f, sgy = 0.0f, sgz = 0.0f, ssq = 0.0f, count = 0.0f;
+  const float4 p = pred[i];
   const bool fast = (c.shortMath & kShortSqrtGrad) != 0;
-  walk27<CL, (MODE & (kNbRecord | kNbReplay))>(p, pred, se, c, [](uint32_t) { return 0; },
-             [&](uint32_t, int, float dx, float dy, float dz, float d2) {
-    if ((MODE & kDensOnly) && fast) {
-      const float r = sqrt_cr(d2);
-      if (r < c.h) {
-        dens = dens + poly6_in(r, c);
-        return;
-      }
-    } else if (fast) {
-      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
-      if (q.in) {
-        dens = dens + poly6_in(q.r, c);
-        if (MODE & kFeatures)
-          count += 1.0f;
-        // gradient +-0 for r <= kFloatEps (the reference adds nothing): no sum changes
-        sgx = sgx + q.g.x;
-        sgy = sgy + q.g.y;
-        sgz = sgz + q.g.z;
-        ssq = ssq + (q.g.x * q.g.x + q.g.y * q.g.y + q.g.z * q.g.z);
-        return;
-      }
-    }
-    const float r = __builtin_sqrtf(d2);
-    const float t = r < c.h ? 1.0f : 0.0f;
-    dens = dens + poly6(r, t, c);
-    if (MODE & kFeatures)
-      count += t;
-    if (!(MODE & kDensOnly) && r > kFloatEps) {
-      const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-      sgx = sgx + g.x;
-      sgy = sgy + g.y;
-      sgz = sgz + g.z;
-      ssq = ssq + (g.x * g.x + g.y * g.y + g.z * g.z);
-    }
-  }, T);
-  density[i] = dens;
-  if (MODE & kDensOnly)
+  if constexpr ((MODE & kDensOnly) != 0) {
+    DensityOnlyBody b{ c, fast };
+    walk27(p, pred, se, c, b, T);
+    density[i] = b.dens;
     return;
+  }
+  DensityBody b{ c, fast };
+  walk27<(MODE & (kNbRecord | kNbReplay))>(p, pred, se, c, b, T);
+  const float dens = b.dens, sgx = b.sgx, sgy = b.sgy, sgz = b.sgz, ssq = b.ssq, count = b.count;
+  density[i] = dens;
   const float C = dens / c.p.restDensity - 1.0f;
   float sq = ssq + (sgx * sgx + sgy * sgy + sgz * sgz);
   sq = sq / c.rho0sq;
@@ -755,7 +867,6 @@ __global__ __launch_bounds__(256) void k_density_lambda(const float4* __restrict
 //   kNextIter : fld_applyBoundaryCondition of the next iteration
 //   kLastVel  : fld_updateVel (:263-273) and, without vorticity, fld_updatePosition (:444-450)
 //   kLastOnly : nothing more (the learned step updates the velocity after its fallback)
-// MODE bit kClampIn as for k_density_lambda.
 // The cell the next pass's walk starts from, the key of the next thread order.
 __device__ __forceinline__ void record_cell(uint32_t i, const float4 q, const PbfConsts& c,
                                             const PassOrder& po)
@@ -800,6 +911,49 @@ __device__ __forceinline__ void correct_out(uint32_t i, const float4 p, float cx
     posOut[i] = q;
 }
 
+struct CorrectBody {
+  using Data = float;
+  struct Term {
+    float x, y, z;
+  };
+  const PbfConsts& c;
+  const float* __restrict__ lambda;
+  bool fast;
+  float li, ywdq;
+  float cx = 0.0f, cy = 0.0f, cz = 0.0f;
+  __device__ __forceinline__ float ld(uint32_t e) const { return lambda[e]; }
+  template <bool CK>
+  __device__ __forceinline__ Term term(const float4 p, const float4 o, float le, bool& odd) const
+  {
+    const Pair k = pair_short(p, o, c);
+    const float s = li + le + art_pressure_in(poly6_in(k.r, c), ywdq, c);
+    Term u{ s * k.g.x, s * k.g.y, s * k.g.z };
+    if (CK)
+      where_pair_odd(k, fast, c, odd, [&]() {
+        const float r = __builtin_sqrtf(k.d2);
+        const float t = r < c.h ? 1.0f : 0.0f;
+        const float sg = li + le + art_pressure(poly6(r, t, c), c);
+        Grad g{ 0.0f, 0.0f, 0.0f };  // gradSpiky returns the zero vector for r <= kFloatEps
+        if (r > kFloatEps)
+          g = grad_spiky(p.x - o.x, p.y - o.y, p.z - o.z, r, t, c);
+        u = Term{ sg * g.x, sg * g.y, sg * g.z };
+      });
+    return u;
+  }
+  __device__ __forceinline__ void add(const Term& u)
+  {
+    cx = cx + u.x;
+    cy = cy + u.y;
+    cz = cz + u.z;
+  }
+  __device__ __forceinline__ void quad(bool v, const Term& u)
+  {
+    cx = quad_add(cx, v ? u.x : 0.0f);
+    cy = quad_add(cy, v ? u.y : 0.0f);
+    cz = quad_add(cz, v ? u.z : 0.0f);
+  }
+};
+
 template <int MODE>
 __device__ __forceinline__ void correct_body(uint32_t i, const float4* __restrict__ pred,
                                              const float* __restrict__ lambda,
@@ -811,39 +965,11 @@ __device__ __forceinline__ void correct_body(uint32_t i, const float4* __restric
                                              const WalkCtx& T, const PassOrder& po)
 {
   (void)la;
-  constexpr bool CL = (MODE & kClampIn) != 0;
-  const float4 p = ldp<CL>(pred, i, c);
-  const float li = lambda[i];
-  float cx = 0.0f, cy = 0.0f, cz = 0.0f;
-  const bool fast = (c.shortMath & kShortSqrtGrad) != 0;
+  const float4 p = pred[i];
   const float ywdq = (c.shortMath & kShortArtDiv) ? rcp_refined(c.wdq) : 0.0f;
-  walk27<CL, (MODE & (kNbRecord | kNbReplay))>(p, pred, se, c, [&](uint32_t e) { return lambda[e]; },
-             [&](uint32_t, float le, float dx, float dy, float dz, float d2) {
-    if (fast) {
-      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
-      if (q.in) {
-        const float s = li + le + art_pressure_in(poly6_in(q.r, c), ywdq, c);
-        cx = cx + s * q.g.x;
-        cy = cy + s * q.g.y;
-        cz = cz + s * q.g.z;
-        return;
-      }
-    }
-    const float r = __builtin_sqrtf(d2);
-    const float t = r < c.h ? 1.0f : 0.0f;
-    const float s = li + le + art_pressure(poly6(r, t, c), c);
-    if (r > kFloatEps) {
-      const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-      cx = cx + s * g.x;
-      cy = cy + s * g.y;
-      cz = cz + s * g.z;
-    } else {  // gradSpiky returns the zero vector
-      cx = cx + s * 0.0f;
-      cy = cy + s * 0.0f;
-      cz = cz + s * 0.0f;
-    }
-  }, T);
-  correct_out(i, p, cx, cy, cz, predOut, pos, vel, posOut, last, c, po);
+  CorrectBody b{ c, lambda, (c.shortMath & kShortSqrtGrad) != 0, lambda[i], ywdq };
+  walk27<(MODE & (kNbRecord | kNbReplay))>(p, pred, se, c, b, T);
+  correct_out(i, p, b.cx, b.cy, b.cz, predOut, pos, vel, posOut, last, c, po);
 }
 
 template <int MODE>
@@ -1109,37 +1235,39 @@ __device__ __forceinline__ uint32_t quad_ranges(const float4 p, const uint2* __r
 
 // Runs the body over survivors 0..cnt-1 of the quad (src(k): survivor k), four at a time
 // (lane u: survivors u, u + 4, ...), loading each round's data during the previous round's
-// bodies; rec(v, k, e) sees every round first.  The wave loops until its longest quad is
+// bodies; rec(v, k, e) sees every round first.  CK: terms with the checks; returns whether one
+// of the lane's needed them.  The wave loops until its longest quad is
 // done; empty lanes run the body on the particle itself and add +0.
-template <class S, class R, class B>
-__device__ __forceinline__ void quad_run(uint32_t cnt, uint32_t self, const float4 p,
-                                         const float4* __restrict__ pred, const PbfConsts& c,
-                                         S&& src, R&& rec, B& b)
+template <bool CK, class S, class R, class B>
+__device__ __forceinline__ bool quad_run(uint32_t cnt, uint32_t self, const float4 p,
+                                         const float4* __restrict__ pred, S&& src, R&& rec, B& b)
 {
+  bool odd = false;
   const uint32_t u = threadIdx.x & 3u;
   bool v = u < cnt;
   uint32_t e = v ? src(u) : self;
-  float4 o = ldn<false>(pred, e, c);
+  float4 o = ldn(pred, e);
   auto x = b.ld(e);
   for (uint32_t k = u; __builtin_amdgcn_ballot_w64(k - u < cnt) != 0; k += 4u) {
     const uint32_t k1 = k + 4u;
     const bool v1 = k1 < cnt;
     const uint32_t e1 = v1 ? src(k1) : self;
-    const float4 o1 = ldn<false>(pred, e1, c);
+    const float4 o1 = ldn(pred, e1);
     const auto x1 = b.ld(e1);
     rec(v, k, e);
-    b.add(v, p, o, x);
+    b.quad(v, b.template term<CK>(p, o, x, odd));
     v = v1;
     e = e1;
     o = o1;
     x = x1;
   }
+  return odd;
 }
 
 // The quad's walk over its nr ranges rl (in LDS): candidates are queued (the test of offer)
 // and the queues drained by quad_run whenever one of the wave's quads has fewer than 16
 // free entries, and at the end.  With REC the survivors go to the quad's survivor list
-// (slot `slot`, the first kNbCap of them) and their number to its count.
+// (slot `slot`, the first kNbCap of them) and their number, with kNbOdd, to its count.
 template <bool REC, class B>
 __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t* q,
                                           uint32_t self, const float4 p,
@@ -1148,6 +1276,7 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
 {
   const uint32_t u = threadIdx.x & 3u, below = (1u << u) - 1u;
   uint32_t ri = 0, cur = 1u, hi = 0u, qn = 0, tot = 0;
+  bool odd = false;
   if (nr > 0) {
     const uint2 r = rl[0];
     cur = r.x;
@@ -1155,11 +1284,11 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
   }
   auto drain = [&]() {
     wave_sync();
-    quad_run(qn, self, p, pred, c, [&](uint32_t k) { return q[k]; },
-             [&](bool v, uint32_t k, uint32_t e) {
-               if (REC && v & record & (tot + k < kNbCap))
-                 *nb_word(nb, slot, tot + k) = e;
-             }, b);
+    odd |= quad_run<true>(qn, self, p, pred, [&](uint32_t k) { return q[k]; },
+                          [&](bool v, uint32_t k, uint32_t e) {
+                            if (REC && v & record & (tot + k < kNbCap))
+                              *nb_word(nb, slot, tot + k) = e;
+                          }, b);
     tot += qn;
     qn = 0;
     wave_sync();
@@ -1172,10 +1301,7 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
     for (int j = 0; j < 4; ++j) {
       e[j] = cur + u + 4u * (uint32_t)j;
       const bool valid = act & (e[j] <= hi);
-      const float4 o = ldn<false>(pred, valid ? e[j] : self, c);
-      const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-      const float d2 = __builtin_fmaf(dz, dz, __builtin_fmaf(dy, dy, dx * dx));
-      keep[j] = valid & !((d2 >= c.cullFused) & (d2 < c.farFused));
+      keep[j] = valid & near_or_far(p, ldn(pred, valid ? e[j] : self), c);
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1197,97 +1323,15 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
       drain();
   }
   drain();
-  if (REC && record && u == 0u)
-    nb.count[slot] = tot;
+  if (REC) {
+    const bool any = quad_bits(odd) != 0u;
+    if (record && u == 0u)
+      nb.count[slot] = tot | (any ? kNbOdd : 0u);
+  }
 }
 
-// density_lambda_body's sums (MODE 0) as quad terms.
-struct QuadDensity {
-  const PbfConsts& c;
-  bool fast;
-  float dens = 0.0f, sgx = 0.0f, sgy = 0.0f, sgz = 0.0f, ssq = 0.0f;
-  __device__ __forceinline__ int ld(uint32_t) const { return 0; }
-  __device__ __forceinline__ void add(bool v, const float4 p, const float4 o, int)
-  {
-    const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-    const float d2 = dx * dx + dy * dy + dz * dz;
-    float w = 0.0f, gx = 0.0f, gy = 0.0f, gz = 0.0f, sq = 0.0f;
-    bool done = false;
-    if (fast) {
-      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
-      done = q.in;
-      w = poly6_in(q.r, c);
-      gx = q.g.x;
-      gy = q.g.y;
-      gz = q.g.z;
-      sq = gx * gx + gy * gy + gz * gz;
-    }
-    if (!done) {
-      const float r = __builtin_sqrtf(d2);
-      const float t = r < c.h ? 1.0f : 0.0f;
-      gx = gy = gz = sq = 0.0f;
-      w = poly6(r, t, c);
-      if (r > kFloatEps) {  // else the reference adds no gradient: +0 here
-        const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-        gx = g.x;
-        gy = g.y;
-        gz = g.z;
-        sq = gx * gx + gy * gy + gz * gz;
-      }
-    }
-    dens = quad_add(dens, v ? w : 0.0f);
-    sgx = quad_add(sgx, v ? gx : 0.0f);
-    sgy = quad_add(sgy, v ? gy : 0.0f);
-    sgz = quad_add(sgz, v ? gz : 0.0f);
-    ssq = quad_add(ssq, v ? sq : 0.0f);
-  }
-};
-
-// correct_body's sums as quad terms.
-struct QuadCorrect {
-  const PbfConsts& c;
-  const float* __restrict__ lambda;
-  bool fast;
-  float li, ywdq;
-  float cx = 0.0f, cy = 0.0f, cz = 0.0f;
-  __device__ __forceinline__ float ld(uint32_t e) const { return lambda[e]; }
-  __device__ __forceinline__ void add(bool v, const float4 p, const float4 o, float le)
-  {
-    const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-    const float d2 = dx * dx + dy * dy + dz * dz;
-    float tx = 0.0f, ty = 0.0f, tz = 0.0f;
-    bool done = false;
-    if (fast) {
-      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
-      done = q.in;
-      const float s = li + le + art_pressure_in(poly6_in(q.r, c), ywdq, c);
-      tx = s * q.g.x;
-      ty = s * q.g.y;
-      tz = s * q.g.z;
-    }
-    if (!done) {
-      const float r = __builtin_sqrtf(d2);
-      const float t = r < c.h ? 1.0f : 0.0f;
-      const float s = li + le + art_pressure(poly6(r, t, c), c);
-      if (r > kFloatEps) {
-        const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-        tx = s * g.x;
-        ty = s * g.y;
-        tz = s * g.z;
-      } else {  // gradSpiky returns the zero vector
-        tx = s * 0.0f;
-        ty = s * 0.0f;
-        tz = s * 0.0f;
-      }
-    }
-    cx = quad_add(cx, v ? tx : 0.0f);
-    cy = quad_add(cy, v ? ty : 0.0f);
-    cz = quad_add(cz, v ? tz : 0.0f);
-  }
-};
-
 // density_lambda_body's outputs (MODE 0) from a quad's sums.
-__device__ __forceinline__ void density_lambda_out(uint32_t i, const QuadDensity& b,
+__device__ __forceinline__ void density_lambda_out(uint32_t i, const DensityBody& b,
                                                    float* __restrict__ density,
                                                    float* __restrict__ lambda, const PbfConsts& c)
 {
@@ -1310,10 +1354,14 @@ __device__ __forceinline__ void quad_neighbours(bool on, uint32_t i, uint32_t sl
   const uint32_t g = threadIdx.x >> 2;
   bool listed = false;
   if constexpr (NB == kNbReplay) {
-    const uint32_t lc = on ? nb.count[slot] : 0u;
+    const uint32_t word = on ? nb.count[slot] : 0u, lc = word & ~kNbOdd;
     listed = on & (lc <= kNbCap);
-    quad_run(listed ? lc : 0u, i, p, pred, c, [&](uint32_t m) { return *nb_word(nb, slot, m); },
-             [](bool, uint32_t, uint32_t) {}, b);
+    const bool plain = word == lc;  // unchecked terms, as in walk27
+    auto src = [&](uint32_t m) { return *nb_word(nb, slot, m); };
+    auto none = [](bool, uint32_t, uint32_t) {};
+    quad_run<false>(listed & plain ? lc : 0u, i, p, pred, src, none, b);
+    if (__builtin_amdgcn_ballot_w64(listed & !plain) != 0)
+      quad_run<true>(listed & !plain ? lc : 0u, i, p, pred, src, none, b);
   }
   const uint32_t nr = (on & !listed) ? quad_ranges(p, se, c.g, lds.ranges[g]) : 0u;
   // a recording walk writes every recorded count, also of a particle without candidates
@@ -1338,8 +1386,8 @@ __global__ __launch_bounds__(kQuadBlock) void k_density_lambda_quad(
     const uint32_t k = base + g;
     const bool on = k < cnt;
     const uint32_t i = on ? (k < cs ? fs.list[k] : fs.halo[k - cs]) : 0u;
-    const float4 p = ldp<false>(pred, i, c);
-    QuadDensity b{ c, fast };
+    const float4 p = pred[i];
+    DensityBody b{ c, fast };
     quad_neighbours<REC ? kNbRecord : 0>(on, i, k, on & (k < cs), p, pred, se, c, nb, lds, b);
     if (on && (threadIdx.x & 3u) == 0u)
       density_lambda_out(i, b, density, lambda, c);
@@ -1365,8 +1413,8 @@ __global__ __launch_bounds__(kQuadBlock) void k_correct_quad(
     const uint32_t k = base + g;
     const bool on = k < cnt;
     const uint32_t i = on ? fs.list[k] : 0u;
-    const float4 p = ldp<false>(pred, i, c);
-    QuadCorrect b{ c, lambda, fast, lambda[i], ywdq };
+    const float4 p = pred[i];
+    CorrectBody b{ c, lambda, fast, lambda[i], ywdq };
     quad_neighbours<REPLAY ? kNbReplay : 0>(on, i, k, false, p, pred, se, c, nb, lds, b);
     if (on && (threadIdx.x & 3u) == 0u)
       correct_out(i, p, b.cx, b.cy, b.cz, predOut, nullptr, nullptr, nullptr, last, c, po);
@@ -1403,6 +1451,52 @@ __global__ __launch_bounds__(256) void k_update_vel(const float4* __restrict__ p
 
 // fld_computeVorticity (fluids.cl:278-324).  The w lane of the output carries
 // fast_length(vort) for the confinement pass.
+struct VorticityBody {
+  using Data = float4;
+  struct Term {
+    float x, y, z;
+  };
+  const PbfConsts& c;
+  const float4* __restrict__ vel;
+  bool fast;
+  float4 vi;
+  float wx = 0.0f, wy = 0.0f, wz = 0.0f;
+  __device__ __forceinline__ float4 ld(uint32_t e) const { return ldn(vel, e); }
+  template <bool CK>
+  __device__ __forceinline__ Term term(const float4 p, const float4 o, const float4 ve,
+                                       bool& odd) const
+  {
+    const Pair k = pair_short(p, o, c);
+    const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
+    const Grad g = k.g;
+    // for r <= kFloatEps nothing is added: g is +-0 there and the velocities are finite (the
+    // velocity update clamps them), so the term is +-0
+    Term u{ ay * g.z - az * g.y, az * g.x - ax * g.z, ax * g.y - ay * g.x };
+    if (CK)
+      where_pair_odd(k, fast, c, odd, [&]() {
+        const float r = __builtin_sqrtf(k.d2);
+        u = Term{ 0.0f, 0.0f, 0.0f };
+        if (r > kFloatEps) {
+          const Grad s = grad_spiky(p.x - o.x, p.y - o.y, p.z - o.z, r, r < c.h ? 1.0f : 0.0f, c);
+          u = Term{ ay * s.z - az * s.y, az * s.x - ax * s.z, ax * s.y - ay * s.x };
+        }
+      });
+    return u;
+  }
+  __device__ __forceinline__ void add(const Term& u)
+  {
+    wx = wx + u.x;
+    wy = wy + u.y;
+    wz = wz + u.z;
+  }
+  __device__ __forceinline__ void quad(bool v, const Term& u)
+  {
+    wx = quad_add(wx, v ? u.x : 0.0f);
+    wy = quad_add(wy, v ? u.y : 0.0f);
+    wz = quad_add(wz, v ? u.z : 0.0f);
+  }
+};
+
 template <int NB = 0>
 __device__ __forceinline__ void vorticity_body(uint32_t i, const float4* __restrict__ pred,
                                                const uint2* __restrict__ se,
@@ -1411,34 +1505,9 @@ __device__ __forceinline__ void vorticity_body(uint32_t i, const float4* __restr
                                                const WalkCtx& T)
 {
   const float4 p = pred[i];
-  const float4 vi = vel[i];
-  float wx = 0.0f, wy = 0.0f, wz = 0.0f;
-  const bool fast = (c.shortMath & kShortSqrtGrad) != 0;
-  walk27<false, NB>(p, pred, se, c, [&](uint32_t e) { return vel[e]; },
-         [&](uint32_t, const float4 ve, float dx, float dy, float dz, float d2) {
-    if (fast) {
-      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
-      if (q.in) {
-        const Grad g = q.g;
-        const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
-        const bool on = q.r > kFloatEps;  // else nothing is added, whatever the velocities
-        wx = on ? wx + (ay * g.z - az * g.y) : wx;
-        wy = on ? wy + (az * g.x - ax * g.z) : wy;
-        wz = on ? wz + (ax * g.y - ay * g.x) : wz;
-        return;
-      }
-    }
-    const float r = __builtin_sqrtf(d2);
-    if (r > kFloatEps) {
-      const float t = r < c.h ? 1.0f : 0.0f;
-      const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-      const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
-      wx = wx + (ay * g.z - az * g.y);
-      wy = wy + (az * g.x - ax * g.z);
-      wz = wz + (ax * g.y - ay * g.x);
-    }
-  }, T);
-  vort[i] = make_float4(wx, wy, wz, __builtin_sqrtf(wx * wx + wy * wy + wz * wz));
+  VorticityBody b{ c, vel, (c.shortMath & kShortSqrtGrad) != 0, vel[i] };
+  walk27<NB>(p, pred, se, c, b, T);
+  vort[i] = make_float4(b.wx, b.wy, b.wz, __builtin_sqrtf(b.wx * b.wx + b.wy * b.wy + b.wz * b.wz));
 }
 
 template <int NB>
@@ -1480,6 +1549,47 @@ __device__ __forceinline__ void confinement_out(uint32_t i, float nx, float ny, 
 
 // fld_applyVorticityConfinement (fluids.cl:329-377), writing the confined velocity to
 // velOut (the copy fld_applyXsphViscosityCorrection reads, Fluids.cpp:451).
+struct ConfinementBody {
+  using Data = float;
+  struct Term {
+    float x, y, z;
+  };
+  const PbfConsts& c;
+  const float4* __restrict__ vort;
+  bool fast;
+  float nx = 0.0f, ny = 0.0f, nz = 0.0f;
+  __device__ __forceinline__ float ld(uint32_t e) const { return vort[e].w; }
+  template <bool CK>
+  __device__ __forceinline__ Term term(const float4 p, const float4 o, float le, bool& odd) const
+  {
+    const Pair k = pair_short(p, o, c);
+    const float l = k.r > kFloatEps ? le : 0.0f;  // else nothing is added, whatever le
+    Term u{ l * k.g.x, l * k.g.y, l * k.g.z };
+    if (CK)
+      where_pair_odd(k, fast, c, odd, [&]() {
+        const float r = __builtin_sqrtf(k.d2);
+        u = Term{ 0.0f, 0.0f, 0.0f };
+        if (r > kFloatEps) {
+          const Grad g = grad_spiky(p.x - o.x, p.y - o.y, p.z - o.z, r, r < c.h ? 1.0f : 0.0f, c);
+          u = Term{ le * g.x, le * g.y, le * g.z };
+        }
+      });
+    return u;
+  }
+  __device__ __forceinline__ void add(const Term& u)
+  {
+    nx = nx + u.x;
+    ny = ny + u.y;
+    nz = nz + u.z;
+  }
+  __device__ __forceinline__ void quad(bool v, const Term& u)
+  {
+    nx = quad_add(nx, v ? u.x : 0.0f);
+    ny = quad_add(ny, v ? u.y : 0.0f);
+    nz = quad_add(nz, v ? u.z : 0.0f);
+  }
+};
+
 template <int NB = 0>
 __device__ __forceinline__ void confinement_body(uint32_t i, const float4* __restrict__ pred,
                                                  const uint2* __restrict__ se,
@@ -1489,30 +1599,9 @@ __device__ __forceinline__ void confinement_body(uint32_t i, const float4* __res
                                                  const WalkCtx& T)
 {
   const float4 p = pred[i];
-  float nx = 0.0f, ny = 0.0f, nz = 0.0f;
-  const bool fast = (c.shortMath & kShortSqrtGrad) != 0;
-  walk27<false, NB>(p, pred, se, c, [&](uint32_t e) { return vort[e].w; },
-         [&](uint32_t, float l, float dx, float dy, float dz, float d2) {
-    if (fast) {
-      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
-      if (q.in) {
-        const bool on = q.r > kFloatEps;  // else nothing is added, whatever l
-        nx = on ? nx + l * q.g.x : nx;
-        ny = on ? ny + l * q.g.y : ny;
-        nz = on ? nz + l * q.g.z : nz;
-        return;
-      }
-    }
-    const float r = __builtin_sqrtf(d2);
-    if (r > kFloatEps) {
-      const float t = r < c.h ? 1.0f : 0.0f;
-      const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-      nx = nx + l * g.x;
-      ny = ny + l * g.y;
-      nz = nz + l * g.z;
-    }
-  }, T);
-  confinement_out(i, nx, ny, nz, vort, vel, velOut, c);
+  ConfinementBody b{ c, vort, (c.shortMath & kShortSqrtGrad) != 0 };
+  walk27<NB>(p, pred, se, c, b, T);
+  confinement_out(i, b.nx, b.ny, b.nz, vort, vel, velOut, c);
 }
 
 template <int NB>
@@ -1532,6 +1621,44 @@ __global__ __launch_bounds__(256) void k_confinement(const float4* __restrict__ 
 }
 
 // fld_applyXsphViscosityCorrection (fluids.cl:383-430) + fld_updatePosition (:444-450).
+struct XsphBody {
+  using Data = float4;
+  struct Term {
+    float x, y, z;
+  };
+  const PbfConsts& c;
+  const float4* __restrict__ velIn;
+  bool fast;
+  float4 vi;
+  float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+  __device__ __forceinline__ float4 ld(uint32_t e) const { return ldn(velIn, e); }
+  template <bool CK>
+  __device__ __forceinline__ Term term(const float4 p, const float4 o, const float4 ve,
+                                       bool& odd) const
+  {
+    const float d2 = dist_sq(p, o), rs = root_short(d2).r;
+    float w = poly6_in(rs, c);
+    if (CK)
+      where_root_odd(d2, rs, fast, c, odd, [&]() {
+        const float r = __builtin_sqrtf(d2);
+        w = poly6(r, r < c.h ? 1.0f : 0.0f, c);
+      });
+    return Term{ (ve.x - vi.x) * w, (ve.y - vi.y) * w, (ve.z - vi.z) * w };
+  }
+  __device__ __forceinline__ void add(const Term& u)
+  {
+    sx = sx + u.x;
+    sy = sy + u.y;
+    sz = sz + u.z;
+  }
+  __device__ __forceinline__ void quad(bool v, const Term& u)
+  {
+    sx = quad_add(sx, v ? u.x : 0.0f);
+    sy = quad_add(sy, v ? u.y : 0.0f);
+    sz = quad_add(sz, v ? u.z : 0.0f);
+  }
+};
+
 template <int NB = 0>
 __device__ __forceinline__ void xsph_body(uint32_t i, const float4* __restrict__ pred,
                                           const uint2* __restrict__ se,
@@ -1541,19 +1668,10 @@ __device__ __forceinline__ void xsph_body(uint32_t i, const float4* __restrict__
 {
   const float4 p = pred[i];
   const float4 vi = velIn[i];
-  float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-  const bool fast = (c.shortMath & kShortSqrtGrad) != 0;
-  walk27<false, NB>(p, pred, se, c, [&](uint32_t e) { return velIn[e]; },
-         [&](uint32_t, const float4 ve, float, float, float, float d2) {
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
-    const float t = r < c.h ? 1.0f : 0.0f;
-    const float w = (fast && r < c.h) ? poly6_in(r, c) : poly6(r, t, c);
-    sx = sx + (ve.x - vi.x) * w;
-    sy = sy + (ve.y - vi.y) * w;
-    sz = sz + (ve.z - vi.z) * w;
-  }, T);
+  XsphBody b{ c, velIn, (c.shortMath & kShortSqrtGrad) != 0, vi };
+  walk27<NB>(p, pred, se, c, b, T);
   const float k = c.p.xsphViscosityCoeff;
-  velOut[i] = make_float4(vi.x + k * sx, vi.y + k * sy, vi.z + k * sz, 0.0f);
+  velOut[i] = make_float4(vi.x + k * b.sx, vi.y + k * b.sy, vi.z + k * b.sz, 0.0f);
   posOut[i] = make_float4(p.x, p.y, p.z, 0.0f);
 }
 
@@ -1579,106 +1697,6 @@ __global__ __launch_bounds__(256) void k_xsph(const float4* __restrict__ pred,
 // same sums in the same order.  For scenes too small to give every SIMD several waves with
 // one lane per particle.
 
-// vorticity_body's sums as quad terms.
-struct QuadVorticity {
-  const PbfConsts& c;
-  const float4* __restrict__ vel;
-  bool fast;
-  float4 vi;
-  float wx = 0.0f, wy = 0.0f, wz = 0.0f;
-  __device__ __forceinline__ float4 ld(uint32_t e) const { return vel[e]; }
-  __device__ __forceinline__ void add(bool v, const float4 p, const float4 o, const float4 ve)
-  {
-    const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-    const float d2 = dx * dx + dy * dy + dz * dz;
-    float tx = 0.0f, ty = 0.0f, tz = 0.0f;
-    const float ax = ve.x - vi.x, ay = ve.y - vi.y, az = ve.z - vi.z;
-    bool done = false;
-    if (fast) {
-      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
-      const Grad g = q.g;
-      done = q.in;
-      const bool on = q.r > kFloatEps;  // else nothing is added, whatever the velocities
-      tx = on ? ay * g.z - az * g.y : 0.0f;
-      ty = on ? az * g.x - ax * g.z : 0.0f;
-      tz = on ? ax * g.y - ay * g.x : 0.0f;
-    }
-    if (!done) {
-      const float r = __builtin_sqrtf(d2);
-      const float t = r < c.h ? 1.0f : 0.0f;
-      tx = ty = tz = 0.0f;
-      if (r > kFloatEps) {
-        const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-        tx = ay * g.z - az * g.y;
-        ty = az * g.x - ax * g.z;
-        tz = ax * g.y - ay * g.x;
-      }
-    }
-    wx = quad_add(wx, v ? tx : 0.0f);
-    wy = quad_add(wy, v ? ty : 0.0f);
-    wz = quad_add(wz, v ? tz : 0.0f);
-  }
-};
-
-// confinement_body's sums as quad terms.
-struct QuadConfinement {
-  const PbfConsts& c;
-  const float4* __restrict__ vort;
-  bool fast;
-  float nx = 0.0f, ny = 0.0f, nz = 0.0f;
-  __device__ __forceinline__ float ld(uint32_t e) const { return vort[e].w; }
-  __device__ __forceinline__ void add(bool v, const float4 p, const float4 o, float l)
-  {
-    const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-    const float d2 = dx * dx + dy * dy + dz * dz;
-    float tx = 0.0f, ty = 0.0f, tz = 0.0f;
-    bool done = false;
-    if (fast) {
-      const PairGrad q = pair_grad(dx, dy, dz, d2, c);
-      done = q.in;
-      const bool on = q.r > kFloatEps;  // else nothing is added, whatever l
-      tx = on ? l * q.g.x : 0.0f;
-      ty = on ? l * q.g.y : 0.0f;
-      tz = on ? l * q.g.z : 0.0f;
-    }
-    if (!done) {
-      const float r = __builtin_sqrtf(d2);
-      const float t = r < c.h ? 1.0f : 0.0f;
-      tx = ty = tz = 0.0f;
-      if (r > kFloatEps) {
-        const Grad g = grad_spiky(dx, dy, dz, r, t, c);
-        tx = l * g.x;
-        ty = l * g.y;
-        tz = l * g.z;
-      }
-    }
-    nx = quad_add(nx, v ? tx : 0.0f);
-    ny = quad_add(ny, v ? ty : 0.0f);
-    nz = quad_add(nz, v ? tz : 0.0f);
-  }
-};
-
-// xsph_body's sums as quad terms.
-struct QuadXsph {
-  const PbfConsts& c;
-  const float4* __restrict__ velIn;
-  bool fast;
-  float4 vi;
-  float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-  __device__ __forceinline__ float4 ld(uint32_t e) const { return velIn[e]; }
-  __device__ __forceinline__ void add(bool v, const float4 p, const float4 o, const float4 ve)
-  {
-    const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
-    const float d2 = dx * dx + dy * dy + dz * dz;
-    const float r = fast ? sqrt_cr(d2) : __builtin_sqrtf(d2);
-    const float t = r < c.h ? 1.0f : 0.0f;
-    const float w = (fast && r < c.h) ? poly6_in(r, c) : poly6(r, t, c);
-    sx = quad_add(sx, v ? (ve.x - vi.x) * w : 0.0f);
-    sy = quad_add(sy, v ? (ve.y - vi.y) * w : 0.0f);
-    sz = quad_add(sz, v ? (ve.z - vi.z) * w : 0.0f);
-  }
-};
-
 // The quad's thread t, its particle and whether it has one (quads past n stand in for
 // particle 0 and write nothing).
 #define RTP_QUAD_PROLOGUE                                                     \
@@ -1699,8 +1717,8 @@ __global__ __launch_bounds__(kQuadBlock) void k_density_lambda_q(const float4* _
                                                                  PassOrder po)
 {
   RTP_QUAD_PROLOGUE
-  const float4 p = ldp<false>(pred, i, c);
-  QuadDensity b{ c, fast };
+  const float4 p = pred[i];
+  DensityBody b{ c, fast };
   quad_neighbours<NB>(on, i, t, on, p, pred, se, c, po.nb, lds, b);
   if (lead)
     density_lambda_out(i, b, density, lambda, c);
@@ -1718,9 +1736,9 @@ __global__ __launch_bounds__(kQuadBlock) void k_correct_q(const float4* __restri
                                                           int last, PbfConsts c, PassOrder po)
 {
   RTP_QUAD_PROLOGUE
-  const float4 p = ldp<false>(pred, i, c);
+  const float4 p = pred[i];
   const float ywdq = (c.shortMath & kShortArtDiv) ? rcp_refined(c.wdq) : 0.0f;
-  QuadCorrect b{ c, lambda, fast, lambda[i], ywdq };
+  CorrectBody b{ c, lambda, fast, lambda[i], ywdq };
   quad_neighbours<NB>(on, i, t, false, p, pred, se, c, po.nb, lds, b);
   if (lead)
     correct_out(i, p, b.cx, b.cy, b.cz, predOut, pos, vel, posOut, last, c, po);
@@ -1736,7 +1754,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_vorticity_q(const float4* __rest
 {
   RTP_QUAD_PROLOGUE
   const float4 p = pred[i];
-  QuadVorticity b{ c, vel, fast, vel[i] };
+  VorticityBody b{ c, vel, fast, vel[i] };
   quad_neighbours<NB>(on, i, t, on, p, pred, se, c, po.nb, lds, b);
   if (lead)
     vort[i] = make_float4(b.wx, b.wy, b.wz, __builtin_sqrtf(b.wx * b.wx + b.wy * b.wy + b.wz * b.wz));
@@ -1753,7 +1771,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_confinement_q(const float4* __re
 {
   RTP_QUAD_PROLOGUE
   const float4 p = pred[i];
-  QuadConfinement b{ c, vort, fast };
+  ConfinementBody b{ c, vort, fast };
   quad_neighbours<NB>(on, i, t, false, p, pred, se, c, po.nb, lds, b);
   if (lead)
     confinement_out(i, b.nx, b.ny, b.nz, vort, vel, velOut, c);
@@ -1770,7 +1788,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_xsph_q(const float4* __restrict_
 {
   RTP_QUAD_PROLOGUE
   const float4 p = pred[i];
-  QuadXsph b{ c, velIn, fast, velIn[i] };
+  XsphBody b{ c, velIn, fast, velIn[i] };
   quad_neighbours<NB>(on, i, t, false, p, pred, se, c, po.nb, lds, b);
   if (lead) {
     const float k = c.p.xsphViscosityCoeff;
@@ -1783,16 +1801,16 @@ __global__ __launch_bounds__(kQuadBlock) void k_xsph_q(const float4* __restrict_
 // --------------------------------------------------------------- LDS-tiled wrappers
 // Same passes with the wave tiles staged first.  Every lane takes part in staging (lanes
 // past n stand in for the last particle), then only real particles run the pass.
-#define RTP_TILED_PROLOGUE(CLV)                                                \
+#define RTP_TILED_PROLOGUE                                                     \
   __shared__ TileLds tl;                                                       \
   extern __shared__ uint32_t rtpQueue[];                                       \
   const uint32_t t0 = particle_index(remap);                                   \
   const bool active = t0 < n;                                                  \
   const uint32_t i = po.particle(active ? t0 : n - 1u);                        \
   WalkCtx T;                                                                   \
-  T.qslot = &rtpQueue[threadIdx.x];                                            \
+  T.qslot = queue_slot(rtpQueue, qdepth);                                      \
   T.qcap = qdepth;                                                             \
-  build_tile<CLV>(ldp<CLV>(pred, i, c), pred, se, c, tl, T);                   \
+  build_tile(pred[i], pred, se, c, tl, T);                                     \
   __syncthreads();
 
 template <int MODE>
@@ -1803,7 +1821,7 @@ __global__ __launch_bounds__(256) void k_density_lambda_t(const float4* __restri
                                                           PbfConsts c, int remap, LearnArgs la, uint32_t qdepth,
                      PassOrder po)
 {
-  RTP_TILED_PROLOGUE((MODE & kClampIn) != 0)
+  RTP_TILED_PROLOGUE
   if (active)
     density_lambda_body<MODE>(i, pred, se, density, lambda, c, la, T);
 }
@@ -1819,7 +1837,7 @@ __global__ __launch_bounds__(256) void k_correct_t(const float4* __restrict__ pr
                                                    int last, PbfConsts c, int remap, LearnArgs la, uint32_t qdepth,
                      PassOrder po)
 {
-  RTP_TILED_PROLOGUE((MODE & kClampIn) != 0)
+  RTP_TILED_PROLOGUE
   if (active)
     correct_body<MODE>(i, pred, lambda, se, predOut, pos, vel, posOut, last, c, la, T, po);
 }
@@ -1831,7 +1849,7 @@ __global__ __launch_bounds__(256) void k_vorticity_t(const float4* __restrict__ 
                                                      PbfConsts c, int remap, uint32_t qdepth,
                      PassOrder po)
 {
-  RTP_TILED_PROLOGUE(false)
+  RTP_TILED_PROLOGUE
   if (active)
     vorticity_body(i, pred, se, vel, vort, c, T);
 }
@@ -1844,7 +1862,7 @@ __global__ __launch_bounds__(256) void k_confinement_t(const float4* __restrict_
                                                        PbfConsts c, int remap, uint32_t qdepth,
                      PassOrder po)
 {
-  RTP_TILED_PROLOGUE(false)
+  RTP_TILED_PROLOGUE
   if (active)
     confinement_body(i, pred, se, vort, vel, velOut, c, T);
 }
@@ -1857,7 +1875,7 @@ __global__ __launch_bounds__(256) void k_xsph_t(const float4* __restrict__ pred,
                                                 PbfConsts c, int remap, uint32_t qdepth,
                      PassOrder po)
 {
-  RTP_TILED_PROLOGUE(false)
+  RTP_TILED_PROLOGUE
   if (active)
     xsph_body(i, pred, se, velIn, velOut, posOut, c, T);
 }

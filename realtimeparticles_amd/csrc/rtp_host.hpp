@@ -415,7 +415,11 @@ void refresh_pbf_consts(PbfConsts& c)
     c.hi[a] = c.g.absWall[a] - 0.1f;
   }
   c.cullFused = float_above((double)c.cullSq * (1.0 + 0x1p-20));
-  c.farFused = float_below((double)kFarD2 * (1.0 - 0x1p-20));
+  // (below 0 for a cell larger than the far distance: every candidate is kept)
+  const float far = float_below((double)kFarD2 * (1.0 - 0x1p-20) - (double)c.cullFused);
+  c.farBits = 0;
+  if (far > 0.0f)
+    std::memcpy(&c.farBits, &far, sizeof far);
   // The short forms' operand ranges hold for every neighbour with r < h when
   // 2^-7 <= h <= 2^4: r in (1e-8, h), gradient numerators |n| <= 45/(pi h^3) <= 2^25
   // (tiny nonzero ones are checked per neighbour), so quotients in [2^-94, 2^52]; poly6

@@ -48,18 +48,19 @@ struct PbfConsts {
   float gdt;       // -ABS_GRAVITY_ACC_Y * timeStep (fluids.cl:71)
   float lo[3];     // fld_applyBoundaryCondition lower bounds (fluids.cl:437)
   float hi[3];     // upper bounds (fluids.cl:438)
-  // Candidate test on the fused squared distance fma(dz,dz, fma(dy,dy, dx*dx)), which is
-  // within 4 ulp of the reference's unfused one: skipping at fused >= cullFused (cullSq
-  // plus 2^-20 relative) and < farFused (kFarD2 less 2^-20 relative) skips only what the
-  // unfused test would.
+  // Candidate test on t = fma(dz,dz, fma(dy,dy, fma(dx,dx, -cullFused))), cullFused = cullSq plus
+  // 2^-20 relative: a candidate whose t is a number in [0, far) for the float far of the bits
+  // farBits (kFarD2 less 2^-20 relative, less cullFused) has an unfused d2 in [cullSq, kFarD2).
   float cullFused;
-  float farFused;
+  uint32_t farBits;
   int32_t shortMath;  // kShortSqrtGrad | kShortArtDiv: which short correctly rounded forms apply
 };
 
 // Squared distances at and above this take the reference's exact expressions (its
 // zero-weighted poly6 overflows to NaN well above it).
 constexpr float kFarD2 = 1.0e12f;
+// Positions past the last that a neighbour walk's loads of four may read (and drop).
+constexpr uint32_t kPosPad = 3;
 enum ShortMath { kShortSqrtGrad = 1, kShortArtDiv = 2 };
 
 struct BoidsConsts {
@@ -235,7 +236,7 @@ struct LearnArgs {
 // kNbRecord / kNbReplay: the pass records its threads' survivor lists / replays them
 // (NbList below).
 enum PassMode {
-  kFeatures = 1, kAccum = 2, kDensOnly = 4, kClampIn = 8, kNbRecord = 32, kNbReplay = 64
+  kFeatures = 1, kAccum = 2, kDensOnly = 4, kNbRecord = 32, kNbReplay = 64
 };
 // Survivor lists.  Two neighbour passes over the same positions, the same cell table and
 // the same thread order visit the same candidates and run their bodies on the same
@@ -244,9 +245,11 @@ enum PassMode {
 // granule list[(k / 4) * stride + t], so each thread stores four at a time and a wave's
 // stores and loads of one granule row are contiguous -- and their number to count[t].  The
 // second runs its body over the recorded indices instead of walking the cells, or walks
-// when count[t] > kNbCap.  256 entries (1 KiB per thread slot) hold the survivors of the
+// when the number exceeds kNbCap.  count[t] has the bit kNbOdd if a recorded pair needs the
+// neighbour terms' checks.  256 entries (1 KiB per thread slot) hold the survivors of the
 // clumps the dam-break coefficients form, whose cells fill to the cap.
 constexpr uint32_t kNbCap = 256;
+constexpr uint32_t kNbOdd = 0x80000000u;
 struct NbList {
   uint4* list = nullptr;      // kNbCap / 4 x stride granules
   uint32_t* count = nullptr;  // stride words

@@ -414,6 +414,38 @@ def test_short_math_general_lanes_keep_bits():
         gpu.close()
 
 
+@pytest.mark.parametrize("flags,queue", [(0, 8), (8, 8), (13, 16), (29, 24), (64, 16), (72, 16)])
+@pytest.mark.parametrize("n", [1, 3, 61, 127, 1000])
+def test_checked_pairs_in_lists_keep_bits(flags, queue, n):
+    """Pairs that the unchecked terms of a replayed survivor list would get wrong, in models down
+    to one particle (the first few survivors of a list, the last partial wave): coincident
+    particles, distances within a few ulp of h on either side, a squared distance in (0, 2^-52),
+    numerators in (0, 2^-90), and a plane of equal z, whose zero numerators need no check."""
+    h = 0.1
+    rng = np.random.default_rng(n)
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :3] = 0.25 * rng.random((n, 3), dtype=np.float32) + np.float32(0.05)
+    pos[: n // 3, 2] = np.float32(0.15)
+    k = n // 8
+    pos[k: 2 * k, :3] = pos[:k, :3]  # coincident
+    pos[2 * k: 3 * k, :3] = pos[:k, :3]
+    pos[2 * k: 3 * k, 0] += np.float32(h) * (1 + np.arange(-(k // 2), k - k // 2, dtype=np.float32) * np.float32(2.0 ** -23))
+    if n > 8:
+        pos[-1, :3], pos[-2, :3] = (1e-9, 0.2, 0.2), (2e-9, 0.2, 0.2)
+        pos[-3, :3], pos[-4, :3] = (1e-33, 0.1, 0.2), (0.0, 0.15, 0.2)
+    sc = scenes.dam_break((4, 4, 4), (4, 2, 2), (40, 20, 20), seed=1)
+    sc.pos, sc.vel, sc.n, sc.max_n = pos, np.zeros_like(pos), n, 1024
+    for mapping in ("stable", "literal"):
+        gpu, orc = make_pbf_pair(sc, iters=2, **sc.params(mapping))
+        gpu.set_tuning(64, flags, 0, queue)
+        for step in range(1, 4):
+            log(f"checked pairs, n {n}, flags {flags}, {mapping}, step {step}")
+            gpu.update(1)
+            orc.step(1)
+            compare_pbf(gpu, orc, sc.n, step)
+        gpu.close()
+
+
 @pytest.mark.parametrize("box", [(0.2, 0.1, 0.1), (800.0, 400.0, 400.0)])
 def test_general_forms_outside_short_range(box):
     """Effect radius h = 0.005 and h = 20, outside [2^-7, 2^4] where the short correctly
