@@ -1164,17 +1164,25 @@ __global__ __launch_bounds__(256) void k_fb_scatter(float4* __restrict__ pred,
 // SIMDs idle while each wave waits out its own long chain of loads.  Here a particle has a
 // quad of four lanes.  The quad scans its candidates sixteen at a time (lane u takes
 // candidates u, u + 4, u + 8 and u + 12 of each step) into a survivor queue in LDS, in walk
-// order, and then runs the bodies of four survivors at once, one per lane; the four terms
+// order (quad_slots), and then runs the bodies of four survivors at once, one per lane; the four terms
 // enter every sum in walk order (a DPP broadcast within the quad and one add each), so each
 // sum adds the same terms in the same order as walk_cells' one-lane walk.  Lanes without a
 // survivor add +0, which leaves every sum (started at +0) unchanged.
+//
+// Bound by latency where a scene leaves SIMDs with a wave or less (8,192 particles: 512 waves), by
+// VALU issue beyond (131,072 particles: 81% of the density pass's cycles).  Against a quad that
+// found every range in all four lanes, loaded a step's candidates only when it tested them and
+// placed survivors by two ballot shifts and two bit counts each: 17.3 -> 12.8 us at 8,192
+// particles, 45.5 -> 35.6 us at 131,072, and 51 -> 46 us in the 65,536-particle run with lists.
+// Four consecutive candidates a lane would save the byte sums but double the cache lines a load
+// touches (47 us at 131,072).
 constexpr uint32_t kQuadBlock = 64;                // threads per block: one wave, 16 particles
 constexpr uint32_t kQuadGroups = kQuadBlock / 4u;
 constexpr uint32_t kQuadQueue = 64;                // queued survivors per particle
 constexpr uint32_t kQuadRanges = 27;               // index ranges per particle (<= one per cell)
 
 struct QuadLds {
-  uint32_t queue[kQuadGroups][kQuadQueue];
+  uint32_t queue[kQuadGroups][kQuadQueue + 1];  // the last takes what is not kept
   uint2 ranges[kQuadGroups][kQuadRanges];
 };
 
@@ -1186,86 +1194,117 @@ __device__ __forceinline__ uint32_t* nb_word(const NbList& nb, uint32_t s, uint3
 
 // walk_cells' index ranges of position p in its order, empty ones left out: per (x, y)
 // column one range when its non-empty cells are back to back, else one per non-empty cell.
-// Returns their number (at most 27).
+// Lane u of the quad finds columns u, u + 4 and u + 8.  Returns their number (at most 27).
 __device__ __forceinline__ uint32_t quad_ranges(const float4 p, const uint2* __restrict__ se,
                                                 const GridConsts& g, uint2* out)
 {
+  const uint32_t u = threadIdx.x & 3u;
   uint32_t cx, cy, cz;
   cell3d(p, g, cx, cy, cz);
   const int32_t rx = g.res[0], ry = g.res[1], rz = g.res[2];
   const int32_t z0 = wrap((int32_t)cz - 1, rz), z1 = wrap((int32_t)cz, rz),
                 z2 = wrap((int32_t)cz + 1, rz);
+  uint2 cells[3][3];
+#pragma unroll
+  for (uint32_t m = 0; m < 3u; ++m) {
+    const uint32_t k = 4u * m + u;  // column (ix, iy) = (k / 3 - 1, k % 3 - 1)
+    cells[m][0] = cells[m][1] = cells[m][2] = make_uint2(1u, 0u);
+    if (k < 9u) {
+      const uint32_t kx = (k * 11u) >> 5;
+      const int32_t nx = wrap((int32_t)(cx + kx) - 1, rx);
+      const int32_t row = (nx * ry + wrap((int32_t)(cy + k - 3u * kx) - 1, ry)) * rz;
+      cells[m][0] = se[row + z0];
+      cells[m][1] = se[row + z1];
+      cells[m][2] = se[row + z2];
+    }
+  }
   uint32_t nr = 0;
 #pragma unroll
-  for (int ix = -1; ix <= 1; ++ix) {
-    const int32_t nx = wrap((int32_t)cx + ix, rx);
+  for (uint32_t m = 0; m < 3u; ++m) {
+    uint32_t lo = 1u, hi = 0u, cnt = 0;
+    bool ok = true;
 #pragma unroll
-    for (int iy = -1; iy <= 1; ++iy) {
-      const int32_t row = (nx * ry + wrap((int32_t)cy + iy, ry)) * rz;
-      const uint2 cells[3] = { se[row + z0], se[row + z1], se[row + z2] };
-      uint32_t lo = 1u, hi = 0u;
-      bool ok = true;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const uint2 r = cells[k];
-        if (r.x > r.y)
-          continue;
-        if (lo > hi) {
-          lo = r.x;
-          hi = r.y;
-        } else if (r.x == hi + 1u) {
-          hi = r.y;
-        } else {
-          ok = false;
-        }
-      }
-      if (ok) {
-        if (lo <= hi)
-          out[nr++] = make_uint2(lo, hi);
+    for (int k = 0; k < 3; ++k) {
+      const uint2 r = cells[m][k];
+      if (r.x > r.y)
+        continue;
+      ++cnt;
+      if (lo > hi) {
+        lo = r.x;
+        hi = r.y;
+      } else if (r.x == hi + 1u) {
+        hi = r.y;
       } else {
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if (cells[k].x <= cells[k].y)
-            out[nr++] = cells[k];
+        ok = false;
       }
     }
+    if (ok)
+      cnt = min(cnt, 1u);
+    const QuadSum at = quad_sum(cnt);
+    uint2* w = out + nr + at.below;
+    if (ok) {
+      if (cnt != 0u)
+        *w = make_uint2(lo, hi);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (cells[m][k].x <= cells[m][k].y)
+          *w++ = cells[m][k];
+    }
+    nr += at.all;
   }
   return nr;
 }
 
-// Runs the body over survivors 0..cnt-1 of the quad (src(k): survivor k), four at a time
-// (lane u: survivors u, u + 4, ...), loading each round's data during the previous round's
-// bodies; rec(v, k, e) sees every round first.  CK: terms with the checks; returns whether one
-// of the lane's needed them.  The wave loops until its longest quad is
-// done; empty lanes run the body on the particle itself and add +0.
+// Runs the body over survivors 0..cnt-1 of the quad (src(v, k): survivor k, when v), four at a
+// time (lane u: survivors u, u + 4, ...), loading each round's data during the previous round's
+// bodies, in two register sets by turns; rec(v, k, e) sees every round first.  CK: terms with the
+// checks; returns whether one of the lane's needed them.  The wave loops until its longest quad
+// is done; empty lanes run the body on the particle itself and add +0.
 template <bool CK, class S, class R, class B>
 __device__ __forceinline__ bool quad_run(uint32_t cnt, uint32_t self, const float4 p,
                                          const float4* __restrict__ pred, S&& src, R&& rec, B& b)
 {
   bool odd = false;
+  if (__builtin_amdgcn_ballot_w64(cnt != 0u) == 0)
+    return odd;
   const uint32_t u = threadIdx.x & 3u;
-  bool v = u < cnt;
-  uint32_t e = v ? src(u) : self;
-  float4 o = ldn(pred, e);
-  auto x = b.ld(e);
-  for (uint32_t k = u; __builtin_amdgcn_ballot_w64(k - u < cnt) != 0; k += 4u) {
-    const uint32_t k1 = k + 4u;
-    const bool v1 = k1 < cnt;
-    const uint32_t e1 = v1 ? src(k1) : self;
-    const float4 o1 = ldn(pred, e1);
-    const auto x1 = b.ld(e1);
-    rec(v, k, e);
-    b.quad(v, b.template term<CK>(p, o, x, odd));
-    v = v1;
-    e = e1;
-    o = o1;
-    x = x1;
+  uint32_t k = u;
+  struct Round {
+    bool v;
+    uint32_t e;
+    float4 o;
+    typename B::Data x;
+  };
+  auto load = [&](Round& r, uint32_t at) {
+    r.v = at < cnt;
+    r.e = self;
+    if (r.v)
+      r.e = src(at);
+    r.o = ldn(pred, r.e);
+    r.x = b.ld(r.e);
+  };
+  auto run = [&](const Round& r) {
+    rec(r.v, k, r.e);
+    b.quad(r.v, b.template term<CK>(p, r.o, r.x, odd));
+    k += 4u;
+    return __builtin_amdgcn_ballot_w64(k - u < cnt) != 0;
+  };
+  Round r0, r1;
+  load(r0, k);
+  for (;;) {
+    load(r1, k + 4u);
+    if (!run(r0))
+      break;
+    load(r0, k + 4u);
+    if (!run(r1))
+      break;
   }
   return odd;
 }
 
 // The quad's walk over its nr ranges rl (in LDS): candidates are queued (the test of offer)
-// and the queues drained by quad_run whenever one of the wave's quads has fewer than 16
+// and the queues drained by quad_run whenever one of the wave's quads has fewer than 32
 // free entries, and at the end.  With REC the survivors go to the quad's survivor list
 // (slot `slot`, the first kNbCap of them) and their number, with kNbOdd, to its count.
 template <bool REC, class B>
@@ -1274,14 +1313,10 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
                                           const float4* __restrict__ pred, const PbfConsts& c,
                                           B& b, const NbList& nb, uint32_t slot, bool record)
 {
-  const uint32_t u = threadIdx.x & 3u, below = (1u << u) - 1u;
-  uint32_t ri = 0, cur = 1u, hi = 0u, qn = 0, tot = 0;
+  const uint32_t u = threadIdx.x & 3u;
+  uint32_t ri = 0, qn = 0, tot = 0;
   bool odd = false;
-  if (nr > 0) {
-    const uint2 r = rl[0];
-    cur = r.x;
-    hi = r.y;
-  }
+  wave_sync();  // the quad's lanes wrote the ranges
   auto drain = [&]() {
     wave_sync();
     odd |= quad_run<true>(qn, self, p, pred, [&](uint32_t k) { return q[k]; },
@@ -1293,34 +1328,52 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
     qn = 0;
     wave_sync();
   };
-  while (__builtin_amdgcn_ballot_w64(ri < nr) != 0) {
-    const bool act = ri < nr;
-    uint32_t e[4];
-    bool keep[4];
+  // the lane's first candidate of the step and the last of the quad's range (none: 1 and 0)
+  uint32_t e = 1u, hi = 0u;
+  auto range = [&]() {
+    const uint2 r = rl[ri];
+    e = r.x + u;
+    hi = r.y;
+  };
+  auto load = [&](float4* o) {  // also past the range (kPosPad)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      e[j] = cur + u + 4u * (uint32_t)j;
-      const bool valid = act & (e[j] <= hi);
-      keep[j] = valid & near_or_far(p, ldn(pred, valid ? e[j] : self), c);
+    for (uint32_t j = 0; j < 4u; ++j)
+      o[j] = ldn(pred + e, 4u * j);
+  };
+  // tests the step whose positions are in o; the next one's load meanwhile
+  auto step = [&](const float4* o, float4* next) {
+    const uint32_t first = e;
+    const int32_t left = (int32_t)(hi - e);
+    e += 16u;
+    if (ri < nr && e - u > hi) {
+      e = 1u;
+      hi = 0u;
+      if (++ri < nr)
+        range();
     }
+    load(next);
+    bool k[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t m = quad_bits(keep[j]);
-      if (keep[j])
-        q[qn + (uint32_t)__builtin_popcount(m & below)] = e[j];
-      qn += (uint32_t)__builtin_popcount(m);
-    }
-    cur += 16u;
-    if (act & (cur > hi)) {
-      ++ri;
-      if (ri < nr) {
-        const uint2 r = rl[ri];
-        cur = r.x;
-        hi = r.y;
-      }
-    }
-    if (__builtin_amdgcn_ballot_w64(qn > kQuadQueue - 16u) != 0)
-      drain();
+    for (int j = 0; j < 4; ++j)
+      k[j] = near_or_far(p, o[j], c) & (left >= 4 * j);
+    const QuadSlots at = quad_slots(k);
+    uint32_t* const w = q + qn;
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j)
+      *(k[j] ? w + at.slot(j) : q + kQuadQueue) = first + 4u * j;
+    qn += at.all();
+  };
+  if (nr > 0)
+    range();
+  if (__builtin_amdgcn_ballot_w64(nr > 0) != 0) {
+    float4 o0[4], o1[4];
+    load(o0);
+    do {
+      step(o0, o1);
+      step(o1, o0);
+      if (__builtin_amdgcn_ballot_w64(qn > kQuadQueue - 32u) != 0)
+        drain();
+    } while (__builtin_amdgcn_ballot_w64(ri < nr) != 0);
   }
   drain();
   if (REC) {

@@ -121,6 +121,49 @@ __device__ __forceinline__ float quad_add(float s, float t)
   return s + quad_lane<3>(t);
 }
 
+// x of the quad's lane A in lane 0, B in lane 1, C in lane 2 and D in lane 3.
+template <int A, int B, int C, int D>
+__device__ __forceinline__ uint32_t quad_perm(uint32_t x)
+{
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, A | B << 2 | C << 4 | D << 6, 0xF, 0xF, true);
+}
+
+// Sum of x over the quad's lanes below this one, and over all four.
+struct QuadSum {
+  uint32_t below, all;
+};
+__device__ __forceinline__ QuadSum quad_sum(uint32_t x)
+{
+  const uint32_t u = threadIdx.x & 3u;
+  const uint32_t a = quad_perm<0, 0, 1, 2>(x);
+  uint32_t s = x + (u >= 1u ? a : 0u);
+  const uint32_t b = quad_perm<0, 0, 0, 1>(s);
+  s += u >= 2u ? b : 0u;
+  return QuadSum{ s - x, quad_perm<3, 3, 3, 3>(s) };
+}
+
+// Places for what a quad keeps of sixteen items, item u + 4 j being lane u's k[j], in the items'
+// order: the four counts of each lane as bytes of one word, summed over the quad's lanes below
+// and over the bytes below.
+struct QuadSlots {
+  uint32_t at, sum;  // bytes: place of item j, items kept up to and with group j
+  __device__ __forceinline__ uint32_t slot(uint32_t j) const { return (at >> (8u * j)) & 0xffu; }
+  __device__ __forceinline__ uint32_t all() const { return sum >> 24; }
+};
+__device__ __forceinline__ QuadSlots quad_slots(const bool k[4])
+{
+  uint32_t x[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    x[j] = k[j] ? 1u << (8 * j) : 0u;
+    asm("" : "+v"(x[j]));  // one selection each
+  }
+  const QuadSum s = quad_sum(x[0] | x[1] | x[2] | x[3]);
+  uint32_t t = s.all + (s.all << 8);
+  t = t + (t << 16);
+  return QuadSlots{ (t << 8) + s.below, t };
+}
+
 // The quad's four bits of a wave ballot, lane 0 lowest.
 __device__ __forceinline__ uint32_t quad_bits(bool x)
 {
