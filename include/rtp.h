@@ -117,7 +117,9 @@ typedef struct {
                                   order; for scenes too small to fill the GPU one lane per
                                   particle (results unchanged; not with RTP_LAUNCH_LDS_TILES).
                                   The default shape of a model of at most 262,144 particles
-                                  (maxNbParticles) has it; set_tuning / autotune replace it */
+                                  (maxNbParticles) has it, and a fluids model's also
+                                  RTP_LAUNCH_NB_LIST where the device has the memory;
+                                  set_tuning / autotune replace it */
 
 /* Which buffers rtp_fluids_read_field copies. */
 typedef enum {
