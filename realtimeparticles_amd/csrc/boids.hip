@@ -375,15 +375,18 @@ __global__ __launch_bounds__(256) void k_boids_step(const float4* __restrict__ p
 // ------------------------------------------------------------------- the quad walk
 // For flocks too small to fill the GPU with one lane per boid (RTP_LAUNCH_QUAD), each boid
 // gets a quad of four lanes: the quad lists the boid's ranges as boids_sums_queued does (in
-// LDS), scans them sixteen candidates per step (lane u: candidates u, u + 4, u + 8, u + 12),
-// queues the neighbours in walk order, and runs four queued bodies at once, one per lane,
-// adding their terms to every sum in walk order (quad_add).  The sums therefore add the same
-// terms in the same order as one lane's walk.
+// LDS), scans them sixteen candidates per step (lane u: candidates u, u + 4, u + 8, u + 12; the
+// next step's load while one is tested), queues the neighbours in walk order (quad_slots), and
+// runs four queued bodies at once, one per lane, adding their terms to every sum in walk order
+// (quad_add).  The sums therefore add the same terms in the same order as one lane's walk.
+// Bound by latency at 8,192 boids (512 waves), by VALU issue at 131,072.  With the ranges found
+// in every lane, a step's loads waited for and two ballot shifts a candidate the step took 18.0
+// and 97 us; 11.2 and 75 us this way.
 constexpr uint32_t kBoidsQuadGroups = 16;  // boids per 64-lane workgroup
 constexpr uint32_t kBoidsQuadQueue = 64;   // queued neighbours per boid
 
 struct BoidsQuadLds {
-  uint32_t queue[kBoidsQuadGroups][kBoidsQuadQueue];
+  uint32_t queue[kBoidsQuadGroups][kBoidsQuadQueue + 1];  // the last takes what is not kept
   uint2 ranges[kBoidsQuadGroups][kBoidsRanges];
 };
 
@@ -397,10 +400,10 @@ __device__ __forceinline__ void boids_pair_quad(bool v, const float4 p, const fl
   const float y = rcp_refined(sq);
   float qx = div_unsigned_zero(vx, sq, y), qy = div_unsigned_zero(vy, sq, y),
         qz = div_unsigned_zero(vz, sq, y);
-  const bool general = !c.shortDiv || tiny_numerator3(vx, vy, vz);
-  if (__builtin_amdgcn_ballot_w64(general) != 0) {
+  const bool tiny = tiny_numerator3(vx, vy, vz);
+  if (__builtin_amdgcn_ballot_w64(tiny) != 0 || !c.shortDiv) {
     rare_path();
-    if (general) {
+    if (tiny | !c.shortDiv) {
       qx = vx / sq;
       qy = vy / sq;
       qz = vz / sq;
@@ -418,6 +421,63 @@ __device__ __forceinline__ void boids_pair_quad(bool v, const float4 p, const fl
   S.count += __builtin_popcount(quad_bits(v));
 }
 
+// The boid's ranges in walk order into rl (LDS), a z-column's cells as one range when its
+// non-empty ones are back to back; returns their number.  Lane u of the quad finds columns u,
+// u + 4 and u + 8 of the 3-D rules' nine.
+__device__ __forceinline__ uint32_t boids_quad_ranges(const float4 p, const uint2* __restrict__ se,
+                                                      const BoidsConsts& c, uint2* rl)
+{
+  const uint32_t u = threadIdx.x & 3u;
+  uint32_t cx, cy, cz;
+  cell3d(p, c.g, cx, cy, cz);
+  const int32_t rx = c.g.res[0], ry = c.g.res[1], rz = c.g.res[2];
+  uint2 cells[3][3];
+#pragma unroll
+  for (uint32_t m = 0; m < 3u; ++m) {
+    const uint32_t k = 4u * m + u, kx = (k * 11u) >> 5;  // column (k / 3 - 1, k % 3 - 1)
+    const int32_t nx = (int32_t)(cx + kx) - 1, ny = (int32_t)(cy + k - 3u * kx) - 1;
+    const bool in = k < 9u && nx >= 0 && nx < rx && ny >= 0 && ny < ry;
+    const int32_t row = (nx * ry + ny) * rz;
+#pragma unroll
+    for (int iz = 0; iz < 3; ++iz) {
+      const int32_t nz = (int32_t)cz + iz - 1;
+      cells[m][iz] = make_uint2(1u, 0u);
+      if (in && nz >= 0 && nz < rz)
+        cells[m][iz] = se[row + nz];
+    }
+  }
+  uint32_t nr = 0;
+#pragma unroll
+  for (uint32_t m = 0; m < 3u; ++m)
+    nr += quad_column(cells[m], rl + nr, 0u);
+  return nr;
+}
+
+// ... of the 2-D rules' cells, which every lane of the quad lists alike.
+__device__ __forceinline__ uint32_t boids_quad_ranges2d(const float4 p, const uint2* __restrict__ se,
+                                                        const BoidsConsts& c, uint2* rl)
+{
+  uint32_t nr = 0, lo = 1u, hi = 0u;
+  int lastCol = -1;
+  boids_cells<1>(p, c, [&](uint32_t cell, int col, int) {
+    const uint2 r = se[cell];
+    if (r.x > r.y)
+      return;
+    if (col == lastCol && lo <= hi && r.x == hi + 1u) {
+      hi = r.y;
+      return;
+    }
+    if (lo <= hi)
+      rl[nr++] = make_uint2(lo, hi);
+    lo = r.x;
+    hi = r.y;
+    lastCol = col;
+  });
+  if (lo <= hi)
+    rl[nr++] = make_uint2(lo, hi);
+  return nr;
+}
+
 template <int DIM2>
 __device__ __forceinline__ void boids_sums_quad(bool on, uint32_t self, const float4 p,
                                                 const float4* __restrict__ position,
@@ -426,83 +486,97 @@ __device__ __forceinline__ void boids_sums_quad(bool on, uint32_t self, const fl
                                                 const BoidsConsts& c, BoidsQuadLds& lds,
                                                 BoidsSums& S)
 {
-  const uint32_t gq = threadIdx.x >> 2, u = threadIdx.x & 3u, below = (1u << u) - 1u;
+  const uint32_t gq = threadIdx.x >> 2, u = threadIdx.x & 3u;
   uint2* const rl = lds.ranges[gq];
   uint32_t* const q = lds.queue[gq];
-  // the boid's ranges (every lane of the quad lists the same ones)
-  uint32_t nr = 0, e = 1u, hi = 0u;
-  if (on) {
-    uint32_t lo = 1u;
-    int lastCol = -1;
-    boids_cells<DIM2>(p, c, [&](uint32_t cell, int col, int) {
-      const uint2 r = se[cell];
-      if (r.x > r.y)
-        return;
-      if (col == lastCol && lo <= hi && r.x == hi + 1u) {
-        hi = r.y;
-        return;
-      }
-      if (lo <= hi)
-        rl[nr++] = make_uint2(lo, hi);
-      lo = r.x;
-      hi = r.y;
-      lastCol = col;
-    });
-    if (lo <= hi)
-      rl[nr++] = make_uint2(lo, hi);
-    hi = 0u;
-  }
+  uint32_t nr = 0;
+  if (on)
+    nr = DIM2 ? boids_quad_ranges2d(p, se, c, rl) : boids_quad_ranges(p, se, c, rl);
+  if (__builtin_amdgcn_ballot_w64(nr > 0u) == 0)
+    return;
+  wave_sync();
   uint32_t ri = 0, qn = 0;
-  if (nr > 0) {
-    e = rl[0].x;
-    hi = rl[0].y;
-  }
+  struct Round {
+    bool v;
+    float4 q, nv;
+  };
   const auto drain = [&]() {
     wave_sync();
-    bool v = u < qn;
-    uint32_t ev = v ? q[u] : self;
-    float4 qq = position[ev], nv = unitVel[ev];
-    for (uint32_t k = u; __builtin_amdgcn_ballot_w64(k - u < qn) != 0; k += 4u) {
-      const uint32_t k1 = k + 4u;
-      const bool v1 = k1 < qn;
-      const uint32_t e1 = v1 ? q[k1] : self;
-      const float4 q1 = position[e1], nv1 = unitVel[e1];
-      boids_pair_quad(v, p, qq, nv, S, c);
-      v = v1;
-      qq = q1;
-      nv = nv1;
+    uint32_t k = u;
+    const auto load = [&](Round& r, uint32_t at) {
+      r.v = at < qn;
+      uint32_t e = self;
+      if (r.v)
+        e = q[at];
+      r.q = position[e];
+      r.nv = unitVel[e];
+    };
+    const auto run = [&](const Round& r) {
+      boids_pair_quad(r.v, p, r.q, r.nv, S, c);
+      k += 4u;
+      return __builtin_amdgcn_ballot_w64(k - u < qn) != 0;
+    };
+    if (__builtin_amdgcn_ballot_w64(qn != 0u) != 0) {
+      Round r0, r1;
+      load(r0, k);
+      for (;;) {
+        load(r1, k + 4u);
+        if (!run(r0))
+          break;
+        load(r0, k + 4u);
+        if (!run(r1))
+          break;
+      }
     }
     qn = 0;
     wave_sync();
   };
-  while (__builtin_amdgcn_ballot_w64(ri < nr) != 0) {
-    const bool act = ri < nr;
-    uint32_t ej[4];
-    bool kept[4];
+  // the lane's first candidate of the step and the last of the quad's range (none: 1 and 0)
+  uint32_t e = 1u, hi = 0u;
+  const auto range = [&]() {
+    e = rl[ri].x + u;
+    hi = rl[ri].y;
+  };
+  const auto load = [&](float4* o) {  // also past the range (kPosPad)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      ej[j] = e + u + 4u * (uint32_t)j;
-      const bool valid = act & (ej[j] <= hi);
-      kept[j] = valid & boids_near(boids_sq(p, position[valid ? ej[j] : self]), c);
+    for (uint32_t j = 0; j < 4u; ++j) {
+      const float* f = reinterpret_cast<const float*>(position + e + 4u * j);
+      o[j] = make_float4(f[0], f[1], f[2], 0.0f);
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t m = quad_bits(kept[j]);
-      if (kept[j])
-        q[qn + (uint32_t)__builtin_popcount(m & below)] = ej[j];
-      qn += (uint32_t)__builtin_popcount(m);
-    }
+  };
+  // tests the step whose positions are in o; the next one's load meanwhile
+  const auto step = [&](const float4* o, float4* next) {
+    const uint32_t first = e;
+    const int32_t left = (int32_t)(hi - e);
     e += 16u;
-    if (act & (e > hi)) {
-      ++ri;
-      if (ri < nr) {
-        e = rl[ri].x;
-        hi = rl[ri].y;
-      }
+    if (ri < nr && e - u > hi) {
+      e = 1u;
+      hi = 0u;
+      if (++ri < nr)
+        range();
     }
-    if (__builtin_amdgcn_ballot_w64(qn > kBoidsQuadQueue - 16u) != 0)
+    load(next);
+    bool k[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      k[j] = boids_near(boids_sq(p, o[j]), c) & (left >= 4 * j);
+    const QuadSlots at = quad_slots(k);
+    uint32_t* const w = q + qn;
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j)
+      *(k[j] ? w + at.slot(j) : q + kBoidsQuadQueue) = first + 4u * j;
+    qn += at.all();
+  };
+  if (nr > 0)
+    range();
+  float4 o0[4], o1[4];
+  load(o0);
+  do {
+    step(o0, o1);
+    step(o1, o0);
+    if (__builtin_amdgcn_ballot_w64(qn > kBoidsQuadQueue - 32u) != 0)
       drain();
-  }
+  } while (__builtin_amdgcn_ballot_w64(ri < nr) != 0);
   drain();
 }
 

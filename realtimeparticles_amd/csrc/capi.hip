@@ -1398,8 +1398,8 @@ int rtp_boids_create(const rtp_model_desc* d, rtp_boids** out)
     return fail(RTP_ERR_HIP, "hipStreamCreate failed");
   }
   const uint32_t maxN = d->maxNbParticles;
-  if ((rc = h->grid.alloc(maxN)) || (rc = dev_alloc(&h->pos[0], maxN)) ||
-      (rc = dev_alloc(&h->pos[1], maxN)) || (rc = dev_alloc(&h->vel[0], maxN)) ||
+  if ((rc = h->grid.alloc(maxN)) || (rc = dev_alloc(&h->pos[0], maxN + kPosPad)) ||
+      (rc = dev_alloc(&h->pos[1], maxN + kPosPad)) || (rc = dev_alloc(&h->vel[0], maxN)) ||
       (rc = dev_alloc(&h->vel[1], maxN)) || (rc = dev_alloc(&h->acc, maxN)) ||
       (rc = dev_alloc(&h->unitVel, maxN))) {
     h->release();

@@ -1220,39 +1220,8 @@ __device__ __forceinline__ uint32_t quad_ranges(const float4 p, const uint2* __r
   }
   uint32_t nr = 0;
 #pragma unroll
-  for (uint32_t m = 0; m < 3u; ++m) {
-    uint32_t lo = 1u, hi = 0u, cnt = 0;
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const uint2 r = cells[m][k];
-      if (r.x > r.y)
-        continue;
-      ++cnt;
-      if (lo > hi) {
-        lo = r.x;
-        hi = r.y;
-      } else if (r.x == hi + 1u) {
-        hi = r.y;
-      } else {
-        ok = false;
-      }
-    }
-    if (ok)
-      cnt = min(cnt, 1u);
-    const QuadSum at = quad_sum(cnt);
-    uint2* w = out + nr + at.below;
-    if (ok) {
-      if (cnt != 0u)
-        *w = make_uint2(lo, hi);
-    } else {
-#pragma unroll
-      for (int k = 0; k < 3; ++k)
-        if (cells[m][k].x <= cells[m][k].y)
-          *w++ = cells[m][k];
-    }
-    nr += at.all;
-  }
+  for (uint32_t m = 0; m < 3u; ++m)
+    nr += quad_column(cells[m], out + nr, 0u);
   return nr;
 }
 

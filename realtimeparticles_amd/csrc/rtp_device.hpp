@@ -164,6 +164,44 @@ __device__ __forceinline__ QuadSlots quad_slots(const bool k[4])
   return QuadSlots{ (t << 8) + s.below, t };
 }
 
+// The index ranges of each lane's column of three cells (first, last; empty: first > last), the
+// quad's columns in lane order, into out with `tag` in the first indices: one range when the
+// non-empty cells are back to back, else one each.  Returns the quad's number of ranges.
+__device__ __forceinline__ uint32_t quad_column(const uint2 cells[3], uint2* out, uint32_t tag)
+{
+  uint32_t lo = 1u, hi = 0u, cnt = 0;
+  bool ok = true;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const uint2 r = cells[k];
+    if (r.x > r.y)
+      continue;
+    ++cnt;
+    if (lo > hi) {
+      lo = r.x;
+      hi = r.y;
+    } else if (r.x == hi + 1u) {
+      hi = r.y;
+    } else {
+      ok = false;
+    }
+  }
+  if (ok)
+    cnt = min(cnt, 1u);
+  const QuadSum at = quad_sum(cnt);
+  uint2* w = out + at.below;
+  if (ok) {
+    if (cnt != 0u)
+      *w = make_uint2(lo | tag, hi);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      if (cells[k].x <= cells[k].y)
+        *w++ = make_uint2(cells[k].x | tag, cells[k].y);
+  }
+  return at.all;
+}
+
 // The quad's four bits of a wave ballot, lane 0 lowest.
 __device__ __forceinline__ uint32_t quad_bits(bool x)
 {
