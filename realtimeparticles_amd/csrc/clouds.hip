@@ -113,6 +113,7 @@ constexpr uint32_t kNearVv = 0x25800000u;  // 2^-52
 struct CldPair {
   float r;
   float4 g;
+  float w;  // poly6_r(r, c)
 };
 __device__ __forceinline__ CldPair cld_pair(float4 vec, float vv, const PbfConsts& c)
 {
@@ -125,14 +126,23 @@ __device__ __forceinline__ CldPair cld_pair(float4 vec, float vv, const PbfConst
   const float y = root_rcp(q);
   o.g = make_float4(div_unsigned_zero(n.x, q.r, y), div_unsigned_zero(n.y, q.r, y),
                     div_unsigned_zero(n.z, q.r, y), n.w);
-  const bool general = !((c.shortMath & kShortSqrtGrad) != 0 && q.r < c.h) |
-                       (__float_as_uint(vv) - 1u < kNearVv - 1u) | tiny_numerator3(n.x, n.y, n.z) |
-                       ones_significand(q.r);
-  if (__builtin_amdgcn_ballot_w64(general) != 0) {
+  o.w = c.poly6 * cube(c.hh - q.r * q.r);
+  // whether some lane may need the general expressions, as in the fluids' pairs: a root ending
+  // in 16 ones, or a numerator under vv * 2^-38 (at least 2^-90 beyond the near bound)
+  const bool near = __float_as_uint(vv) - 1u < kNearVv - 1u;
+  const bool out = !(q.r < c.h);
+  const bool shortForm = (c.shortMath & kShortSqrtGrad) != 0;
+  const float m = __builtin_fminf(__builtin_fminf(__builtin_fabsf(n.x), __builtin_fabsf(n.y)),
+                                  __builtin_fabsf(n.z));
+  const bool low = (uint16_t)__float_as_uint(q.r) == 0xffffu;
+  if ((__builtin_amdgcn_ballot_w64(near) | __builtin_amdgcn_ballot_w64(out) |
+       __builtin_amdgcn_ballot_w64(m < vv * 0x1p-38f) | __builtin_amdgcn_ballot_w64(low)) != 0 ||
+      !shortForm) {
     rare_path();
-    if (general) {
+    if (near | out | !shortForm | tiny_numerator3(n.x, n.y, n.z) | ones_significand(q.r)) {
       o.r = __builtin_sqrtf(vv);
       o.g = grad_spiky_r(vec, o.r, c);
+      o.w = poly6_r(o.r, c);
     }
   }
   return o;
@@ -231,12 +241,11 @@ __device__ __forceinline__ float4 cld_shift(uint32_t code, const GridConsts& g)
 }
 
 // The non-empty candidate ranges of the 27-cell walk of clouds.cl:322-353 in its order (x
-// outer, z inner), as {first | shift code << 28, last}, every STRIDE-th entry of out from
+// outer, z inner), as {first | shift code << 28, last}, every kCldLanes-th entry of out from
 // out[0]; returns their count.  A wrapped neighbour's position is shifted by the code's
 // +-2 absWall; y cells beyond the walls are skipped.  The three cells of a z-column are one
 // range when none of them wraps in z and their non-empty ranges are back to back (cells are
 // numbered z-minor), which lists the same candidates in the same order.
-template <uint32_t STRIDE = kCldLanes>
 __device__ __forceinline__ uint32_t cld_ranges(const float4 pos, const uint2* __restrict__ se,
                                                const GridConsts& g, uint2* __restrict__ out)
 {
@@ -247,7 +256,7 @@ __device__ __forceinline__ uint32_t cld_ranges(const float4 pos, const uint2* __
   const bool zInside = cz - 1 >= 0 && cz + 1 < rz;
   uint32_t nr = 0;
   const auto push = [&](uint32_t lo, uint32_t hi, uint32_t code) {
-    out[nr * STRIDE] = make_uint2(lo | (code << kCldIndexBits), hi);
+    out[nr * kCldLanes] = make_uint2(lo | (code << kCldIndexBits), hi);
     ++nr;
   };
 #pragma unroll
@@ -479,6 +488,8 @@ __device__ __forceinline__ void cld_flag(bool safe, uint32_t* flags, uint32_t bi
   if (bad != 0 && (threadIdx.x & 63u) == (uint32_t)__builtin_ctzll(bad))
     atomicOr(flags, bit);
 }
+constexpr uint32_t kCldFlagWords = 2u;
+constexpr uint32_t kCldTempWord = 1u;  // nonzero: some temperature is not finite and below 2^60
 constexpr uint32_t kFlagLambdaT = 1u, kFlagVort = 2u, kFlagVelTmp = 4u;
 constexpr uint32_t kFlagLambda0 = 8u;   // iteration k: kFlagLambda0 << k for k < kFlagIters
 constexpr uint32_t kFlagIters = 29u;
@@ -495,6 +506,15 @@ __device__ __forceinline__ bool negligible(float4 vec, const PbfConsts& c)
   return (d2 >= c.cullSq) & (d2 < kFarD2);
 }
 
+// false only for a negligible candidate: its fused squared distance less a bound just above the
+// exact one (without the w lane, which only adds), as bits, for both ends in one comparison;
+// negative, very far, infinite and NaN differences lie at or above farBits.
+__device__ __forceinline__ bool near_or_far(float4 vec, const PbfConsts& c)
+{
+  const float t = __builtin_fmaf(vec.z, vec.z, __builtin_fmaf(vec.y, vec.y, __builtin_fmaf(vec.x, vec.x, -c.cullFused)));
+  return __float_as_uint(t) >= c.farBits;
+}
+
 __device__ __forceinline__ bool finite4(float4 v)
 {
   return __builtin_isfinite(v.x) & __builtin_isfinite(v.y) & __builtin_isfinite(v.z) &
@@ -506,70 +526,148 @@ inline uint32_t blocks_for(uint32_t n, uint32_t b) { return (n + b - 1u) / b; }
 // ------------------------------------------------------------------------ quad walks
 // With quads (the default for scenes up to kQuadDefaultMaxN particles) each walk kernel gives a
 // particle four lanes of a 64-lane workgroup.  The quad builds the particle's ranges
-// (cld_ranges) in LDS and scans them sixteen candidates per step, lane u taking candidates
-// u, u + 4, u + 8 and u + 12 with the pass's keep test; the kept ones go to a queue of
-// kCqQueue entries per particle in LDS, in walk order.  A drain runs four queued bodies at
+// (cq_ranges: cld_ranges with the columns split over its lanes) in LDS and scans them sixteen
+// candidates per step, lane u taking candidates u, u + 4, u + 8 and u + 12 (the next step's load
+// while one is tested); the kept ones go to a queue of kCqQueue entries per particle in LDS, in
+// walk order (quad_slots).  A recording walk tests positions alone: the neighbour data its
+// terms multiply are known to be finite, or else it keeps every candidate (keepAll).  A drain runs four queued bodies at
 // once, one per lane, and adds the four terms into every sum in walk order (quad_add), so
 // each sum adds the same terms in the same order as cld_walk's one-lane walk; lanes
 // without an entry add +0, which leaves a sum started at +0 unchanged.  Survivor lists keep
 // cld_walk's layout and codes, so either kind of walk replays the other's lists.
+//
+// Bound by VALU issue and, with 4,096 waves of which six fit a SIMD, by latency.  With every range
+// found in all four lanes (27 integer remainders), each candidate's data loaded and tested for
+// finiteness, its shift subtracted and its place found by two ballot shifts, the passes over the
+// 65,536-particle cumulus took (now): density 49.6 (42.2) us, temperature 59 (49), vorticity 49 (34).
 constexpr uint32_t kCqGroups = kCldLanes / 4u;  // particles per workgroup
 constexpr uint32_t kCqQueue = 64;               // queued survivors per particle
 
 struct CqLds {
-  uint32_t queue[kCqGroups][kCqQueue];
+  uint32_t queue[kCqGroups][kCqQueue + 1];  // the last takes what is not kept
   uint2 ranges[kCqGroups][kCldRanges];
 };
 
+// cld_ranges for a quad: lane u lists the columns u, u + 4 and u + 8.
+__device__ __forceinline__ uint32_t cq_ranges(const float4 pos, const uint2* __restrict__ se,
+                                              const GridConsts& g, uint2* __restrict__ out)
+{
+  const uint32_t u = threadIdx.x & 3u;
+  uint32_t cx, cy, cz;
+  cell3d(pos, g, cx, cy, cz);
+  const int32_t rx = g.res[0], ry = g.res[1], rz = g.res[2];
+  const auto wrapped = [](int32_t v, int32_t res) {  // v in [-1, res + 1], res 1 included
+    v = wrap(v, res);
+    return v >= res ? v - res : v;
+  };
+  const bool zInside = cz >= 1u && (int32_t)cz + 1 < rz;
+  uint2 cells[3][3];
+  uint32_t tag[3];
+#pragma unroll
+  for (uint32_t m = 0; m < 3u; ++m) {
+    const uint32_t k = 4u * m + u, kx = (k * 11u) >> 5;  // column (k / 3 - 1, k % 3 - 1)
+    const int32_t ax = (int32_t)(cx + kx) - 1, ay = (int32_t)(cy + k - 3u * kx) - 1;
+    tag[m] = (ax >= rx ? 1u : (ax < 0 ? 2u : 0u)) << kCldIndexBits;
+    const bool in = k < 9u && ay >= 0 && ay < ry;
+    const int32_t row = (wrapped(ax, rx) * ry + ay) * rz;
+#pragma unroll
+    for (int iz = 0; iz < 3; ++iz) {
+      cells[m][iz] = make_uint2(1u, 0u);
+      if (in)
+        cells[m][iz] = se[row + wrapped((int32_t)cz + iz - 1, rz)];
+    }
+  }
+  uint32_t nr = 0;
+#pragma unroll
+  for (uint32_t m = 0; m < 3u; ++m) {
+    if (zInside) {  // the same in the quad's four lanes
+      nr += quad_column(cells[m], out + nr, tag[m]);
+    } else {
+      // cells that wrap in z carry their own codes: one range each
+      uint32_t cnt = 0;
+#pragma unroll
+      for (int iz = 0; iz < 3; ++iz)
+        cnt += cells[m][iz].x <= cells[m][iz].y ? 1u : 0u;
+      const QuadSum at = quad_sum(cnt);
+      uint2* w = out + nr + at.below;
+#pragma unroll
+      for (int iz = 0; iz < 3; ++iz) {
+        const int32_t az = (int32_t)cz + iz - 1;
+        const uint32_t zcode = (az >= rz ? 4u : (az < 0 ? 8u : 0u)) << kCldIndexBits;
+        if (cells[m][iz].x <= cells[m][iz].y)
+          *w++ = make_uint2(cells[m][iz].x | tag[m] | zcode, cells[m][iz].y);
+      }
+      nr += at.all;
+    }
+  }
+  return nr;
+}
+
+// vec less the shift of the code's wrapped cell; in a wave without one, vec itself (x - 0 = x).
+__device__ __forceinline__ float4 cq_shifted(float4 vec, uint32_t code, const GridConsts& g)
+{
+  if (__builtin_amdgcn_ballot_w64((code >> kCldIndexBits) != 0u) != 0)
+    vec = sub4(vec, cld_shift(code >> kCldIndexBits, g));
+  return vec;
+}
+
 // The body over entries 0..cnt-1 of the quad (entry(k): entry k, an index with its shift
-// code), four at a time, loading each round's data during the previous round's bodies;
-// rec(v, k, code) sees every round first.  The wave loops until its longest quad is done;
-// lanes without an entry run the body on the particle itself and add +0.
+// code), four at a time, loading each round's data during the previous round's bodies, in two
+// register sets by turns; rec(v, k, code) sees every round first.  The wave loops until its
+// longest quad is done; lanes without an entry run the body on the particle itself and add +0.
 template <class S, class R, class B>
 __device__ __forceinline__ void cq_run(uint32_t cnt, uint32_t self, const float4 pos,
                                        const float4* __restrict__ src, const GridConsts& g,
                                        S&& entry, R&& rec, B& b)
 {
+  if (__builtin_amdgcn_ballot_w64(cnt != 0u) == 0)
+    return;
   const uint32_t u = threadIdx.x & 3u;
-  bool v = u < cnt;
-  uint32_t code = v ? entry(u) : self;
-  float4 o = src[code & kCldIndexMask];
-  auto x = b.ld(code & kCldIndexMask);
-  for (uint32_t k = u; __builtin_amdgcn_ballot_w64(k - u < cnt) != 0; k += 4u) {
-    const uint32_t k1 = k + 4u;
-    const bool v1 = k1 < cnt;
-    const uint32_t code1 = v1 ? entry(k1) : self;
-    const float4 o1 = src[code1 & kCldIndexMask];
-    const auto x1 = b.ld(code1 & kCldIndexMask);
-    rec(v, k, code);
-    b.add(v, x, sub4(sub4(pos, o), cld_shift(code >> kCldIndexBits, g)));
-    v = v1;
-    code = code1;
-    o = o1;
-    x = x1;
+  uint32_t k = u;
+  struct Round {
+    bool v;
+    uint32_t code;
+    float4 o;
+    decltype(b.ld(0u)) x;
+  };
+  const auto load = [&](Round& r, uint32_t at) {
+    r.v = at < cnt;
+    r.code = self;
+    if (r.v)
+      r.code = entry(at);
+    r.o = src[r.code & kCldIndexMask];
+    r.x = b.ld(r.code & kCldIndexMask);
+  };
+  const auto run = [&](const Round& r) {
+    rec(r.v, k, r.code);
+    b.add(r.v, r.x, cq_shifted(sub4(pos, r.o), r.code, g));
+    k += 4u;
+    return __builtin_amdgcn_ballot_w64(k - u < cnt) != 0;
+  };
+  Round r0, r1;
+  load(r0, k);
+  for (;;) {
+    load(r1, k + 4u);
+    if (!run(r0))
+      break;
+    load(r0, k + 4u);
+    if (!run(r1))
+      break;
   }
 }
 
-// The quad's walk of particle `self` over its nr ranges rl (in LDS), queued in q; with REC
-// (and `record`) the kept candidates go to the particle's survivor list.
+// The quad's walk of particle `self` over its nr ranges rl (in LDS), queued in q.  REC: a
+// recording walk (a candidate is kept by its distance, all of them with keepAll), whose kept
+// candidates go to the particle's survivor list when `record`; else the body's own test.
 template <bool REC, class B>
 __device__ __forceinline__ void cq_walk(uint32_t nr, const uint2* rl, uint32_t* q, uint32_t self,
                                         const float4 pos, const float4* __restrict__ src,
                                         const GridConsts& g, B& b, const CldList& list,
-                                        bool record)
+                                        bool record, bool keepAll)
 {
-  const uint32_t u = threadIdx.x & 3u, below = (1u << u) - 1u;
-  uint32_t ri = 0, e = 1u, hi = 0u, tag = 0u, qn = 0, tot = 0;
-  float4 shift = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  const auto range = [&](uint32_t k) {
-    const uint2 r = rl[k];
-    e = r.x & kCldIndexMask;
-    tag = r.x & ~kCldIndexMask;
-    hi = r.y;
-    shift = cld_shift(r.x >> kCldIndexBits, g);
-  };
-  if (nr > 0)
-    range(0);
+  const uint32_t u = threadIdx.x & 3u;
+  uint32_t ri = 0, qn = 0, tot = 0;
+  wave_sync();  // the quad's lanes wrote the ranges
   const auto drain = [&]() {
     wave_sync();
     cq_run(qn, self, pos, src, g, [&](uint32_t k) { return q[k]; },
@@ -581,34 +679,60 @@ __device__ __forceinline__ void cq_walk(uint32_t nr, const uint2* rl, uint32_t* 
     qn = 0;
     wave_sync();
   };
-  while (__builtin_amdgcn_ballot_w64(ri < nr) != 0) {
-    const bool act = ri < nr;
-    uint32_t code[4];
-    bool kept[4];
+  // the lane's first candidate of the step, the last of the quad's range (none: 1 and 0) and
+  // the range's shift code
+  uint32_t e = 1u, hi = 0u, tag = 0u;
+  const auto range = [&]() {
+    const uint2 r = rl[ri];
+    e = (r.x & kCldIndexMask) + u;
+    tag = r.x & ~kCldIndexMask;
+    hi = r.y;
+  };
+  const auto load = [&](float4* o) {  // also past the range (kPosPad)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t ej = e + u + 4u * (uint32_t)j;
-      const bool valid = act & (ej <= hi);
-      const uint32_t at = valid ? ej : self;
-      const float4 o = src[at];
-      kept[j] = valid & b.keep(b.ld(at), sub4(sub4(pos, o), shift));
-      code[j] = ej | tag;
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t m = quad_bits(kept[j]);
-      if (kept[j])
-        q[qn + (uint32_t)__builtin_popcount(m & below)] = code[j];
-      qn += (uint32_t)__builtin_popcount(m);
-    }
+    for (uint32_t j = 0; j < 4u; ++j)
+      o[j] = src[e + 4u * j];
+  };
+  // tests the step whose positions are in o; the next one's load meanwhile
+  const auto step = [&](const float4* o, float4* next) {
+    const uint32_t first = e, code = tag;
+    const int32_t left = (int32_t)(hi - e);
     e += 16u;
-    if (act & (e > hi)) {
-      ++ri;
-      if (ri < nr)
-        range(ri);
+    if (ri < nr && e - u > hi) {
+      e = 1u;
+      hi = 0u;
+      tag = 0u;
+      if (++ri < nr)
+        range();
     }
-    if (__builtin_amdgcn_ballot_w64(qn > kCqQueue - 16u) != 0)
-      drain();
+    load(next);
+    bool k[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 vec = cq_shifted(sub4(pos, o[j]), code, g);
+      if constexpr (REC)
+        k[j] = (keepAll | near_or_far(vec, b.c.f)) & (left >= 4 * j);
+      else
+        k[j] = (left >= 4 * j) && b.keep(b.ld(first + 4u * j), vec);
+    }
+    const QuadSlots at = quad_slots(k);
+    uint32_t* const w = q + qn;
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j)
+      *(k[j] ? w + at.slot(j) : q + kCqQueue) = (first + 4u * j) | code;
+    qn += at.all();
+  };
+  if (nr > 0)
+    range();
+  if (__builtin_amdgcn_ballot_w64(nr > 0u) != 0) {
+    float4 o0[4], o1[4];
+    load(o0);
+    do {
+      step(o0, o1);
+      step(o1, o0);
+      if (__builtin_amdgcn_ballot_w64(qn > kCqQueue - 32u) != 0)
+        drain();
+    } while (__builtin_amdgcn_ballot_w64(ri < nr) != 0);
   }
   drain();
   if (REC && record && u == 0u)
@@ -616,14 +740,14 @@ __device__ __forceinline__ void cq_walk(uint32_t nr, const uint2* rl, uint32_t* 
 }
 
 // The candidates of particle i into the body b: a recording walk (MODE kCqRecord), a
-// replay of its list when useList and the list is complete, else a walk (kCqReplay), or a
-// walk (kCqWalk).
-constexpr int kCqWalk = 0, kCqRecord = 1, kCqReplay = 2;
+// replay of its list when useList and the list is complete, else a walk (kCqReplay).
+constexpr int kCqRecord = 1, kCqReplay = 2;
 template <int MODE, class B>
 __device__ __forceinline__ void cq_neighbours(bool on, uint32_t i, bool useList, const float4 pos,
                                               const float4* __restrict__ src,
                                               const uint2* __restrict__ se, const GridConsts& g,
-                                              const CldList& list, CqLds& lds, B& b)
+                                              const CldList& list, CqLds& lds, B& b,
+                                              bool keepAll = false)
 {
   const uint32_t gq = threadIdx.x >> 2;
   bool listed = false;
@@ -634,10 +758,13 @@ __device__ __forceinline__ void cq_neighbours(bool on, uint32_t i, bool useList,
            [&](uint32_t m) { return list.entry[m * list.stride + i]; },
            [](bool, uint32_t, uint32_t) {}, b);
   }
-  const uint32_t nr = (on & !listed) ? cld_ranges<1>(pos, se, g, lds.ranges[gq]) : 0u;
+  uint32_t nr = 0;
+  if (on & !listed)
+    nr = cq_ranges(pos, se, g, lds.ranges[gq]);
   // a recording walk writes every recorded count, also of a particle without candidates
   if (MODE == kCqRecord || __builtin_amdgcn_ballot_w64(nr > 0u) != 0)
-    cq_walk<MODE == kCqRecord>(nr, lds.ranges[gq], lds.queue[gq], i, pos, src, g, b, list, on);
+    cq_walk<MODE == kCqRecord>(nr, lds.ranges[gq], lds.queue[gq], i, pos, src, g, b, list, on,
+                               keepAll);
 }
 
 // --------------------------------------------------------------------------------- kernels
@@ -680,8 +807,8 @@ __global__ __launch_bounds__(256) void k_cld_thermo(const float4* __restrict__ p
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t < c.f.g.numCells)
     startEnd[t] = make_uint2(1u, 0u);
-  if (t == 0)
-    *flags = 0u;  // the survivor-list flags of this step's passes
+  if (t < kCldFlagWords)
+    flags[t] = 0u;  // the flags of this step's passes
   if (t >= n)
     return;
   const rtp_cloud_params& q = c.q;
@@ -722,8 +849,9 @@ struct CloudGather {
   const float* src[5];
   float* dst[5];
 };
+// src[0] is the temperature, whose word of the flags it sets.
 __global__ __launch_bounds__(256) void k_cld_gather(const uint32_t* __restrict__ idx, uint32_t sortN,
-                                                    CloudGather a)
+                                                    CloudGather a, uint32_t* __restrict__ flags)
 {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= sortN)
@@ -731,8 +859,12 @@ __global__ __launch_bounds__(256) void k_cld_gather(const uint32_t* __restrict__
   const uint32_t j = idx[i];
   a.totOut[i] = a.tot[0][j];
 #pragma unroll
-  for (int k = 0; k < 5; ++k)
-    a.dst[k][i] = a.src[k][j];
+  for (int k = 0; k < 5; ++k) {
+    const float v = a.src[k][j];
+    a.dst[k][i] = v;
+    if (k == 0)
+      cld_flag(cld_safe(v), flags + kCldTempWord, 1u);
+  }
 }
 
 // The outputs of the walk kernels from their sums (shared by the one-lane and quad kernels);
@@ -804,7 +936,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_temp_lambda(const float4* __r
                                                          float* __restrict__ lap,
                                                          float* __restrict__ lambdaT, uint32_t n,
                                                          CloudConsts c, CldList list,
-                                                         uint32_t* __restrict__ flags)
+                                                         uint32_t* __restrict__ flags, int)
 {
   const uint32_t i = logical_block(1) * kCldLanes + threadIdx.x;
   if (i >= n)
@@ -882,7 +1014,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_density_lambda(const float4* 
   const auto keep = [&](int, float4 vec) { return !negligible(vec, c.f); };
   cld_walk_record(i, pos, pred, se, c.f.g, lds, list, [](uint32_t) { return 0; }, keep, [&](uint32_t, int, float4 vec) {
     const CldPair q = cld_pair(vec, dot4(vec, vec), c.f);
-    fluidDensity = fluidDensity + poly6_r(q.r, c.f);
+    fluidDensity = fluidDensity + q.w;
     const float4 grad = q.g;
     sumGradCi = add4(sumGradCi, grad);
     sumSqGradC = sumSqGradC + dot4(grad, grad);
@@ -919,7 +1051,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_correct(const float4* __restr
   cld_walk_replay(i, pos, pred, se, c.f.g, lds, list, useList && bit && !(*flags & bit),
                   [&](uint32_t e) { return lambda[e]; }, keep, [&](uint32_t, float le, float4 vec) {
     const CldPair q = cld_pair(vec, dot4(vec, vec), c.f);
-    const float s = lambdaI + le + art_pressure_w(poly6_r(q.r, c.f), ywdq, c.f);
+    const float s = lambdaI + le + art_pressure_w(q.w, ywdq, c.f);
     corr = add4(corr, muls4(s, q.g));
   });
   cld_correct_out(i, pos, corr, predOut, totCorr, vel, c);
@@ -945,7 +1077,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_vorticity(const float4* __res
                                                        const float4* __restrict__ vel,
                                                        float4* __restrict__ vort, uint32_t n,
                                                        CloudConsts c, CldList list,
-                                                       uint32_t* __restrict__ flags)
+                                                       uint32_t* __restrict__ flags, int)
 {
   const uint32_t i = logical_block(1) * kCldLanes + threadIdx.x;
   if (i >= n)
@@ -1046,8 +1178,15 @@ __global__ __launch_bounds__(256) void k_cld_update_pos(const float4* __restrict
 // s + t component by component in quad order (t counts only when v).
 __device__ __forceinline__ float4 quad_add4(float4 s, bool v, const float4 t)
 {
-  return make_float4(quad_add(s.x, v ? t.x : 0.0f), quad_add(s.y, v ? t.y : 0.0f),
-                     quad_add(s.z, v ? t.z : 0.0f), quad_add(s.w, v ? t.w : 0.0f));
+  s.x = quad_add(s.x, v ? t.x : 0.0f);
+  s.y = quad_add(s.y, v ? t.y : 0.0f);
+  s.z = quad_add(s.z, v ? t.z : 0.0f);
+  // a w lane is +-0, which changes no sum, until some factor is not finite
+  if (__builtin_amdgcn_ballot_w64(!(t.w == 0.0f)) != 0) {
+    rare_path();
+    s.w = quad_add(s.w, v ? t.w : 0.0f);
+  }
+  return s;
 }
 
 struct CqTempLambda {
@@ -1104,7 +1243,7 @@ struct CqDensity {
   __device__ __forceinline__ void add(bool v, int, float4 vec)
   {
     const CldPair q = cld_pair(vec, dot4(vec, vec), c.f);
-    const float w = poly6_r(q.r, c.f);
+    const float w = q.w;
     const float4 grad = q.g;
     const float sq = dot4(grad, grad);
     fluidDensity = quad_add(fluidDensity, v ? w : 0.0f);
@@ -1126,7 +1265,7 @@ struct CqCorrect {
   __device__ __forceinline__ void add(bool v, float le, float4 vec)
   {
     const CldPair q = cld_pair(vec, dot4(vec, vec), c.f);
-    const float s = lambdaI + le + art_pressure_w(poly6_r(q.r, c.f), ywdq, c.f);
+    const float s = lambdaI + le + art_pressure_w(q.w, ywdq, c.f);
     corr = quad_add4(corr, v, muls4(s, q.g));
   }
 };
@@ -1196,12 +1335,14 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_temp_lambda_q(const float4* _
                                                                  float* __restrict__ lambdaT,
                                                                  uint32_t n, CloudConsts c,
                                                                  CldList list,
-                                                                 uint32_t* __restrict__ flags)
+                                                                 uint32_t* __restrict__ flags,
+                                                                 int useList)
 {
   RTP_CQ_PROLOGUE
   const float4 pos = posP[i];
   CqTempLambda b{ c, tempP, tempP[i], c.q.restDensity };
-  cq_neighbours<kCqRecord>(on, i, true, pos, posP, se, c.f.g, list, lds, b);
+  cq_neighbours<kCqRecord>(on, i, true, pos, posP, se, c.f.g, list, lds, b,
+                           !useList || flags[kCldTempWord] != 0u);
   float lt = 0.0f;
   if (lead)
     lt = cld_temp_lambda_out(i, b.laplacian, b.sumGradCi, b.sumSqGradC, lap, lambdaT, c);
@@ -1271,12 +1412,13 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_vorticity_q(const float4* __r
                                                                const float4* __restrict__ vel,
                                                                float4* __restrict__ vort, uint32_t n,
                                                                CloudConsts c, CldList list,
-                                                               uint32_t* __restrict__ flags)
+                                                               uint32_t* __restrict__ flags, int useList)
 {
   RTP_CQ_PROLOGUE
   const float4 pos = pred[i];
+  // the velocities of this step's particles are finite: the velocity update clamped them
   CqVorticity b{ c, vel, vel[i] };
-  cq_neighbours<kCqRecord>(on, i, true, pos, pred, se, c.f.g, list, lds, b);
+  cq_neighbours<kCqRecord>(on, i, true, pos, pred, se, c.f.g, list, lds, b, !useList);
   if (lead)
     vort[i] = b.w;
   cld_flag(!lead | cld_safe(b.w), flags, kFlagVort);
@@ -1458,7 +1600,7 @@ struct rtp_clouds {
       }
       RTP_PROF(prof, "cld_gather", s,
                hipLaunchKernelGGL(k_cld_gather, dim3(blocks_for(G.sortedN, 256)), dim3(256), 0, s,
-                                  G.idx[G.idxCur], G.sortedN, gth));
+                                  G.idx[G.idxCur], G.sortedN, gth, flags));
     }
     cur = 1 - cur;
     pc = 1 - pc;
@@ -1477,7 +1619,7 @@ struct rtp_clouds {
       RTP_HIP_TRY(hipStreamWaitEvent(t, fork, 0));
       RTP_PROF(prof, "cld_temp_lambda", t,
                hipLaunchKernelGGL(qd ? k_cld_temp_lambda_q : k_cld_temp_lambda, dim3(bw), dim3(kCldLanes), 0, t, pos[cur], temp[cur],
-                                  G.startEnd, lap, lambdaT, n, c, listT, flags));
+                                  G.startEnd, lap, lambdaT, n, c, listT, flags, useList));
       RTP_PROF(prof, "cld_temp_correct", t,
                hipLaunchKernelGGL(qd ? k_cld_temp_correct_q : k_cld_temp_correct, dim3(bw), dim3(kCldLanes), 0, t, pos[cur], lambdaT,
                                   G.startEnd, temp[cur], n, c, listT, flags, useList));
@@ -1508,7 +1650,7 @@ struct rtp_clouds {
     if (c.f.p.isVorticityConfEnabled) {
       RTP_PROF(prof, "cld_vorticity", s,
                hipLaunchKernelGGL(qd ? k_cld_vorticity_q : k_cld_vorticity, dim3(bw), dim3(kCldLanes), 0, s, pred[pc], G.startEnd,
-                                  vel[cur], vort, n, c, list, flags));
+                                  vel[cur], vort, n, c, list, flags, useList));
       RTP_PROF(prof, "cld_confinement", s,
                hipLaunchKernelGGL(qd ? k_cld_confinement_q : k_cld_confinement, dim3(bw), dim3(kCldLanes), 0, s, pred[pc],
                                   G.startEnd, vort, vel[cur], velTmp, n, c, list, flags, useList));
@@ -1584,8 +1726,8 @@ int rtp_clouds_create(const rtp_model_desc* d, rtp_clouds** out)
   const uint32_t maxN = d->maxNbParticles;
   rc = h->grid.alloc(maxN);
   for (int k = 0; k < 2 && !rc; ++k) {
-    if ((rc = dev_alloc(&h->pos[k], maxN)) || (rc = dev_alloc(&h->vel[k], maxN)) ||
-        (rc = dev_alloc(&h->tot[k], maxN)) || (rc = dev_alloc(&h->pred[k], maxN)) ||
+    if ((rc = dev_alloc(&h->pos[k], maxN + kPosPad)) || (rc = dev_alloc(&h->vel[k], maxN)) ||
+        (rc = dev_alloc(&h->tot[k], maxN)) || (rc = dev_alloc(&h->pred[k], maxN + kPosPad)) ||
         (rc = dev_alloc(&h->temp[k], maxN)) || (rc = dev_alloc(&h->buoy[k], maxN)) ||
         (rc = dev_alloc(&h->vapor[k], maxN)) || (rc = dev_alloc(&h->cloud[k], maxN)) ||
         (rc = dev_alloc(&h->pid[k], maxN)))
@@ -1596,7 +1738,7 @@ int rtp_clouds_create(const rtp_model_desc* d, rtp_clouds** out)
            (rc = dev_alloc(&h->density, maxN)) || (rc = dev_alloc(&h->lambda, maxN)) ||
            (rc = dev_alloc(&h->lap, maxN)) || (rc = dev_alloc(&h->lambdaT, maxN)) ||
            (rc = dev_alloc(&h->list.entry, (size_t)kCldListCap * maxN)) ||
-           (rc = dev_alloc(&h->list.count, maxN)) || (rc = dev_alloc(&h->flags, 1)) ||
+           (rc = dev_alloc(&h->list.count, maxN)) || (rc = dev_alloc(&h->flags, kCldFlagWords)) ||
            (rc = dev_alloc(&h->listT.entry, (size_t)kCldListCap * maxN)) ||
            (rc = dev_alloc(&h->listT.count, maxN)));
   h->list.stride = maxN;
