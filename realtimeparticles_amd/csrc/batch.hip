@@ -595,8 +595,11 @@ int rtp_batch_restore_checkpoint(rtp_batch* h)
   if (!h->ckValid)
     return fail(RTP_ERR_STATE, "no checkpoint saved");
   RTP_HIP_TRY(hipSetDevice(h->device));
-  RTP_HIP_TRY(hipMemcpyAsync(h->pos[h->cur], h->ckPos, sizeof(float4) * h->total, hipMemcpyDeviceToDevice, h->stream));
-  RTP_HIP_TRY(hipMemcpyAsync(h->vel[h->cur], h->ckVel, sizeof(float4) * h->total, hipMemcpyDeviceToDevice, h->stream));
+  CopyList l;
+  l.add(h->pos[h->cur], h->ckPos, sizeof(float4) * h->total);
+  l.add(h->vel[h->cur], h->ckVel, sizeof(float4) * h->total);
+  launch_copy_buffers(l, h->stream);
+  RTP_HIP_TRY(hipGetLastError());
   return RTP_OK;
 }
 

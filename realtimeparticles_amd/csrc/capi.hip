@@ -1187,28 +1187,25 @@ int rtp_fluids_restore_checkpoint(rtp_fluids* h)
   // that range is unchanged since the save, the current buffers alone need the copy;
   // otherwise both partners get it.
   const bool same = h->grid.dirtyEnd == h->ckDirty && h->grid.sortedN == h->ckSorted && h->n == h->ckN;
-  for (int k = 0; k < 2; ++k) {
+  CopyList l;
+  for (int k = 0; k < (same ? 1 : 2); ++k) {
     const bool current = k == 0;
-    if (!current && same)
-      break;
-    float4* pos = current ? h->pos[h->cur] : h->pos[1 - h->cur];
-    float4* vel = current ? h->vel[h->cur] : h->vel[1 - h->cur];
-    float4* pred = current ? h->pred[h->predFinal] : h->pred[1 - h->predFinal];
-    uint32_t* key = current ? h->grid.key[h->grid.keyCur] : h->grid.key[1 - h->grid.keyCur];
-    RTP_HIP_TRY(hipMemcpyAsync(pos, h->ckPos, sizeof(float4) * maxN, hipMemcpyDeviceToDevice, h->stream));
-    RTP_HIP_TRY(hipMemcpyAsync(vel, h->ckVel, sizeof(float4) * maxN, hipMemcpyDeviceToDevice, h->stream));
-    RTP_HIP_TRY(hipMemcpyAsync(pred, h->ckPred, sizeof(float4) * maxN, hipMemcpyDeviceToDevice, h->stream));
-    RTP_HIP_TRY(hipMemcpyAsync(key, h->ckKey, sizeof(uint32_t) * maxN, hipMemcpyDeviceToDevice, h->stream));
+    l.add(h->pos[current ? h->cur : 1 - h->cur], h->ckPos, sizeof(float4) * maxN);
+    l.add(h->vel[current ? h->cur : 1 - h->cur], h->ckVel, sizeof(float4) * maxN);
+    l.add(h->pred[current ? h->predFinal : 1 - h->predFinal], h->ckPred, sizeof(float4) * maxN);
+    l.add(h->grid.key[current ? h->grid.keyCur : 1 - h->grid.keyCur], h->ckKey, sizeof(uint32_t) * maxN);
   }
   // p_col and p_cameraDist into both partners: their gather and sort ranges need not be
   // those of the save
   if (h->ckRender && h->render.on) {
     for (int k = 0; k < 2; ++k) {
-      RTP_HIP_TRY(hipMemcpyAsync(h->render.col[k], h->ckCol, sizeof(float4) * maxN, hipMemcpyDeviceToDevice, h->stream));
-      RTP_HIP_TRY(hipMemcpyAsync(h->render.key[k], h->ckCam, sizeof(uint32_t) * maxN, hipMemcpyDeviceToDevice, h->stream));
+      l.add(h->render.col[k], h->ckCol, sizeof(float4) * maxN);
+      l.add(h->render.key[k], h->ckCam, sizeof(uint32_t) * maxN);
     }
     h->render.high = h->ckHigh;
   }
+  launch_copy_buffers(l, h->stream);
+  RTP_HIP_TRY(hipGetLastError());
   h->n = h->ckN;
   h->grid.dirtyEnd = h->ckDirty;
   h->grid.sortedN = h->ckSorted;

@@ -203,6 +203,21 @@ struct ReorderArgs {
   GridConsts g;
 };
 void launch_reorder(const ReorderArgs& a, hipStream_t s);
+// Whole-buffer device copies of one launch (hipMalloc'd buffers: 16-byte aligned).
+struct CopyList {
+  static constexpr int kMax = 12;
+  void* dst[kMax];
+  const void* src[kMax];
+  size_t words[kMax];
+  int n = 0;
+  void add(void* to, const void* from, size_t bytes)
+  {
+    dst[n] = to;
+    src[n] = from;
+    words[n++] = bytes / 4u;
+  }
+};
+void launch_copy_buffers(const CopyList& l, hipStream_t s);
 void launch_copy_f4(float4* dst, const float4* src, uint32_t begin, uint32_t end, hipStream_t s);
 
 // ------------------------------------------------------------------ rendering side of a frame
