@@ -598,7 +598,9 @@ int rtp_batch_restore_checkpoint(rtp_batch* h)
   CopyList l;
   l.add(h->pos[h->cur], h->ckPos, sizeof(float4) * h->total);
   l.add(h->vel[h->cur], h->ckVel, sizeof(float4) * h->total);
-  launch_copy_buffers(l, h->stream);
+  const int rc = launch_copy_buffers(l, h->stream);
+  if (rc)
+    return rc;
   RTP_HIP_TRY(hipGetLastError());
   return RTP_OK;
 }

@@ -688,7 +688,7 @@ __global__ __launch_bounds__(512) void k_boids_persistent(BoidsPersistentArgs a,
   for (uint32_t step = 0; step < a.steps; ++step) {
     for (uint32_t t = t0; t < nc; t += stride)  // resetStartEndCell (k_boids_hash)
       a.startEnd[t] = make_uint2(1u, 0u);
-    if (blockIdx.x == 0)  // k_sort_small: the sorted keys land in key[kc ^ res]
+    if (blockIdx.x == 0)  // the sorted keys land in key[kc ^ res]
       small_sort_block<16>(a.key[kc], a.key[1 - kc], a.idx[0], a.idx[1], sn, a.passes, lds);
     kc = res ? 1 - kc : kc;
     grid_barrier(a.bar, gen);

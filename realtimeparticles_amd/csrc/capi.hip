@@ -122,7 +122,8 @@ struct RenderState {
 // (its name on the host is a stand-in, not a device address); it passes the address
 // hipGetSymbolAddress returns on each device.
 constexpr uint32_t kNoAllocMax = RTP_NOALLOC_MAX_PARTICLES;
-// (the sort here keeps subtiles of kSortItems keys per lane at every size)
+// (the sort here keeps subtiles of kSortItems keys per lane from 2^18 keys on; below, the count
+// table of sort_items' four keys per lane is no larger than theirs at kNoAllocMax)
 constexpr size_t kNoAllocWords = 2 * (size_t)kNoAllocMax + count_words(kNoAllocMax, kSortItems);
 static __device__ __align__(256) uint32_t scratch[kNoAllocWords];
 
@@ -1204,7 +1205,9 @@ int rtp_fluids_restore_checkpoint(rtp_fluids* h)
     }
     h->render.high = h->ckHigh;
   }
-  launch_copy_buffers(l, h->stream);
+  const int rc = launch_copy_buffers(l, h->stream);
+  if (rc)
+    return rc;
   RTP_HIP_TRY(hipGetLastError());
   h->n = h->ckN;
   h->grid.dirtyEnd = h->ckDirty;
@@ -2127,7 +2130,8 @@ int rtp_grid_build_noalloc(const rtp_model_desc* d, const float* pos4, uint32_t*
   // the caller's keys and idx.  No scratch word needs to start at zero: every count a sort
   // pass reads is written earlier in that pass, and the partners are read only where a pass
   // has written them.
-  const SortPlan plan = make_sort_plan(n, max_active_key(g), 0, kSortItems);
+  static_assert(count_words((1u << 18) - 1u, 4) <= count_words(kNoAllocMax, kSortItems), "scratch");
+  const SortPlan plan = make_sort_plan(n, max_active_key(g), 0, n < (1u << 18) ? 0 : kSortItems);
   const bool inB = sort_result_in_b(plan);
   uint32_t* const keyA = inB ? keyScratch : keys;
   uint32_t* const keyB = inB ? keys : keyScratch;

@@ -190,6 +190,57 @@ __global__ __launch_bounds__(256) void k_scan_apply(uint32_t* __restrict__ data,
   }
 }
 
+// A wave's ITEMS x 64 keys and indices (the identity without idxIn) from `base` on.
+template <int ITEMS>
+__device__ __forceinline__ void sort_load(const uint32_t* __restrict__ keysIn,
+                                          const uint32_t* __restrict__ idxIn, uint32_t n,
+                                          uint32_t base, uint32_t kr[ITEMS], uint32_t vr[ITEMS])
+{
+  const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const uint32_t i = base + (uint32_t)(k * 64) + lane;
+    const bool valid = i < n;
+    kr[k] = valid ? keysIn[i] : 0u;
+    vr[k] = valid ? (idxIn ? idxIn[i] : i) : 0u;
+  }
+}
+
+// Ranks them with ballot-based match and scatters; run: the wave's next place per digit (LDS).
+template <int BITS, int ITEMS>
+__device__ __forceinline__ void sort_scatter(const uint32_t kr[ITEMS], const uint32_t vr[ITEMS],
+                                             uint32_t n, uint32_t base, int shift, uint32_t* run,
+                                             uint32_t* __restrict__ keysOut,
+                                             uint32_t* __restrict__ idxOut)
+{
+  constexpr uint32_t RADIX = 1u << BITS;
+  const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const bool valid = base + (uint32_t)(k * 64) + lane < n;
+    const uint32_t d = (kr[k] >> shift) & (RADIX - 1u);
+    uint64_t peers = __ballot(valid);
+#pragma unroll
+    for (int bit = 0; bit < BITS; ++bit) {
+      const bool set = (d >> bit) & 1u;
+      const uint64_t m = __ballot(set);
+      peers &= set ? m : ~m;
+    }
+    const uint32_t rank = mbcnt64(peers);
+    const uint32_t start = run[d];
+    if (valid && rank == 0)
+      run[d] = start + (uint32_t)__popcll(peers);
+    if (valid) {
+      keysOut[start + rank] = kr[k];
+      idxOut[start + rank] = vr[k];
+    }
+  }
+}
+
+// Small sorts: keys per lane and per workgroup.
+constexpr int kRowItems = 4;
+constexpr uint32_t kRowKeys = 4u * kRowItems * 64u;
+
 template <int BITS, int ITEMS>
 __global__ __launch_bounds__(256) void k_sort_downsweep(
   const uint32_t* __restrict__ keysIn, const uint32_t* __restrict__ idxIn, uint32_t n, int shift,
@@ -208,34 +259,100 @@ __global__ __launch_bounds__(256) void k_sort_downsweep(
     return;
   const uint32_t base = s * (uint32_t)(ITEMS * 64);
   uint32_t kr[ITEMS], vr[ITEMS];
+  sort_load<ITEMS>(keysIn, idxIn, n, base, kr, vr);
+  sort_scatter<BITS, ITEMS>(kr, vr, n, base, shift, run[w], keysOut, idxOut);
+}
+
+// A pass of a small sort in two launches (run_pass_rows).  The first leaves every workgroup's
+// digit counts as a row of RADIX words.
+template <int BITS>
+__global__ __launch_bounds__(256) void k_sort_rows(const uint32_t* __restrict__ keys, uint32_t n,
+                                                   int shift, uint32_t* __restrict__ rows)
+{
+  constexpr int RADIX = 1 << BITS;
+  __shared__ uint32_t hist[RADIX];
+  for (int d = threadIdx.x; d < RADIX; d += 256)
+    hist[d] = 0;
+  __syncthreads();
+  const uint32_t base = blockIdx.x * kRowKeys + threadIdx.x;
 #pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    const uint32_t i = base + (uint32_t)(k * 64 + lane);
-    const bool valid = i < n;
-    kr[k] = valid ? keysIn[i] : 0u;
-    vr[k] = valid ? (idxIn ? idxIn[i] : i) : 0u;
+  for (int k = 0; k < kRowItems; ++k) {
+    const uint32_t i = base + (uint32_t)k * 256u;
+    if (i < n)
+      atomicAdd(&hist[(keys[i] >> shift) & (RADIX - 1)], 1u);
   }
+  __syncthreads();
+  for (int d = threadIdx.x; d < RADIX; d += 256)
+    rows[(size_t)blockIdx.x * RADIX + d] = hist[d];
+}
+
+// The second: every workgroup adds up the columns of the rows (the whole column and the rows
+// before its own), scans the digits' totals, and ranks and scatters its keys as
+// k_sort_downsweep does.
+template <int BITS>
+__global__ __launch_bounds__(256) void k_sort_scatter_rows(
+  const uint32_t* __restrict__ keysIn, const uint32_t* __restrict__ idxIn, uint32_t n, int shift,
+  const uint32_t* __restrict__ rows, uint32_t* __restrict__ keysOut, uint32_t* __restrict__ idxOut)
+{
+  constexpr int RADIX = 1 << BITS;
+  __shared__ uint32_t run[4][RADIX];
+  __shared__ uint32_t tot[RADIX], before[RADIX];
+  const uint32_t t = threadIdx.x;
+  const int lane = t & 63, w = t >> 6;
+  const uint32_t base = blockIdx.x * kRowKeys + (uint32_t)w * (kRowItems * 64u);
+  uint32_t kr[kRowItems], vr[kRowItems];
+  sort_load<kRowItems>(keysIn, idxIn, n, base, kr, vr);
+  for (uint32_t d = t; d < RADIX; d += 256u) {
+    run[0][d] = run[1][d] = run[2][d] = run[3][d] = 0u;
+    tot[d] = before[d] = 0u;
+  }
+  __syncthreads();
 #pragma unroll
-  for (int k = 0; k < ITEMS; ++k) {
-    const uint32_t i = base + (uint32_t)(k * 64 + lane);
-    const bool valid = i < n;
-    const uint32_t d = (kr[k] >> shift) & (uint32_t)(RADIX - 1);
-    uint64_t peers = __ballot(valid);
-#pragma unroll
-    for (int bit = 0; bit < BITS; ++bit) {
-      const bool set = (d >> bit) & 1u;
-      const uint64_t m = __ballot(set);
-      peers &= set ? m : ~m;
+  for (int k = 0; k < kRowItems; ++k)
+    if (base + (uint32_t)(k * 64 + lane) < n)
+      atomicAdd(&run[w][(kr[k] >> shift) & (RADIX - 1)], 1u);
+  // 256 / RADIX threads a column, or RADIX / 256 columns a thread
+  constexpr uint32_t kParts = RADIX < 256 ? 256u / RADIX : 1u;
+  for (uint32_t d = t & (RADIX - 1); d < RADIX; d += 256u) {
+    uint32_t all = 0, pre = 0;
+    const uint32_t* col = rows + d;
+#pragma unroll 32
+    for (uint32_t r = RADIX < 256 ? t / RADIX : 0u; r < gridDim.x; r += kParts) {
+      const uint32_t v = col[(size_t)r * RADIX];
+      all += v;
+      pre += r < blockIdx.x ? v : 0u;
     }
-    const uint32_t rank = mbcnt64(peers);
-    const uint32_t start = run[w][d];
-    if (valid && rank == 0)
-      run[w][d] = start + (uint32_t)__popcll(peers);
-    if (valid) {
-      keysOut[start + rank] = kr[k];
-      idxOut[start + rank] = vr[k];
+    if (kParts > 1u) {
+      atomicAdd(&tot[d], all);
+      atomicAdd(&before[d], pre);
+    } else {
+      tot[d] = all;
+      before[d] = pre;
     }
   }
+  __syncthreads();
+  constexpr uint32_t kPer = RADIX < 256 ? 1u : RADIX / 256u;  // consecutive digits of a thread
+  uint32_t sum = 0, total = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; ++k)
+    sum += t * kPer + k < RADIX ? tot[t * kPer + k] : 0u;
+  uint32_t start = block_exclusive_256(sum, &total);
+#pragma unroll
+  for (uint32_t k = 0; k < kPer; ++k) {
+    const uint32_t d = t * kPer + k;
+    if (d < RADIX) {
+      uint32_t at = start + before[d];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const uint32_t mine = run[v][d];
+        run[v][d] = at;
+        at += mine;
+      }
+      start += tot[d];
+    }
+  }
+  __syncthreads();
+  sort_scatter<BITS, kRowItems>(kr, vr, n, base, shift, run[w], keysOut, idxOut);
 }
 
 __global__ __launch_bounds__(256) void k_reorder(ReorderArgs a)
@@ -275,21 +392,32 @@ __global__ __launch_bounds__(256) void k_reorder_batch(ReorderArgs a, BatchView 
   reorder_body(i, l, sc.kbase, o);
 }
 
-template <int CH>
-__global__ __launch_bounds__(512) void k_sort_small(uint32_t* __restrict__ keyA,
-                                                    uint32_t* __restrict__ keyB,
-                                                    uint32_t* __restrict__ idxA,
-                                                    uint32_t* __restrict__ idxB, uint32_t n,
-                                                    int passes)
+// A sort whose column sums are short -- kRowLoads row words a thread or fewer, with four keys a
+// lane -- takes two launches a pass: the scan's launches cost more than every workgroup's
+// own sums.  A pass took (upsweep, scan launches, downsweep; now) 10.2 (8.3) us at 8,192 keys of
+// 7 bits, 18.4 (10.0) at 65,536 of 8 and 27.6 (22.1) at 131,072 of 10, the longest sums; 4,000
+// keys 13.4 us for both passes against 18.1 in one workgroup's LDS, 500 keys 9.4 against 12.1.
+// Bound by latency: the sums' loads go 32 at a time (8 at a time took 56 us for the longest).
+constexpr uint32_t kRowLoads = 512;
+template <int BITS>
+bool run_pass_rows(const SortPlan& p, int shift, const uint32_t* kin, const uint32_t* iin,
+                   uint32_t* kout, uint32_t* iout, uint32_t* counts, hipStream_t s)
 {
-  __shared__ SmallSortLds lds;
-  small_sort_block<CH>(keyA, keyB, idxA, idxB, n, passes, lds);
+  const uint32_t blocks = (p.n + kRowKeys - 1u) / kRowKeys;
+  if (p.items != kRowItems || blocks * (BITS > 8 ? 1u << (BITS - 8) : 1u) > kRowLoads)
+    return false;
+  hipLaunchKernelGGL((k_sort_rows<BITS>), dim3(blocks), dim3(256), 0, s, kin, p.n, shift, counts);
+  hipLaunchKernelGGL((k_sort_scatter_rows<BITS>), dim3(blocks), dim3(256), 0, s, kin, iin, p.n,
+                     shift, counts, kout, iout);
+  return true;
 }
 
 template <int BITS, int ITEMS>
 int run_pass(const SortPlan& p, int shift, const uint32_t* kin, const uint32_t* iin,
              uint32_t* kout, uint32_t* iout, uint32_t* counts, hipStream_t s)
 {
+  if (ITEMS == kRowItems && run_pass_rows<BITS>(p, shift, kin, iin, kout, iout, counts, s))
+    return RTP_OK;
   const uint32_t blocks = (p.subtiles + 3u) / 4u;
   hipLaunchKernelGGL((k_sort_upsweep<BITS, ITEMS>), dim3(blocks), dim3(256), 0, s, kin, p.n,
                      shift, p.subtiles, counts);
@@ -405,27 +533,30 @@ __global__ __launch_bounds__(256) void k_order_scatter(const uint32_t* __restric
 
 inline uint32_t blocks_for(uint32_t n, uint32_t b) { return (n + b - 1u) / b; }
 
-// Several buffers in one launch: buffer blockIdx.y, a 16-byte granule a thread and round (the
-// last, partial granule word by word).  A checkpoint's runtime copies kept the host busy: with one
-// launch instead of four copies a restored substep of 8,192 particles takes 55 us among others,
-// with 23 enqueues 86.  Bound by HBM for large models: 4.9 TB/s read and written together at
-// 4,194,304 particles.
+// Several buffers in one launch: buffer blockIdx.y, 16 KiB a workgroup (the last, partial granule
+// word by word).  A checkpoint's runtime copies keep the host for 8 us each: with one launch for
+// all a restored substep of 8,192 particles takes 55 us among others, 86 before.  From
+// kCopyRuntimeWords words (1,048,576 positions) on the runtime's copies are faster: 27 us
+// against 29 there, 86 against 135 at 4,194,304 particles.
+constexpr uint32_t kCopyGranules = 1024;
+constexpr size_t kCopyRuntimeWords = (size_t)1 << 22;
 __global__ __launch_bounds__(256) void k_copy_buffers(CopyList l)
 {
   const int b = blockIdx.y;
-  const size_t words = l.words[b], granules = words >> 2, step = (size_t)gridDim.x * 256u;
+  const size_t words = l.words[b], granules = words >> 2;
   const uint4* __restrict__ src = reinterpret_cast<const uint4*>(l.src[b]);
   uint4* __restrict__ dst = reinterpret_cast<uint4*>(l.dst[b]);
-  size_t g = (size_t)blockIdx.x * 256u + threadIdx.x;
-  for (; g + 3u * step < granules; g += 4u * step) {
-    const uint4 v0 = src[g], v1 = src[g + step], v2 = src[g + 2u * step], v3 = src[g + 3u * step];
+  const size_t g = (size_t)blockIdx.x * kCopyGranules + threadIdx.x;
+  if (g + 768u < granules) {
+    const uint4 v0 = src[g], v1 = src[g + 256u], v2 = src[g + 512u], v3 = src[g + 768u];
     dst[g] = v0;
-    dst[g + step] = v1;
-    dst[g + 2u * step] = v2;
-    dst[g + 3u * step] = v3;
+    dst[g + 256u] = v1;
+    dst[g + 512u] = v2;
+    dst[g + 768u] = v3;
+  } else {
+    for (size_t k = g; k < granules; k += 256u)
+      dst[k] = src[k];
   }
-  for (; g < granules; g += step)
-    dst[g] = src[g];
   if (blockIdx.x == 0 && threadIdx.x < (words & 3u)) {
     const size_t w = granules * 4u + threadIdx.x;
     reinterpret_cast<uint32_t*>(l.dst[b])[w] = reinterpret_cast<const uint32_t*>(l.src[b])[w];
@@ -481,8 +612,8 @@ SortPlan make_sort_plan(uint32_t n, uint32_t maxKey, int bitsOverride, int fixed
   return p;
 }
 
-// Whether the current device gives one workgroup the LDS k_sort_small declares (checked
-// once per device; otherwise small sorts take the multi-launch path).
+// Whether the current device gives one workgroup the LDS of the one-workgroup sort (checked
+// once per device).
 bool small_sort_fits()
 {
   static int ok[64] = {};  // 0 unknown, 1 yes, 2 no
@@ -490,25 +621,15 @@ bool small_sort_fits()
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64)
     return false;
   if (ok[dev] == 0) {
-    hipFuncAttributes a{};
     int limit = 0;
-    const bool q = hipFuncGetAttributes(&a, reinterpret_cast<const void*>(&k_sort_small<16>)) == hipSuccess &&
-                   hipDeviceGetAttribute(&limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess;
-    ok[dev] = (q && a.sharedSizeBytes <= (size_t)limit) ? 1 : 2;
+    const bool q = hipDeviceGetAttribute(&limit, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess;
+    ok[dev] = (q && sizeof(SmallSortLds) <= (size_t)limit) ? 1 : 2;
   }
   return ok[dev] == 1;
 }
 
 // Passes of the one-workgroup sort: 4-bit digits over the significant bits.
 static int small_sort_passes(const SortPlan& p) { return (p.keyBits + 3) / 4; }
-
-// sort_pairs takes the one-workgroup sort up to kSmallSortFaster keys, where it beats the
-// multi-launch sort (21.0 against 23.8 us at 4,096 keys, 32.5 against 25.1 at 6,144, on the
-// boids flock); the persistent boids update, whose step runs in one launch, takes it up to
-// kSmallSortMax.
-constexpr uint32_t kSmallSortFaster = 4096;
-
-static bool use_small_sort(const SortPlan& p) { return p.n <= kSmallSortFaster && small_sort_fits(); }
 
 int small_sort_pass_count(const SortPlan& p)
 {
@@ -519,7 +640,7 @@ bool sort_result_in_b(const SortPlan& p)
 {
   if (p.n == 0)
     return false;
-  return ((use_small_sort(p) ? small_sort_passes(p) : p.passes) & 1) != 0;
+  return (p.passes & 1) != 0;
 }
 
 int sort_pairs(const SortPlan& p, uint32_t* keyA, uint32_t* keyB, uint32_t* idxA, uint32_t* idxB,
@@ -528,17 +649,6 @@ int sort_pairs(const SortPlan& p, uint32_t* keyA, uint32_t* keyB, uint32_t* idxA
   *resultInB = false;
   if (p.n == 0)
     return RTP_OK;
-  if (use_small_sort(p)) {  // one workgroup, all passes in LDS
-    const int passes = small_sort_passes(p);
-    if (p.n <= 4096u)
-      hipLaunchKernelGGL(k_sort_small<8>, dim3(1), dim3(kSmallThreads), 0, s, keyA, keyB, idxA, idxB,
-                         p.n, passes);
-    else
-      hipLaunchKernelGGL(k_sort_small<16>, dim3(1), dim3(kSmallThreads), 0, s, keyA, keyB, idxA,
-                         idxB, p.n, passes);
-    *resultInB = (passes & 1) != 0;
-    return RTP_OK;
-  }
   uint32_t *kin = keyA, *kout = keyB, *iin = idxA, *iout = idxB;
   bool inB = false;
   for (int pass = 0; pass < p.passes; ++pass) {
@@ -588,16 +698,21 @@ void launch_copy_f4(float4* dst, const float4* src, uint32_t begin, uint32_t end
                      begin, end);
 }
 
-void launch_copy_buffers(const CopyList& l, hipStream_t s)
+int launch_copy_buffers(const CopyList& l, hipStream_t s)
 {
   size_t words = 0;
   for (int b = 0; b < l.n; ++b)
     words = l.words[b] > words ? l.words[b] : words;
   if (words == 0)
-    return;
-  const size_t blocks = (words + 4u * 4u * 256u - 1u) / (4u * 4u * 256u);
-  hipLaunchKernelGGL(k_copy_buffers, dim3((uint32_t)(blocks < 4096u ? blocks : 4096u), l.n),
-                     dim3(256), 0, s, l);
+    return RTP_OK;
+  if (words >= kCopyRuntimeWords) {
+    for (int b = 0; b < l.n; ++b)
+      RTP_HIP_TRY(hipMemcpyAsync(l.dst[b], l.src[b], 4u * l.words[b], hipMemcpyDeviceToDevice, s));
+    return RTP_OK;
+  }
+  const size_t blocks = (words + 4u * kCopyGranules - 1u) / (4u * kCopyGranules);
+  hipLaunchKernelGGL(k_copy_buffers, dim3((uint32_t)blocks, l.n), dim3(256), 0, s, l);
+  return RTP_OK;
 }
 
 void launch_reorder_batch(const BatchView& bv, const ReorderArgs& a, hipStream_t s)

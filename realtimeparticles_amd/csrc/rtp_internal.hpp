@@ -138,7 +138,7 @@ struct SortPlan {
   size_t countWords = 0;   // radix * subtiles
   int keyBits = 0;         // significant bits of the largest key
 };
-// The one-workgroup LDS sort (all passes in one launch) takes at most this many keys.
+// The one-workgroup LDS sort of the persistent boids update takes at most this many keys.
 constexpr uint32_t kSmallSortMax = 8192;
 constexpr int kSortItems = 32;  // keys per lane of a subtile, for 2^22 keys and more
 // Keys per lane of a subtile for a sort of n keys: smaller subtiles below 2^22 keys, so a
@@ -217,7 +217,7 @@ struct CopyList {
     words[n++] = bytes / 4u;
   }
 };
-void launch_copy_buffers(const CopyList& l, hipStream_t s);
+int launch_copy_buffers(const CopyList& l, hipStream_t s);
 void launch_copy_f4(float4* dst, const float4* src, uint32_t begin, uint32_t end, hipStream_t s);
 
 // ------------------------------------------------------------------ rendering side of a frame
