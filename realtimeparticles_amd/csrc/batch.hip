@@ -62,6 +62,8 @@ struct rtp_batch {
   uint32_t nbThreads = 0;
   uint4* nbList = nullptr;
   uint32_t* nbCount = nullptr;
+  uint2* cols = nullptr;  // the walks' column ranges, laid out like startEnd
+  uint32_t maxCells = 0;  // of a scene
   bool constsDirty = true;
   int cur = 0;
   int predFinal = 1;
@@ -120,6 +122,7 @@ struct rtp_batch {
     dev_free(opart);
     dev_free(nbList);
     dev_free(nbCount);
+    dev_free(cols);
     if (stream)
       (void)hipStreamDestroy(stream);
     stream = nullptr;
@@ -202,7 +205,10 @@ struct rtp_batch {
     // neighbour passes: threads in the grid's order first, then (resort) by current cell;
     // with lists the density / vorticity passes record survivors and the correction,
     // confinement and XSPH passes replay them
+    RTP_PROF(prof, "pbf_columns", s,
+             launch_pbf_columns_batch(bv, startEnd, cols, (uint32_t)scenes.size(), maxCells, s));
     BatchView nb = bv;
+    nb.cols = cols;
     if (lists)
       nb.nb = NbList{ nbList, nbCount, bv.numBlocks * bv.block };
     BatchView cb = nb;
@@ -361,6 +367,7 @@ int rtp_batch_create(int device, const rtp_batch_scene* sc, uint32_t count, rtp_
     S.slot.n = sc[s].nbParticles;
     S.slot.kbase = (uint32_t)keys;
     S.slot.keySpan = max_active_key(g) + 1u;
+    h->maxCells = std::max(h->maxCells, g.numCells);
     total += S.slot.n;
     keys += S.slot.keySpan;
     if (total > 0x7fffffffu || keys > 0xffffffffu) {
@@ -388,7 +395,7 @@ int rtp_batch_create(int device, const rtp_batch_scene* sc, uint32_t count, rtp_
       (rc = dev_alloc(&h->key[0], N)) || (rc = dev_alloc(&h->key[1], N)) ||
       (rc = dev_alloc(&h->idx[0], N)) || (rc = dev_alloc(&h->idx[1], N)) ||
       (rc = dev_alloc(&h->counts, count_capacity(N))) ||
-      (rc = dev_alloc(&h->startEnd, h->keySpace)) ||
+      (rc = dev_alloc(&h->startEnd, h->keySpace)) || (rc = dev_alloc(&h->cols, h->keySpace)) ||
       (rc = dev_alloc(&h->dSlots, count)) || (rc = dev_alloc(&h->dConsts, count)) ||
       (rc = dev_alloc(&h->dBlocks, maxBlocks)) || (rc = dev_alloc(&h->okey, N)) ||
       (rc = dev_alloc(&h->orank, N)) || (rc = dev_alloc(&h->oorder[0], N)) ||

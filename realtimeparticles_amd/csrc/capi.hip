@@ -252,6 +252,7 @@ struct rtp_fluids {
   // survivor lists (RTP_LAUNCH_NB_LIST), allocated when first enabled
   uint4* nbList = nullptr;      // kNbCap / 4 x maxN granules
   uint32_t* nbCount = nullptr;  // maxN
+  uint2* cols = nullptr;        // the one-lane walks' column ranges, one per cell
   float* resDensity = nullptr;
   float* resMetric = nullptr; // max, sum, max compression of the residual pass + partials
   rtp_mlp* mlp = nullptr;
@@ -354,6 +355,12 @@ struct rtp_fluids {
     if (lists) {
       po.nb = NbList{ nbList, nbCount, n };
       pc.nb = po.nb;
+    }
+    // every pass but the plain solver's quad passes walks with one lane
+    if (n > 0 && (L.quad == 0 || L.tile != 0 || wantFeatures || residualPass)) {
+      RTP_PROF(prof, "pbf_columns", s, launch_pbf_columns(G.startEnd, cols, c.g, s));
+      po.cols = cols;
+      pc.cols = cols;
     }
     const uint32_t m16 = L.bricks ? brick_order_cells(c.g) : order_cells(c.g);
     pc.keyOut = resort ? okey : nullptr;
@@ -598,6 +605,7 @@ struct rtp_fluids {
     dev_free(opart);
     dev_free(nbList);
     dev_free(nbCount);
+    dev_free(cols);
     if (stream)
       (void)hipStreamDestroy(stream);
     stream = nullptr;
@@ -897,7 +905,7 @@ int rtp_fluids_create(const rtp_model_desc* d, rtp_fluids** out)
       (rc = dev_alloc(&h->lamAcc, maxN)) || (rc = dev_alloc(&h->resDensity, maxN)) ||
       (rc = dev_alloc(&h->resMetric, kMetricFloats)) || (rc = dev_alloc(&h->okey, maxN)) ||
       (rc = dev_alloc(&h->orank, maxN)) || (rc = dev_alloc(&h->oorder[0], maxN)) ||
-      (rc = dev_alloc(&h->oorder[1], maxN)) ||
+      (rc = dev_alloc(&h->oorder[1], maxN)) || (rc = dev_alloc(&h->cols, h->grid.g.numCells)) ||
       (rc = dev_alloc(&h->ocount.table[0], order_count_words(h->grid.g))) ||
       (rc = dev_alloc(&h->ocount.table[1], order_count_words(h->grid.g))) ||
       (rc = dev_alloc(&h->opart, scan_partials_needed(order_count_words(h->grid.g))))) {

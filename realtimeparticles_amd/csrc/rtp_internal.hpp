@@ -281,6 +281,7 @@ struct PassOrder {
   uint32_t keyBase = 0;             //   plus this (a batched scene's key base)
   int bricks = 0;                   //   1: brick_key of the cell instead of its index
   NbList nb;
+  const uint2* cols = nullptr;      // the walks' column ranges (launch_pbf_columns)
   __device__ uint32_t particle(uint32_t t) const { return order ? order[t] : t; }
 };
 // The thread order's two count tables of `words` words each, both all zero when allocated.
@@ -325,7 +326,12 @@ struct BatchView {
   const uint32_t* order = nullptr;  // batch-wide thread order (scene slices stay in place)
   uint32_t* keyOut = nullptr;       // correction passes: batch-wide key of each output
   NbList nb;                        // survivor lists; a thread's slot is its launch-wide id
+  const uint2* cols = nullptr;      // the walks' column ranges, scene by scene like the cell table
 };
+// The column ranges of the cell table (one per cell) that the one-lane walks read.
+void launch_pbf_columns(const uint2* startEnd, uint2* cols, const GridConsts& g, hipStream_t s);
+void launch_pbf_columns_batch(const BatchView& bv, const uint2* startEnd, uint2* cols,
+                              uint32_t numScenes, uint32_t maxCells, hipStream_t s);
 void launch_fill_start_end(uint2* startEnd, uint32_t count, hipStream_t s);
 void launch_pbf_predict_batch(const BatchView& bv, const float4* pos, const float4* vel,
                               float4* pred, uint32_t* key, hipStream_t s);
