@@ -64,6 +64,7 @@ struct rtp_batch {
   uint32_t* nbCount = nullptr;
   uint2* cols = nullptr;  // the walks' column ranges, laid out like startEnd
   uint32_t maxCells = 0;  // of a scene
+  float4* packed = nullptr;  // PassOrder::packed
   bool constsDirty = true;
   int cur = 0;
   int predFinal = 1;
@@ -123,6 +124,7 @@ struct rtp_batch {
     dev_free(nbList);
     dev_free(nbCount);
     dev_free(cols);
+    dev_free(packed);
     if (stream)
       (void)hipStreamDestroy(stream);
     stream = nullptr;
@@ -209,6 +211,7 @@ struct rtp_batch {
              launch_pbf_columns_batch(bv, startEnd, cols, (uint32_t)scenes.size(), maxCells, s));
     BatchView nb = bv;
     nb.cols = cols;
+    nb.packed = packed;
     if (lists)
       nb.nb = NbList{ nbList, nbCount, bv.numBlocks * bv.block };
     BatchView cb = nb;
@@ -239,6 +242,8 @@ struct rtp_batch {
       RTP_PROF(prof, "pbf_update_vel", s,
                launch_pbf_update_vel_batch(bv, pred[in], pos[cur], vel[cur], vortOn ? nullptr : pos[cur], s));
     predFinal = in;
+    if (nb.order)  // PassOrder::packed
+      nb.packed = nullptr;
     if (vortOn) {
       RTP_PROF(prof, "pbf_vorticity", s,
                launch_pbf_vorticity_batch(nb, pred[in], startEnd, vel[cur], vort, s, rec));
@@ -396,6 +401,7 @@ int rtp_batch_create(int device, const rtp_batch_scene* sc, uint32_t count, rtp_
       (rc = dev_alloc(&h->idx[0], N)) || (rc = dev_alloc(&h->idx[1], N)) ||
       (rc = dev_alloc(&h->counts, count_capacity(N))) ||
       (rc = dev_alloc(&h->startEnd, h->keySpace)) || (rc = dev_alloc(&h->cols, h->keySpace)) ||
+      (rc = dev_alloc(&h->packed, N)) ||
       (rc = dev_alloc(&h->dSlots, count)) || (rc = dev_alloc(&h->dConsts, count)) ||
       (rc = dev_alloc(&h->dBlocks, maxBlocks)) || (rc = dev_alloc(&h->okey, N)) ||
       (rc = dev_alloc(&h->orank, N)) || (rc = dev_alloc(&h->oorder[0], N)) ||

@@ -253,6 +253,7 @@ struct rtp_fluids {
   uint4* nbList = nullptr;      // kNbCap / 4 x maxN granules
   uint32_t* nbCount = nullptr;  // maxN
   uint2* cols = nullptr;        // the one-lane walks' column ranges, one per cell
+  float4* packed = nullptr;     // PassOrder::packed, maxN
   float* resDensity = nullptr;
   float* resMetric = nullptr; // max, sum, max compression of the residual pass + partials
   rtp_mlp* mlp = nullptr;
@@ -356,6 +357,8 @@ struct rtp_fluids {
       po.nb = NbList{ nbList, nbCount, n };
       pc.nb = po.nb;
     }
+    po.packed = packed;
+    pc.packed = packed;
     // every pass but the plain solver's quad passes walks with one lane
     if (n > 0 && (L.quad == 0 || L.tile != 0 || wantFeatures || residualPass)) {
       RTP_PROF(prof, "pbf_columns", s, launch_pbf_columns(G.startEnd, cols, c.g, s));
@@ -394,7 +397,7 @@ struct rtp_fluids {
                launch_pbf_density_lambda(pred[in], G.startEnd, density, lambda, n, c, L, s,
                                          replay ? (mode | kNbRecord) : mode, la, po));
       if (learned && k == 0)
-        RTP_PROF(prof, "mlp_warm_start", s, launch_mlp_forward(feat, n, mlp->dev, lambda, s));
+        RTP_PROF(prof, "mlp_warm_start", s, launch_mlp_forward(feat, n, mlp->dev, lambda, s, packed));
       const int last = !lastIt ? kNextIter : (learned ? kLastOnly : kLastVel);
       RTP_PROF(prof, "pbf_correct", s,
                launch_pbf_correct(pred[in], lambda, G.startEnd, pred[1 - in], pos[cur], vel[cur],
@@ -434,6 +437,8 @@ struct rtp_fluids {
     if (in != 1 - P && G.sortedN > n)
       RTP_PROF(prof, "copy_tail", s, launch_copy_f4(pred[in], pred[1 - P], n, G.sortedN, s));
     predFinal = in;
+    if (po.order)  // PassOrder::packed
+      po.packed = nullptr;
     if (vortOn) {
       RTP_PROF(prof, "pbf_vorticity", s,
                launch_pbf_vorticity(pred[in], G.startEnd, vel[cur], vort, n, c, L, s, po,
@@ -606,6 +611,7 @@ struct rtp_fluids {
     dev_free(nbList);
     dev_free(nbCount);
     dev_free(cols);
+    dev_free(packed);
     if (stream)
       (void)hipStreamDestroy(stream);
     stream = nullptr;
@@ -906,6 +912,7 @@ int rtp_fluids_create(const rtp_model_desc* d, rtp_fluids** out)
       (rc = dev_alloc(&h->resMetric, kMetricFloats)) || (rc = dev_alloc(&h->okey, maxN)) ||
       (rc = dev_alloc(&h->orank, maxN)) || (rc = dev_alloc(&h->oorder[0], maxN)) ||
       (rc = dev_alloc(&h->oorder[1], maxN)) || (rc = dev_alloc(&h->cols, h->grid.g.numCells)) ||
+      (rc = dev_alloc(&h->packed, maxN)) ||
       (rc = dev_alloc(&h->ocount.table[0], order_count_words(h->grid.g))) ||
       (rc = dev_alloc(&h->ocount.table[1], order_count_words(h->grid.g))) ||
       (rc = dev_alloc(&h->opart, scan_partials_needed(order_count_words(h->grid.g))))) {

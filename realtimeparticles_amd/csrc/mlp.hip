@@ -119,7 +119,8 @@ __device__ __forceinline__ float head_sum(f32x4 y)
 // quarter-rate transcendentals each.
 constexpr uint32_t kFwdTiles = 2;
 __global__ __launch_bounds__(256) void k_mlp_forward(const float* __restrict__ feat, uint32_t n, MlpDev m,
-                                                     float* __restrict__ out)
+                                                     float* __restrict__ out,
+                                                     float4* __restrict__ packed)
 {
   const uint32_t l = threadIdx.x & 63u, lr = l % 16u, lq = l / 16u;
   const InputScale inputs(m, lq);
@@ -165,8 +166,11 @@ __global__ __launch_bounds__(256) void k_mlp_forward(const float* __restrict__ f
       }
       const float v = head_sum(y) + b3;
       const uint32_t r = row0 + k * 16u + lr;
-      if (lq == 0 && r < n)
+      if (lq == 0 && r < n) {
         out[r] = v * m.outScale;
+        if (packed)
+          packed[r].w = v * m.outScale;
+      }
     }
   }
 }
@@ -441,13 +445,15 @@ inline uint32_t blocks_for(uint32_t n, uint32_t b) { return (n + b - 1u) / b; }
 
 }  // namespace
 
-void launch_mlp_forward(const float* feat, uint32_t n, const MlpDev& m, float* out, hipStream_t s)
+void launch_mlp_forward(const float* feat, uint32_t n, const MlpDev& m, float* out, hipStream_t s,
+                        float4* packed)
 {
   if (n == 0)
     return;
   // at most four workgroups a CU: a wave's weights are loaded once for all its rows
   const uint32_t blocks = blocks_for(n, 16u * kFwdTiles * 4u);
-  hipLaunchKernelGGL(k_mlp_forward, dim3(blocks < 1024u ? blocks : 1024u), dim3(256), 0, s, feat, n, m, out);
+  hipLaunchKernelGGL(k_mlp_forward, dim3(blocks < 1024u ? blocks : 1024u), dim3(256), 0, s, feat, n, m, out,
+                     packed);
 }
 
 // One workgroup a CU at most, so the partial gradients stay few; small batches spread their

@@ -93,8 +93,7 @@ __device__ __forceinline__ void drain(LaneQueue& q, const float4 p, const float4
       e[j] = rp[j * kQueueStride];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      o[j] = ldn(pred, e[j]);
-      x[j] = b.ld(e[j]);
+      b.fetch(pred, e[j], o[j], x[j]);
     }
     rec.granule(e);
 #pragma unroll
@@ -128,8 +127,7 @@ __device__ __forceinline__ void drain_rest(LaneQueue& q, const float4 p,
   for (uint32_t j = 0; j < 3u; ++j)
     if (j < m) {
       e[j] = q.slot[j * kQueueStride];
-      o[j] = ldn(pred, e[j]);
-      x[j] = b.ld(e[j]);
+      b.fetch(pred, e[j], o[j], x[j]);
     }
   rec.rest(e, m);
 #pragma unroll
@@ -224,6 +222,7 @@ struct WalkCtx {
   const float* y = nullptr;
   const float* z = nullptr;
   const uint2* cols = nullptr;             // the columns' ranges (k_columns)
+  float4* packed = nullptr;                // PassOrder::packed
   NbList nb;                               // survivor lists of a kNbRecord / kNbReplay pass
   uint32_t slot = 0;                       // this thread's column in them
 };
@@ -462,8 +461,7 @@ __device__ __forceinline__ void replay(const uint4* __restrict__ gp, uint32_t st
     typename B::Data x[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      o[j] = ldn(pred, e[j]);
-      x[j] = b.ld(e[j]);
+      b.fetch(pred, e[j], o[j], x[j]);
     }
     if (cnt > 4u) {
       gp += stride;
@@ -479,8 +477,7 @@ __device__ __forceinline__ void replay(const uint4* __restrict__ gp, uint32_t st
 #pragma unroll
   for (uint32_t j = 0; j < 3u; ++j)
     if (j < cnt) {
-      o[j] = ldn(pred, e[j]);
-      x[j] = b.ld(e[j]);
+      b.fetch(pred, e[j], o[j], x[j]);
     }
 #pragma unroll
   for (uint32_t j = 0; j < 3u; ++j)
@@ -675,6 +672,7 @@ __device__ __forceinline__ LdsWord* queue_slot(uint32_t* queue, uint32_t depth)
 #define RTP_NB_CTX   \
   W.nb = po.nb;      \
   W.cols = po.cols;  \
+  W.packed = po.packed; \
   W.slot = t;
 
 // fluids.cl:71-73 (newVel = vel + GRAVITY_ACC * dt; predPos = pos + newVel * dt) and
@@ -763,7 +761,11 @@ struct DensityBody {
   const PbfConsts& c;
   bool fast;
   float dens = 0.0f, sgx = 0.0f, sgy = 0.0f, sgz = 0.0f, ssq = 0.0f, count = 0.0f;
-  __device__ __forceinline__ int ld(uint32_t) const { return 0; }
+  __device__ __forceinline__ void fetch(const float4* __restrict__ pred, uint32_t e, float4& o,
+                                        int&) const
+  {
+    o = ldn(pred, e);
+  }
   // CK: with the checks (a replayed list may be known not to need them, walk27)
   template <bool CK>
   __device__ __forceinline__ Term term(const float4 p, const float4 o, int, bool& odd) const
@@ -811,7 +813,11 @@ struct DensityOnlyBody {
   const PbfConsts& c;
   bool fast;
   float dens = 0.0f;
-  __device__ __forceinline__ int ld(uint32_t) const { return 0; }
+  __device__ __forceinline__ void fetch(const float4* __restrict__ pred, uint32_t e, float4& o,
+                                        int&) const
+  {
+    o = ldn(pred, e);
+  }
   template <bool CK>
   __device__ __forceinline__ Term term(const float4 p, const float4 o, int, bool& odd) const
   {
@@ -852,6 +858,7 @@ __device__ __forceinline__ void density_lambda_body(uint32_t i, const float4* __
   sq = sq / c.rho0sq;
   const float lam = -C / (sq + c.p.relaxCFM);
   lambda[i] = lam;
+  T.packed[i] = make_float4(p.x, p.y, p.z, lam);
   if (MODE & kAccum)
     la.lamAcc[i] = la.accumInit ? lam : la.lamAcc[i] + lam;
   if (MODE & kFeatures) {
@@ -947,17 +954,31 @@ __device__ __forceinline__ void correct_out(uint32_t i, const float4 p, float cx
     posOut[i] = q;
 }
 
+// Positions and lambdas come together (the density pass packs them): a survivor costs one gather
+// instead of two.
+template <bool PACKED>
 struct CorrectBody {
   using Data = float;
   struct Term {
     float x, y, z;
   };
   const PbfConsts& c;
-  const float* __restrict__ lambda;
+  const float4* __restrict__ packed;  // positions with lambda in the w lane, or
+  const float* __restrict__ lambda;   // the lambdas beside the pass's positions
   bool fast;
   float li, ywdq;
   float cx = 0.0f, cy = 0.0f, cz = 0.0f;
-  __device__ __forceinline__ float ld(uint32_t e) const { return lambda[e]; }
+  __device__ __forceinline__ void fetch(const float4* __restrict__ pred, uint32_t e, float4& o,
+                                        float& x) const
+  {
+    if (PACKED) {
+      o = packed[e];
+      x = o.w;
+    } else {
+      o = ldn(pred, e);
+      x = lambda[e];
+    }
+  }
   template <bool CK>
   __device__ __forceinline__ Term term(const float4 p, const float4 o, float le, bool& odd) const
   {
@@ -1001,9 +1022,10 @@ __device__ __forceinline__ void correct_body(uint32_t i, const float4* __restric
                                              const WalkCtx& T, const PassOrder& po)
 {
   (void)la;
+  (void)lambda;
   const float4 p = pred[i];
   const float ywdq = (c.shortMath & kShortArtDiv) ? rcp_refined(c.wdq) : 0.0f;
-  CorrectBody b{ c, lambda, (c.shortMath & kShortSqrtGrad) != 0, lambda[i], ywdq };
+  CorrectBody<true> b{ c, T.packed, nullptr, (c.shortMath & kShortSqrtGrad) != 0, T.packed[i].w, ywdq };
   walk27<(MODE & (kNbRecord | kNbReplay))>(p, pred, se, c, b, T);
   correct_out(i, p, b.cx, b.cy, b.cz, predOut, pos, vel, posOut, last, c, po);
 }
@@ -1286,8 +1308,7 @@ __device__ __forceinline__ bool quad_run(uint32_t cnt, uint32_t self, const floa
     r.e = self;
     if (r.v)
       r.e = src(at);
-    r.o = ldn(pred, r.e);
-    r.x = b.ld(r.e);
+    b.fetch(pred, r.e, r.o, r.x);
   };
   auto run = [&](const Round& r) {
     rec(r.v, k, r.e);
@@ -1391,13 +1412,17 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
 // density_lambda_body's outputs (MODE 0) from a quad's sums.
 __device__ __forceinline__ void density_lambda_out(uint32_t i, const DensityBody& b,
                                                    float* __restrict__ density,
-                                                   float* __restrict__ lambda, const PbfConsts& c)
+                                                   float* __restrict__ lambda, const PbfConsts& c,
+                                                   const float4 p, float4* __restrict__ packed)
 {
   density[i] = b.dens;
   const float C = b.dens / c.p.restDensity - 1.0f;
   float sq = b.ssq + (b.sgx * b.sgx + b.sgy * b.sgy + b.sgz * b.sgz);
   sq = sq / c.rho0sq;
-  lambda[i] = -C / (sq + c.p.relaxCFM);
+  const float lam = -C / (sq + c.p.relaxCFM);
+  lambda[i] = lam;
+  if (packed)
+    packed[i] = make_float4(p.x, p.y, p.z, lam);
 }
 
 // The quad's survivors of particle i, into the body b: with NB == kNbReplay its survivor list
@@ -1448,7 +1473,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_density_lambda_quad(
     DensityBody b{ c, fast };
     quad_neighbours<REC ? kNbRecord : 0>(on, i, k, on & (k < cs), p, pred, se, c, nb, lds, b);
     if (on && (threadIdx.x & 3u) == 0u)
-      density_lambda_out(i, b, density, lambda, c);
+      density_lambda_out(i, b, density, lambda, c, p, nullptr);
   }
 }
 
@@ -1472,7 +1497,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_correct_quad(
     const bool on = k < cnt;
     const uint32_t i = on ? fs.list[k] : 0u;
     const float4 p = pred[i];
-    CorrectBody b{ c, lambda, fast, lambda[i], ywdq };
+    CorrectBody<false> b{ c, nullptr, lambda, fast, lambda[i], ywdq };
     quad_neighbours<REPLAY ? kNbReplay : 0>(on, i, k, false, p, pred, se, c, nb, lds, b);
     if (on && (threadIdx.x & 3u) == 0u)
       correct_out(i, p, b.cx, b.cy, b.cz, predOut, nullptr, nullptr, nullptr, last, c, po);
@@ -1519,7 +1544,12 @@ struct VorticityBody {
   bool fast;
   float4 vi;
   float wx = 0.0f, wy = 0.0f, wz = 0.0f;
-  __device__ __forceinline__ float4 ld(uint32_t e) const { return ldn(vel, e); }
+  __device__ __forceinline__ void fetch(const float4* __restrict__ pred, uint32_t e, float4& o,
+                                        float4& x) const
+  {
+    o = ldn(pred, e);
+    x = ldn(vel, e);
+  }
   template <bool CK>
   __device__ __forceinline__ Term term(const float4 p, const float4 o, const float4 ve,
                                        bool& odd) const
@@ -1565,7 +1595,10 @@ __device__ __forceinline__ void vorticity_body(uint32_t i, const float4* __restr
   const float4 p = pred[i];
   VorticityBody b{ c, vel, (c.shortMath & kShortSqrtGrad) != 0, vel[i] };
   walk27<NB>(p, pred, se, c, b, T);
-  vort[i] = make_float4(b.wx, b.wy, b.wz, __builtin_sqrtf(b.wx * b.wx + b.wy * b.wy + b.wz * b.wz));
+  const float size = __builtin_sqrtf(b.wx * b.wx + b.wy * b.wy + b.wz * b.wz);
+  vort[i] = make_float4(b.wx, b.wy, b.wz, size);
+  if (T.packed)
+    T.packed[i] = make_float4(p.x, p.y, p.z, size);
 }
 
 template <int NB>
@@ -1607,16 +1640,28 @@ __device__ __forceinline__ void confinement_out(uint32_t i, float nx, float ny, 
 
 // fld_applyVorticityConfinement (fluids.cl:329-377), writing the confined velocity to
 // velOut (the copy fld_applyXsphViscosityCorrection reads, Fluids.cpp:451).
+template <bool PACKED>
 struct ConfinementBody {
   using Data = float;
   struct Term {
     float x, y, z;
   };
   const PbfConsts& c;
-  const float4* __restrict__ vort;
+  const float4* __restrict__ packed;  // positions with |vorticity| in the w lane, or
+  const float4* __restrict__ vort;    // the vorticities beside the pass's positions
   bool fast;
   float nx = 0.0f, ny = 0.0f, nz = 0.0f;
-  __device__ __forceinline__ float ld(uint32_t e) const { return vort[e].w; }
+  __device__ __forceinline__ void fetch(const float4* __restrict__ pred, uint32_t e, float4& o,
+                                        float& x) const
+  {
+    if (PACKED) {
+      o = packed[e];
+      x = o.w;
+    } else {
+      o = ldn(pred, e);
+      x = vort[e].w;
+    }
+  }
   template <bool CK>
   __device__ __forceinline__ Term term(const float4 p, const float4 o, float le, bool& odd) const
   {
@@ -1657,8 +1702,8 @@ __device__ __forceinline__ void confinement_body(uint32_t i, const float4* __res
                                                  const WalkCtx& T)
 {
   const float4 p = pred[i];
-  ConfinementBody b{ c, vort, (c.shortMath & kShortSqrtGrad) != 0 };
-  walk27<NB>(p, pred, se, c, b, T);
+  ConfinementBody<(NB & kPacked) != 0> b{ c, T.packed, vort, (c.shortMath & kShortSqrtGrad) != 0 };
+  walk27<(NB & ~kPacked)>(p, pred, se, c, b, T);
   confinement_out(i, b.nx, b.ny, b.nz, vort, vel, velOut, c);
 }
 
@@ -1689,7 +1734,12 @@ struct XsphBody {
   bool fast;
   float4 vi;
   float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-  __device__ __forceinline__ float4 ld(uint32_t e) const { return ldn(velIn, e); }
+  __device__ __forceinline__ void fetch(const float4* __restrict__ pred, uint32_t e, float4& o,
+                                        float4& x) const
+  {
+    o = ldn(pred, e);
+    x = ldn(velIn, e);
+  }
   template <bool CK>
   __device__ __forceinline__ Term term(const float4 p, const float4 o, const float4 ve,
                                        bool& odd) const
@@ -1779,7 +1829,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_density_lambda_q(const float4* _
   DensityBody b{ c, fast };
   quad_neighbours<NB>(on, i, t, on, p, pred, se, c, po.nb, lds, b);
   if (lead)
-    density_lambda_out(i, b, density, lambda, c);
+    density_lambda_out(i, b, density, lambda, c, p, po.packed);
 }
 
 // k_correct (MODE 0 or kNbReplay) with a quad per particle.
@@ -1796,7 +1846,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_correct_q(const float4* __restri
   RTP_QUAD_PROLOGUE
   const float4 p = pred[i];
   const float ywdq = (c.shortMath & kShortArtDiv) ? rcp_refined(c.wdq) : 0.0f;
-  CorrectBody b{ c, lambda, fast, lambda[i], ywdq };
+  CorrectBody<true> b{ c, po.packed, nullptr, fast, po.packed[i].w, ywdq };
   quad_neighbours<NB>(on, i, t, false, p, pred, se, c, po.nb, lds, b);
   if (lead)
     correct_out(i, p, b.cx, b.cy, b.cz, predOut, pos, vel, posOut, last, c, po);
@@ -1814,8 +1864,12 @@ __global__ __launch_bounds__(kQuadBlock) void k_vorticity_q(const float4* __rest
   const float4 p = pred[i];
   VorticityBody b{ c, vel, fast, vel[i] };
   quad_neighbours<NB>(on, i, t, on, p, pred, se, c, po.nb, lds, b);
-  if (lead)
-    vort[i] = make_float4(b.wx, b.wy, b.wz, __builtin_sqrtf(b.wx * b.wx + b.wy * b.wy + b.wz * b.wz));
+  if (lead) {
+    const float size = __builtin_sqrtf(b.wx * b.wx + b.wy * b.wy + b.wz * b.wz);
+    vort[i] = make_float4(b.wx, b.wy, b.wz, size);
+    if (po.packed)
+      po.packed[i] = make_float4(p.x, p.y, p.z, size);
+  }
 }
 
 // k_confinement with a quad per particle.
@@ -1829,8 +1883,8 @@ __global__ __launch_bounds__(kQuadBlock) void k_confinement_q(const float4* __re
 {
   RTP_QUAD_PROLOGUE
   const float4 p = pred[i];
-  ConfinementBody b{ c, vort, fast };
-  quad_neighbours<NB>(on, i, t, false, p, pred, se, c, po.nb, lds, b);
+  ConfinementBody<(NB & kPacked) != 0> b{ c, po.packed, vort, fast };
+  quad_neighbours<(NB & ~kPacked)>(on, i, t, false, p, pred, se, c, po.nb, lds, b);
   if (lead)
     confinement_out(i, b.nx, b.ny, b.nz, vort, vel, velOut, c);
 }
@@ -1869,6 +1923,7 @@ __global__ __launch_bounds__(kQuadBlock) void k_xsph_q(const float4* __restrict_
   T.qslot = queue_slot(rtpQueue, qdepth);                                      \
   T.qcap = qdepth;                                                             \
   T.cols = po.cols;                                                            \
+  T.packed = po.packed;                                                        \
   build_tile(pred[i], pred, se, c, tl, T);                                     \
   __syncthreads();
 
@@ -1951,6 +2006,7 @@ __global__ __launch_bounds__(256) void k_xsph_t(const float4* __restrict__ pred,
 #define RTP_BATCH_NB_CTX             \
   W.nb = bv.nb;                      \
   W.cols = bv.cols + b.slot.kbase;   \
+  W.packed = bv.packed ? bv.packed + b.slot.pbase : nullptr; \
   W.slot = blockIdx.x * blockDim.x + threadIdx.x;
 
 struct BatchSite {
@@ -2376,6 +2432,11 @@ void launch_pbf_update_vel(const float4* pred, const float4* pos, float4* vel, f
     return nb == kNbRecord ? KERNEL<kNbRecord> : (nb == kNbReplay ? KERNEL<kNbReplay> : KERNEL<0>); \
   }
 
+// ... of the confinement: a recorded or replayed list, and packed or separate neighbour data.
+#define RTP_CONFINEMENT(KERNEL, nb, packed)                                                     \
+  ((packed) ? ((nb) == kNbReplay ? KERNEL<kNbReplay | kPacked> : KERNEL<kPacked>)              \
+            : ((nb) == kNbReplay ? KERNEL<kNbReplay> : KERNEL<0>))
+
 void launch_pbf_vorticity(const float4* pred, const uint2* startEnd, const float4* vel,
                           float4* vort, uint32_t n, const PbfConsts& c, const Launch& L,
                           hipStream_t s, const PassOrder& po, int nb)
@@ -2399,11 +2460,11 @@ void launch_pbf_confinement(const float4* pred, const uint2* startEnd, const flo
   if (n == 0)
     return;
   if (L.quad && !L.tile) {
-    hipLaunchKernelGGL(RTP_BY_NB(k_confinement_q)(nb), quad_grid(n), dim3(kQuadBlock), 0, s,
+    hipLaunchKernelGGL(RTP_CONFINEMENT(k_confinement_q, nb, po.packed), quad_grid(n), dim3(kQuadBlock), 0, s,
                        pred, startEnd, vort, vel, velOut, n, c, po);
     return;
   }
-  hipLaunchKernelGGL(L.tile ? k_confinement_t : RTP_BY_NB(k_confinement)(nb),
+  hipLaunchKernelGGL(L.tile ? k_confinement_t : RTP_CONFINEMENT(k_confinement, nb, po.packed),
                      dim3(blocks_for(n, L.block)), dim3(L.block), queue_bytes(L), s, pred,
                      startEnd, vort, vel, velOut, n, c, L.xcdRemap, (uint32_t)L.queue, po);
 }
@@ -2502,7 +2563,8 @@ void launch_pbf_confinement_batch(const BatchView& bv, const float4* pred, const
                                   const float4* vort, const float4* vel, float4* velOut,
                                   hipStream_t s, int nb)
 {
-  RTP_BATCH_LAUNCH(RTP_BATCH_NB(k_confinement_batch), pred, startEnd, vort, vel, velOut);
+  RTP_BATCH_LAUNCH(RTP_CONFINEMENT(k_confinement_batch, nb, bv.packed), pred, startEnd, vort, vel,
+                   velOut);
 }
 
 void launch_pbf_xsph_batch(const BatchView& bv, const float4* pred, const uint2* startEnd,

@@ -252,7 +252,8 @@ struct LearnArgs {
 // kNbRecord / kNbReplay: the pass records its threads' survivor lists / replays them
 // (NbList below).
 enum PassMode {
-  kFeatures = 1, kAccum = 2, kDensOnly = 4, kNbRecord = 32, kNbReplay = 64
+  kFeatures = 1, kAccum = 2, kDensOnly = 4, kNbRecord = 32, kNbReplay = 64,
+  kPacked = 128  // the confinement reads PassOrder::packed
 };
 // Survivor lists.  Two neighbour passes over the same positions, the same cell table and
 // the same thread order visit the same candidates and run their bodies on the same
@@ -282,6 +283,14 @@ struct PassOrder {
   int bricks = 0;                   //   1: brick_key of the cell instead of its index
   NbList nb;
   const uint2* cols = nullptr;      // the walks' column ranges (launch_pbf_columns)
+  // Per particle its position and, in the w lane, the datum the next pass needs of a neighbour:
+  // lambda from the density pass for the correction, |vorticity| (when not null then) for the
+  // confinement: one 16-byte gather a survivor instead of 12 and 4 bytes from two arrays.
+  // Correction 78 -> 64 us, confinement 94 -> 55 us at 968,375 particles in the grid's order.  In
+  // a thread order the packing pass writes scattered granules: the four corrections of 4,194,304
+  // particles gain 284 us against 144 more in the density passes, but the confinement 20 against
+  // 57 in the vorticity pass, so it keeps the separate arrays there.
+  float4* packed = nullptr;
   __device__ uint32_t particle(uint32_t t) const { return order ? order[t] : t; }
 };
 // The thread order's two count tables of `words` words each, both all zero when allocated.
@@ -327,6 +336,7 @@ struct BatchView {
   uint32_t* keyOut = nullptr;       // correction passes: batch-wide key of each output
   NbList nb;                        // survivor lists; a thread's slot is its launch-wide id
   const uint2* cols = nullptr;      // the walks' column ranges, scene by scene like the cell table
+  float4* packed = nullptr;         // PassOrder::packed of the whole batch
 };
 // The column ranges of the cell table (one per cell) that the one-lane walks read.
 void launch_pbf_columns(const uint2* startEnd, uint2* cols, const GridConsts& g, hipStream_t s);

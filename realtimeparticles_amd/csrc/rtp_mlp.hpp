@@ -31,7 +31,9 @@ struct MlpDev {
   float outScale;
 };
 
-void launch_mlp_forward(const float* feat, uint32_t n, const MlpDev& m, float* out, hipStream_t s);
+// packed: also the w lane of each row's float4, if not null.
+void launch_mlp_forward(const float* feat, uint32_t n, const MlpDev& m, float* out, hipStream_t s,
+                        float4* packed = nullptr);
 // Partial gradients of a batch: one per workgroup of the training kernel, kMlpPartial floats
 // each (the gradient in the parameter layout, the squared-error sum, padding).
 constexpr uint32_t kMlpMaxBlocks = 256;
