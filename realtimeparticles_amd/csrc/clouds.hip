@@ -613,7 +613,7 @@ __device__ __forceinline__ float4 cq_shifted(float4 vec, uint32_t code, const Gr
 
 // The body over entries 0..cnt-1 of the quad (entry(k): entry k, an index with its shift
 // code), four at a time, loading each round's data during the previous round's bodies, in two
-// register sets by turns; rec(v, k, code) sees every round first.  The wave loops until its
+// register sets by turns, and its entries a round before; rec(v, k, code) sees every round first.  The wave loops until its
 // longest quad is done; lanes without an entry run the body on the particle itself and add +0.
 template <class S, class R, class B>
 __device__ __forceinline__ void cq_run(uint32_t cnt, uint32_t self, const float4 pos,
@@ -630,13 +630,19 @@ __device__ __forceinline__ void cq_run(uint32_t cnt, uint32_t self, const float4
     float4 o;
     decltype(b.ld(0u)) x;
   };
+  const auto index = [&](uint32_t at) {
+    uint32_t code = self;
+    if (at < cnt)
+      code = entry(at);
+    return code;
+  };
+  uint32_t ahead = index(k);  // of the next round to load
   const auto load = [&](Round& r, uint32_t at) {
     r.v = at < cnt;
-    r.code = self;
-    if (r.v)
-      r.code = entry(at);
+    r.code = ahead;
     r.o = src[r.code & kCldIndexMask];
     r.x = b.ld(r.code & kCldIndexMask);
+    ahead = index(at + 4u);
   };
   const auto run = [&](const Round& r) {
     rec(r.v, k, r.code);

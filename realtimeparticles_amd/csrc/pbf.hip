@@ -1285,7 +1285,7 @@ __device__ __forceinline__ uint32_t quad_ranges(const float4 p, const uint2* __r
 
 // Runs the body over survivors 0..cnt-1 of the quad (src(v, k): survivor k, when v), four at a
 // time (lane u: survivors u, u + 4, ...), loading each round's data during the previous round's
-// bodies, in two register sets by turns; rec(v, k, e) sees every round first.  CK: terms with the
+// bodies, in two register sets by turns, and its indices a round before; rec(v, k, e) sees every round first.  CK: terms with the
 // checks; returns whether one of the lane's needed them.  The wave loops until its longest quad
 // is done; empty lanes run the body on the particle itself and add +0.
 template <bool CK, class S, class R, class B>
@@ -1303,12 +1303,18 @@ __device__ __forceinline__ bool quad_run(uint32_t cnt, uint32_t self, const floa
     float4 o;
     typename B::Data x;
   };
+  auto index = [&](uint32_t at) {
+    uint32_t e = self;
+    if (at < cnt)
+      e = src(at);
+    return e;
+  };
+  uint32_t ahead = index(k);  // of the next round to load: its data wait for one load, not two
   auto load = [&](Round& r, uint32_t at) {
     r.v = at < cnt;
-    r.e = self;
-    if (r.v)
-      r.e = src(at);
+    r.e = ahead;
     b.fetch(pred, r.e, r.o, r.x);
+    ahead = index(at + 4u);
   };
   auto run = [&](const Round& r) {
     rec(r.v, k, r.e);
