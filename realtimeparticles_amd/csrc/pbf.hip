@@ -2051,14 +2051,13 @@ __global__ __launch_bounds__(256) void k_fill_start_end(uint2* __restrict__ se, 
     se[t] = make_uint2(1u, 0u);  // grid.cl:91-96
 }
 
-// k_columns of scene blockIdx.y.
+// k_columns of scene blockIdx.x, its cells over blockIdx.y.
 __global__ __launch_bounds__(256) void k_columns_batch(BatchView bv, const uint2* __restrict__ se,
                                                        uint2* __restrict__ cols)
 {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  const PbfConsts& c = bv.consts[blockIdx.y];
-  const uint32_t base = bv.scenes[blockIdx.y].kbase;
-  if (t < c.g.numCells)
+  const PbfConsts& c = bv.consts[blockIdx.x];
+  const uint32_t base = bv.scenes[blockIdx.x].kbase;
+  for (uint32_t t = blockIdx.y * 256u + threadIdx.x; t < c.g.numCells; t += gridDim.y * 256u)
     column_body(t, se + base, cols + base, c.g);
 }
 
@@ -2278,9 +2277,10 @@ void launch_pbf_columns(const uint2* startEnd, uint2* cols, const GridConsts& g,
 void launch_pbf_columns_batch(const BatchView& bv, const uint2* startEnd, uint2* cols,
                               uint32_t numScenes, uint32_t maxCells, hipStream_t s)
 {
-  if (numScenes && maxCells)
-    hipLaunchKernelGGL(k_columns_batch, dim3(blocks_for(maxCells, 256), numScenes), dim3(256), 0, s,
-                       bv, startEnd, cols);
+  const uint32_t y = blocks_for(maxCells, 256);
+  if (numScenes && y)
+    hipLaunchKernelGGL(k_columns_batch, dim3(numScenes, y < 1024u ? y : 1024u), dim3(256), 0, s, bv,
+                       startEnd, cols);
 }
 
 void launch_pbf_density_lambda(const float4* pred, const uint2* startEnd, float* density,

@@ -241,6 +241,25 @@ def test_dense_ball_overflows_the_survivor_lists_bit_exact(quad):
     gpu.close()
 
 
+@pytest.mark.parametrize("res", [(2, 3, 2), (3, 2, 4), (1, 4, 3), (6, 4, 5)])
+@pytest.mark.parametrize("n", [3, 70, 700])
+def test_small_grids_wrap_in_x_and_z_bit_exact(res, n):
+    """Grids of one to six cells a side, whose neighbour columns wrap in x and z with the shift of
+    their walls, and models down to three particles: the ranges the quad's lanes find together."""
+    rng = np.random.default_rng(n + res[0])
+    box = tuple(float(np.float32(r / 3.0)) for r in res)
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :3] = (rng.random((n, 3), dtype=np.float32) - np.float32(0.5)) * np.array(box, np.float32)
+    sc = scenes.CloudScene("", box, res, n, 1024, pos, np.zeros_like(pos))
+    gpu, orc = make_pair(sc, iters=2, quad=True)
+    for step in range(1, 4):
+        gpu.update(1)
+        orc.step(1)
+        log(f"clouds grid {res}, n {n}, step {step}")
+        compare(gpu, orc, n, f"step {step}")
+    gpu.close()
+
+
 @pytest.mark.parametrize("quad", [True, False])
 def test_infinite_velocity_spreads_nan_bit_exact(quad):
     """One particle with an infinite velocity: its predicted position is infinite, so the

@@ -446,6 +446,33 @@ def test_checked_pairs_in_lists_keep_bits(flags, queue, n):
         gpu.close()
 
 
+@pytest.mark.parametrize("res", [(2, 2, 2), (5, 3, 2), (4, 2, 3), (3, 4, 5)])
+@pytest.mark.parametrize("flags", [0, 2, 8, 13, 64, 72])
+def test_grids_that_wrap_in_every_column(flags, res):
+    """Grids of two to five cells a side: most columns wrap, so their cells are not one index range
+    (and with two cells a side two of them are the same cell), in the one-lane walks' column table
+    and in the quads' ranges."""
+    rng = np.random.default_rng(sum(res))
+    n = 40 * res[0] * res[1] * res[2] // 4
+    box = tuple(np.float32(r * 0.1) for r in res)
+    sc = scenes.dam_break((4, 4, 4), (4, 2, 2), (40, 20, 20), seed=1)
+    sc.box, sc.res, sc.n, sc.max_n = tuple(float(b) for b in box), res, n, 1024
+    sc.pos = np.zeros((n, 4), np.float32)
+    sc.pos[:, :3] = (rng.random((n, 3), dtype=np.float32) - np.float32(0.5)) * np.array(box, np.float32)
+    sc.vel = np.zeros_like(sc.pos)
+    gpu, orc = make_pbf_pair(sc, iters=2, **sc.params("stable"))
+    gpu.set_tuning(64, flags, 0, 16)
+    gpu.save_checkpoint()
+    gpu.update(1)
+    gpu.restore_checkpoint()
+    for step in range(1, 4):
+        log(f"wrapping grid {res}, flags {flags}, step {step}")
+        gpu.update(1)
+        orc.step(1)
+        compare_pbf(gpu, orc, sc.n, step)
+    gpu.close()
+
+
 @pytest.mark.parametrize("box", [(0.2, 0.1, 0.1), (800.0, 400.0, 400.0)])
 def test_general_forms_outside_short_range(box):
     """Effect radius h = 0.005 and h = 20, outside [2^-7, 2^4] where the short correctly
