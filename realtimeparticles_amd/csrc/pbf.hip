@@ -1285,9 +1285,10 @@ __device__ __forceinline__ uint32_t quad_ranges(const float4 p, const uint2* __r
 
 // Runs the body over survivors 0..cnt-1 of the quad (src(v, k): survivor k, when v), four at a
 // time (lane u: survivors u, u + 4, ...), loading each round's data during the previous round's
-// bodies, in two register sets by turns, and its indices a round before; rec(v, k, e) sees every round first.  CK: terms with the
-// checks; returns whether one of the lane's needed them.  The wave loops until its longest quad
-// is done; empty lanes run the body on the particle itself and add +0.
+// bodies, in two register sets by turns, and its indices a round before; rec(v, k, e) sees every
+// round first.  CK: terms with the checks; returns whether one of the lane's needed them.  The
+// wave loops until its longest quad is done; empty lanes run the body on the particle itself and
+// add +0.
 template <bool CK, class S, class R, class B>
 __device__ __forceinline__ bool quad_run(uint32_t cnt, uint32_t self, const float4 p,
                                          const float4* __restrict__ pred, S&& src, R&& rec, B& b)
