@@ -118,7 +118,8 @@ typedef struct {
                                   particle (results unchanged; not with RTP_LAUNCH_LDS_TILES).
                                   The default shape of a model of at most 262,144 particles
                                   (maxNbParticles) has it, and a fluids model's also
-                                  RTP_LAUNCH_NB_LIST where the device has the memory;
+                                  RTP_LAUNCH_NB_LIST when more than half of the device's
+                                  memory is free as it is created;
                                   set_tuning / autotune replace it */
 
 /* Which buffers rtp_fluids_read_field copies. */

@@ -930,13 +930,14 @@ int rtp_fluids_create(const rtp_model_desc* d, rtp_fluids** out)
   // The default shape of a small model replays survivor lists (1 KiB per particle, at most
   // 256 MiB), which takes the walk out of half its passes: 131,072 particles with the app's
   // parameters and rendering steps 236 -> 181 us a frame, 8,192 particles 191 -> 155 us until done.
-  // Without the memory it walks.
-  if (h->L.quad) {
+  // With less than half of the device's memory free it walks: the lists are four times a model's
+  // other buffers, so that half is left to further models' and the program's own.
+  size_t freeBytes = 0, allBytes = 0;
+  if (h->L.quad && hipMemGetInfo(&freeBytes, &allBytes) == hipSuccess && freeBytes > allBytes / 2u)
     h->L.nbList = h->alloc_lists() == RTP_OK ? 1 : 0;
-    if (!h->L.nbList) {
-      (void)hipGetLastError();
-      fail(RTP_OK, "");
-    }
+  if (h->L.quad && !h->L.nbList) {
+    (void)hipGetLastError();
+    fail(RTP_OK, "");
   }
   h->refresh_consts();
   // Zero state and the reset key tail, like the constructor's reset() (Fluids.cpp:91).
