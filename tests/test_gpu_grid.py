@@ -8,7 +8,8 @@ from realtimeparticles_amd import capi, scenes
 pytestmark = pytest.mark.gpu
 
 
-# 4096 / 4097 and 8192 / 8193 straddle the one-workgroup sort's chunk sizes and its limit;
+# 2048, 4096 and 8192 are whole workgroups of the two-launch pass (1,024 keys each), their
+# neighbours not;
 # 2^18, 2^20 and 2^22 the multi-launch sort's subtile sizes (4, 8, 16 and 32 keys per lane)
 @pytest.mark.parametrize("n", [1, 63, 64, 2047, 2048, 2049, 4096, 4097, 8191, 8192, 8193, 65536,
                                100003, (1 << 18) - 1, 1 << 18, (1 << 20) - 1, 1 << 20,
@@ -34,6 +35,21 @@ def test_sort_pairs_every_digit_width(n, bits):
     hi = 2 * 256000 + n
     keys = rng.integers(0, hi, n, dtype=np.uint64).astype(np.uint32)
     out, perm = capi.sort_pairs(keys, max_key=hi - 1, digit_bits=bits)
+    ref = np.argsort(keys, kind="stable")
+    _eq(perm, ref.astype(np.uint32), "perm")
+    _eq(out, keys[ref], "keys")
+
+
+@pytest.mark.parametrize("n, bits", [(1023, 8), (1024, 9), (1025, 10), ((1 << 18) - 1, 8), ((1 << 18) - 1, 9),
+                                     (1 << 17, 10), ((1 << 17) + 1, 10), (1 << 16, 11), ((1 << 16) + 1, 11)])
+def test_sort_pairs_at_the_row_sum_limits(n, bits):
+    """The largest two-launch passes of each width (512 row words a thread) and the smallest sorts past
+    them; half of the keys in one cell, so one digit's column holds most of the count."""
+    log(f"sort_pairs n={n} bits={bits}")
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(0, 1 << (2 * bits), n, dtype=np.uint64).astype(np.uint32)
+    keys[::2] = (1 << (2 * bits)) - 1
+    out, perm = capi.sort_pairs(keys, max_key=(1 << (2 * bits)) - 1, digit_bits=bits)
     ref = np.argsort(keys, kind="stable")
     _eq(perm, ref.astype(np.uint32), "perm")
     _eq(out, keys[ref], "keys")
