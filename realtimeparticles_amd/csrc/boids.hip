@@ -495,7 +495,7 @@ __device__ __forceinline__ void boids_sums_quad(bool on, uint32_t self, const fl
   if (__builtin_amdgcn_ballot_w64(nr > 0u) == 0)
     return;
   wave_sync();
-  uint32_t ri = 0, qn = 0;
+  uint32_t qn = 0;
   struct Round {
     bool v;
     float4 q, nv;
@@ -531,44 +531,31 @@ __device__ __forceinline__ void boids_sums_quad(bool on, uint32_t self, const fl
     qn = 0;
     wave_sync();
   };
-  // the lane's first candidate of the step and the last of the quad's range (none: 1 and 0)
-  uint32_t e = 1u, hi = 0u;
-  const auto range = [&]() {
-    e = rl[ri].x + u;
-    hi = rl[ri].y;
-  };
+  QuadScan<uint2> at(rl, nr, u);
   const auto load = [&](float4* o) {  // also past the range (kPosPad)
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j) {
-      const float* f = reinterpret_cast<const float*>(position + e + 4u * j);
+      const float* f = reinterpret_cast<const float*>(position + at.e + 4u * j);
       o[j] = make_float4(f[0], f[1], f[2], 0.0f);
     }
   };
   // tests the step whose positions are in o; the next one's load meanwhile
   const auto step = [&](const float4* o, float4* next) {
-    const uint32_t first = e;
-    const int32_t left = (int32_t)(hi - e);
-    e += 16u;
-    if (ri < nr && e - u > hi) {
-      e = 1u;
-      hi = 0u;
-      if (++ri < nr)
-        range();
-    }
+    const uint32_t first = at.e;
+    const int32_t left = (int32_t)(at.hi - at.e);
+    at.next();
     load(next);
     bool k[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       k[j] = boids_near(boids_sq(p, o[j]), c) & (left >= 4 * j);
-    const QuadSlots at = quad_slots(k);
+    const QuadSlots places = quad_slots(k);
     uint32_t* const w = q + qn;
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j)
-      *(k[j] ? w + at.slot(j) : q + kBoidsQuadQueue) = first + 4u * j;
-    qn += at.all();
+      *(k[j] ? w + places.slot(j) : q + kBoidsQuadQueue) = first + 4u * j;
+    qn += places.all();
   };
-  if (nr > 0)
-    range();
   float4 o0[4], o1[4];
   load(o0);
   do {
@@ -576,7 +563,7 @@ __device__ __forceinline__ void boids_sums_quad(bool on, uint32_t self, const fl
     step(o1, o0);
     if (__builtin_amdgcn_ballot_w64(qn > kBoidsQuadQueue - 32u) != 0)
       drain();
-  } while (__builtin_amdgcn_ballot_w64(ri < nr) != 0);
+  } while (__builtin_amdgcn_ballot_w64(at.more()) != 0);
   drain();
 }
 

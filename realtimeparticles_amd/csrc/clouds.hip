@@ -672,7 +672,7 @@ __device__ __forceinline__ void cq_walk(uint32_t nr, const uint2* rl, uint32_t* 
                                         bool record, bool keepAll)
 {
   const uint32_t u = threadIdx.x & 3u;
-  uint32_t ri = 0, qn = 0, tot = 0;
+  uint32_t qn = 0, tot = 0;
   wave_sync();  // the quad's lanes wrote the ranges
   const auto drain = [&]() {
     wave_sync();
@@ -685,32 +685,17 @@ __device__ __forceinline__ void cq_walk(uint32_t nr, const uint2* rl, uint32_t* 
     qn = 0;
     wave_sync();
   };
-  // the lane's first candidate of the step, the last of the quad's range (none: 1 and 0) and
-  // the range's shift code
-  uint32_t e = 1u, hi = 0u, tag = 0u;
-  const auto range = [&]() {
-    const uint2 r = rl[ri];
-    e = (r.x & kCldIndexMask) + u;
-    tag = r.x & ~kCldIndexMask;
-    hi = r.y;
-  };
+  QuadScan<uint2, kCldIndexMask> at(rl, nr, u);
   const auto load = [&](float4* o) {  // also past the range (kPosPad)
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j)
-      o[j] = src[e + 4u * j];
+      o[j] = src[at.e + 4u * j];
   };
   // tests the step whose positions are in o; the next one's load meanwhile
   const auto step = [&](const float4* o, float4* next) {
-    const uint32_t first = e, code = tag;
-    const int32_t left = (int32_t)(hi - e);
-    e += 16u;
-    if (ri < nr && e - u > hi) {
-      e = 1u;
-      hi = 0u;
-      tag = 0u;
-      if (++ri < nr)
-        range();
-    }
+    const uint32_t first = at.e, code = at.code;
+    const int32_t left = (int32_t)(at.hi - at.e);
+    at.next();
     load(next);
     bool k[4];
 #pragma unroll
@@ -721,15 +706,13 @@ __device__ __forceinline__ void cq_walk(uint32_t nr, const uint2* rl, uint32_t* 
       else
         k[j] = (left >= 4 * j) && b.keep(b.ld(first + 4u * j), vec);
     }
-    const QuadSlots at = quad_slots(k);
+    const QuadSlots places = quad_slots(k);
     uint32_t* const w = q + qn;
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j)
-      *(k[j] ? w + at.slot(j) : q + kCqQueue) = (first + 4u * j) | code;
-    qn += at.all();
+      *(k[j] ? w + places.slot(j) : q + kCqQueue) = (first + 4u * j) | code;
+    qn += places.all();
   };
-  if (nr > 0)
-    range();
   if (__builtin_amdgcn_ballot_w64(nr > 0u) != 0) {
     float4 o0[4], o1[4];
     load(o0);
@@ -738,7 +721,7 @@ __device__ __forceinline__ void cq_walk(uint32_t nr, const uint2* rl, uint32_t* 
       step(o1, o0);
       if (__builtin_amdgcn_ballot_w64(qn > kCqQueue - 32u) != 0)
         drain();
-    } while (__builtin_amdgcn_ballot_w64(ri < nr) != 0);
+    } while (__builtin_amdgcn_ballot_w64(at.more()) != 0);
   }
   drain();
   if (REC && record && u == 0u)

@@ -1347,7 +1347,7 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
                                           B& b, const NbList& nb, uint32_t slot, bool record)
 {
   const uint32_t u = threadIdx.x & 3u;
-  uint32_t ri = 0, qn = 0, tot = 0;
+  uint32_t qn = 0, tot = 0;
   bool odd = false;
   wave_sync();  // the quad's lanes wrote the ranges
   auto drain = [&]() {
@@ -1361,43 +1361,29 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
     qn = 0;
     wave_sync();
   };
-  // the lane's first candidate of the step and the last of the quad's range (none: 1 and 0)
-  uint32_t e = 1u, hi = 0u;
-  auto range = [&]() {
-    const uint2 r = rl[ri];
-    e = r.x + u;
-    hi = r.y;
-  };
+  QuadScan<uint2> at(rl, nr, u);
   auto load = [&](float4* o) {  // also past the range (kPosPad)
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j)
-      o[j] = ldn(pred + e, 4u * j);
+      o[j] = ldn(pred + at.e, 4u * j);
   };
   // tests the step whose positions are in o; the next one's load meanwhile
   auto step = [&](const float4* o, float4* next) {
-    const uint32_t first = e;
-    const int32_t left = (int32_t)(hi - e);
-    e += 16u;
-    if (ri < nr && e - u > hi) {
-      e = 1u;
-      hi = 0u;
-      if (++ri < nr)
-        range();
-    }
+    const uint32_t first = at.e;
+    const int32_t left = (int32_t)(at.hi - at.e);
+    at.next();
     load(next);
     bool k[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       k[j] = near_or_far(p, o[j], c) & (left >= 4 * j);
-    const QuadSlots at = quad_slots(k);
+    const QuadSlots places = quad_slots(k);
     uint32_t* const w = q + qn;
 #pragma unroll
     for (uint32_t j = 0; j < 4u; ++j)
-      *(k[j] ? w + at.slot(j) : q + kQuadQueue) = first + 4u * j;
-    qn += at.all();
+      *(k[j] ? w + places.slot(j) : q + kQuadQueue) = first + 4u * j;
+    qn += places.all();
   };
-  if (nr > 0)
-    range();
   if (__builtin_amdgcn_ballot_w64(nr > 0) != 0) {
     float4 o0[4], o1[4];
     load(o0);
@@ -1406,7 +1392,7 @@ __device__ __forceinline__ void quad_walk(uint32_t nr, const uint2* rl, uint32_t
       step(o1, o0);
       if (__builtin_amdgcn_ballot_w64(qn > kQuadQueue - 32u) != 0)
         drain();
-    } while (__builtin_amdgcn_ballot_w64(ri < nr) != 0);
+    } while (__builtin_amdgcn_ballot_w64(at.more()) != 0);
   }
   drain();
   if (REC) {

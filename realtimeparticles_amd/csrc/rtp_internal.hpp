@@ -7,6 +7,7 @@
 #include <string>
 
 #include "rtp.h"
+#include "rtp_quad_scan.hpp"
 
 namespace rtp {
 
@@ -59,9 +60,6 @@ struct PbfConsts {
 // Squared distances at and above this take the reference's exact expressions (its
 // zero-weighted poly6 overflows to NaN well above it).
 constexpr float kFarD2 = 1.0e12f;
-// Positions past the last that a neighbour walk's loads of four, or a quad's of sixteen, may read
-// (and drop).
-constexpr uint32_t kPosPad = 16;
 enum ShortMath { kShortSqrtGrad = 1, kShortArtDiv = 2 };
 
 struct BoidsConsts {
