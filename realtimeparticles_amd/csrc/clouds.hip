@@ -109,7 +109,6 @@ __device__ __forceinline__ float len_of(float d2) { return sqrt_cr(d2); }
 // carry w = 0, is +-0 and its own quotient.  The other lanes (nonzero vv under 2^-52, a
 // nonzero numerator under 2^-90, a root whose significand is all ones, r >= h, NaN) take the
 // general expressions.
-constexpr uint32_t kNearVv = 0x25800000u;  // 2^-52
 struct CldPair {
   float r;
   float4 g;
@@ -117,7 +116,7 @@ struct CldPair {
 };
 __device__ __forceinline__ CldPair cld_pair(float4 vec, float vv, const PbfConsts& c)
 {
-  const Root q = root_short(vv);
+  const Root q = root_pair(vv);
   CldPair o;
   o.r = q.r;
   const float p2 = (c.h - q.r) * (c.h - q.r);
@@ -129,17 +128,18 @@ __device__ __forceinline__ CldPair cld_pair(float4 vec, float vv, const PbfConst
   o.w = c.poly6 * cube(c.hh - q.r * q.r);
   // whether some lane may need the general expressions, as in the fluids' pairs: a root ending
   // in 16 ones, or a numerator under vv * 2^-38 (at least 2^-90 beyond the near bound)
-  const bool near = __float_as_uint(vv) - 1u < kNearVv - 1u;
+  const bool near = root_near(vv), apart = vv != 0.0f;
   const bool out = !(q.r < c.h);
   const bool shortForm = (c.shortMath & kShortSqrtGrad) != 0;
   const float m = __builtin_fminf(__builtin_fminf(__builtin_fabsf(n.x), __builtin_fabsf(n.y)),
                                   __builtin_fabsf(n.z));
   const bool low = (uint16_t)__float_as_uint(q.r) == 0xffffu;
-  if ((__builtin_amdgcn_ballot_w64(near) | __builtin_amdgcn_ballot_w64(out) |
-       __builtin_amdgcn_ballot_w64(m < vv * 0x1p-38f) | __builtin_amdgcn_ballot_w64(low)) != 0 ||
+  if (((__builtin_amdgcn_ballot_w64(near) & __builtin_amdgcn_ballot_w64(apart)) |
+       __builtin_amdgcn_ballot_w64(out) | __builtin_amdgcn_ballot_w64(m < vv * 0x1p-38f) |
+       __builtin_amdgcn_ballot_w64(low)) != 0 ||
       !shortForm) {
     rare_path();
-    if (near | out | !shortForm | tiny_numerator3(n.x, n.y, n.z) | ones_significand(q.r)) {
+    if ((near & apart) | out | !shortForm | tiny_numerator3(n.x, n.y, n.z) | ones_significand(q.r)) {
       o.r = __builtin_sqrtf(vv);
       o.g = grad_spiky_r(vec, o.r, c);
       o.w = poly6_r(o.r, c);

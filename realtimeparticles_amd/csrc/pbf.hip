@@ -554,12 +554,13 @@ __device__ __forceinline__ float poly6_in(float r, const PbfConsts& c)
 }
 
 // A pair in the short correctly rounded forms: its squared distance, r = sqrtf(d2) and spiky
-// gradient g (grad_spiky(dx, dy, dz, r, 1, c); +-0 for d2 = 0, whose numerators are +-0).  The
-// reciprocal of the root comes from the same estimate and the quotients take one remainder
-// correction, about 20 issue slots fewer than with separate v_sqrt and v_rcp forms.  Right
-// except where where_pair_odd says.
+// gradient g (grad_spiky(dx, dy, dz, r, 1, c); +-0 for d2 = 0, whose reciprocal is taken as 0:
+// differences whose squares underflow are not 0).  The reciprocal of the root comes from the same
+// estimate and the quotients take one remainder correction, about 20 issue slots fewer than with
+// separate v_sqrt and v_rcp forms.  Right except where where_pair_odd says.
 struct Pair {
   float d2, r;
+  bool near;         // d2 < 2^-52
   float nx, ny, nz;  // numerators of g
   Grad g;
 };
@@ -568,8 +569,9 @@ __device__ __forceinline__ Pair pair_short(const float4 p, const float4 o, const
   const float dx = p.x - o.x, dy = p.y - o.y, dz = p.z - o.z;
   Pair k;
   k.d2 = dx * dx + dy * dy + dz * dz;
-  const Root q = root_short(k.d2);
+  const Root q = root_pair(k.d2);
   k.r = q.r;
+  k.near = root_near(k.d2);
   const float p2 = (c.h - q.r) * (c.h - q.r);
   k.nx = ((dx * c.spiky) * -3.0f) * p2;
   k.ny = ((dy * c.spiky) * -3.0f) * p2;
@@ -581,29 +583,29 @@ __device__ __forceinline__ Pair pair_short(const float4 p, const float4 o, const
   return k;
 }
 
-// f() in the lanes whose pair needs the reference's expressions instead: r >= h or NaN (weight 0, NaN when
-// very far), a parameter set without the short forms, a nonzero d2 under 2^-52 (which covers
-// 0 < r <= kFloatEps and the roots' own 2^-96), a nonzero numerator under 2^-90, or a root whose
-// significand is all ones.  Nearly no wave has such a lane, so six instructions decide first
-// whether one may: the low half of the root for its significand, and the smallest numerator
-// against d2 * 2^-38 (at least 2^-90 beyond the near bound, and 0 for a particle's pair with
-// itself, whose numerators are 0), which a pair with one equal coordinate does not pass.
-constexpr uint32_t kNearD2 = 0x25800000u;  // 2^-52
+// f() in the lanes whose pair needs the reference's expressions instead: r >= h or NaN (weight 0,
+// NaN when very far), a parameter set without the short forms, a nonzero d2 under 2^-52 (which
+// covers 0 < r <= kFloatEps), a nonzero numerator under 2^-90, or a root whose significand is all
+// ones.  Nearly no wave has such a lane, so a few instructions decide first whether one may: the
+// low half of the root for its significand, and the smallest numerator against d2 * 2^-38 (at
+// least 2^-90 beyond the near bound, and 0 for a particle's pair with itself), which a pair with
+// one equal coordinate does not pass.
 template <class F>
 __device__ __forceinline__ void where_pair_odd(const Pair& k, bool fast, const PbfConsts& c,
                                                bool& any, F&& f)
 {
-  const bool near = __float_as_uint(k.d2) - 1u < kNearD2 - 1u;
+  const bool apart = k.d2 != 0.0f;
   const bool out = !(k.r < c.h);
   const float m = __builtin_fminf(__builtin_fminf(__builtin_fabsf(k.nx), __builtin_fabsf(k.ny)),
                                   __builtin_fabsf(k.nz));
   const bool low = (uint16_t)__float_as_uint(k.r) == 0xffffu;
   // a ballot each: ored as scalars, one VALU comparison a test
-  if ((__builtin_amdgcn_ballot_w64(near) | __builtin_amdgcn_ballot_w64(out) |
-       __builtin_amdgcn_ballot_w64(m < k.d2 * 0x1p-38f) | __builtin_amdgcn_ballot_w64(low)) != 0 ||
+  if (((__builtin_amdgcn_ballot_w64(k.near) & __builtin_amdgcn_ballot_w64(apart)) |
+       __builtin_amdgcn_ballot_w64(out) | __builtin_amdgcn_ballot_w64(m < k.d2 * 0x1p-38f) |
+       __builtin_amdgcn_ballot_w64(low)) != 0 ||
       !fast) {
     rare_path();
-    if (near | out | !fast | tiny_numerator3(k.nx, k.ny, k.nz) | ones_significand(k.r)) {
+    if ((k.near & apart) | out | !fast | tiny_numerator3(k.nx, k.ny, k.nz) | ones_significand(k.r)) {
       any = true;
       f();
     }
@@ -621,7 +623,7 @@ template <class F>
 __device__ __forceinline__ void where_root_odd(float d2, float r, bool fast, const PbfConsts& c,
                                                bool& any, F&& f)
 {
-  const bool near = __float_as_uint(d2) - 1u < kNearD2 - 1u;
+  const bool near = __float_as_uint(d2) - 1u < kRootNear - 1u;
   const bool out = !(r < c.h);
   if ((__builtin_amdgcn_ballot_w64(near) | __builtin_amdgcn_ballot_w64(out)) != 0 || !fast) {
     rare_path();

@@ -6,16 +6,18 @@
 // 2^-96 by 2^32 and patches +-0 / +inf afterwards (v_cmp_class); a division range-reduces
 // both operands with v_div_scale, post-scales in v_div_fmas and patches special cases in
 // v_div_fixup.  Inside the ranges below the following shorter sequences return the same bits
-// (checked on the GPU against the compiled general forms: every float for the square root and
-// its reciprocal, every pair of significands for the division; rtp_selfcheck_*):
+// (checked on the GPU against the compiled general forms: every float for the square root, every
+// finite one from 2^-52 on for its reciprocal; for the division every divisor significand against
+// 2,047 numerators at the corners of the ranges, and every pair of significands at one pair of
+// exponents with selfcheck --exhaustive; rtp_selfcheck_*):
 //
 //   square root: y = v_rsq_f32(x), s0 = x*y, s = s0 + (x - s0*s0)*(y/2), for x = 0 (y is
 //   taken of 2^-96 there), x >= 2^-96 or NaN;
 //
 //   reciprocal of a divisor d > 0 in [2^-40, 2^40]: y0 = rcp(d), y = y0 + (1 - d*y0)*y0,
 //   which is the correctly rounded 1/d for every significand.  The same step from y0 =
-//   v_rsq_f32(x) gives the correctly rounded reciprocal of s = sqrtf(x) except where the
-//   significand of s is all ones (there the step's tie goes the wrong way);
+//   v_rsq_f32(x), x >= 2^-52, gives the correctly rounded reciprocal of s = sqrtf(x) except where
+//   the significand of s is all ones (there the step's tie goes the wrong way);
 //
 //   division n / d by such a reciprocal: q0 = n*y, q = q0 + (n - d*q0)*y (Markstein, IBM J.
 //   Res. Dev. 34(1), 1990: one remainder correction is enough when y is the correctly
@@ -50,7 +52,7 @@ __device__ __forceinline__ void rare_path()
 // A square root and the raw estimate of its reciprocal.
 struct Root {
   float r;  // sqrtf(x) for x = 0, x >= 2^-96 or NaN (NaN for +inf)
-  float y;  // v_rsq_f32(max(x, 2^-96))
+  float y;  // v_rsq_f32(x), or of 2^-96 if x is less (root_pair: 0 below 2^-52)
 };
 
 __device__ __forceinline__ Root root_short(float x)
@@ -76,8 +78,21 @@ __device__ __forceinline__ float sqrt_cr(float x)
   return s;
 }
 
-// The reciprocal of a root r = root_short(x).r from its estimate, for x >= 2^-96; wrong in
-// the last bit where ones_significand(r).
+// The root of a pair's squared distance, for quotients by it (root_rcp).  Below 2^-52 (near) root
+// and estimate are 0: right for x = 0, where a quotient has to be 0 also when the differences are
+// not 0 and their squares underflow, and wrong for the others.
+constexpr uint32_t kRootNear = 0x25800000u;  // 2^-52
+__device__ __forceinline__ bool root_near(float x) { return __float_as_uint(x) < kRootNear; }
+__device__ __forceinline__ Root root_pair(float x)
+{
+  float y = __builtin_amdgcn_rsqf(x);
+  y = root_near(x) ? 0.0f : y;
+  const float s = x * y, h = 0.5f * y;
+  return Root{ __builtin_fmaf(__builtin_fmaf(-s, s, x), h, s), y };
+}
+
+// The reciprocal of a root r = sqrtf(x) from its estimate, for finite x >= 2^-52; wrong in the
+// last bit where ones_significand(r).
 __device__ __forceinline__ float root_rcp(Root q)
 {
   return __builtin_fmaf(__builtin_fmaf(-q.r, q.y, 1.0f), q.y, q.y);

@@ -28,9 +28,9 @@ __device__ __noinline__ float div_general(float n, float d)
   return n / d;
 }
 
-// Every bit pattern x in [lo, hi): sqrt_cr(x) against sqrtf(x), and for finite x >= 2^-52
-// root_rcp against the reciprocal of sqrtf(x) unless its significand is all ones.  first[0]
-// keeps the smallest mismatching pattern.
+// Every bit pattern x in [lo, hi): sqrt_cr(x) against sqrtf(x); for finite x >= 2^-52 also
+// root_pair against it, and root_rcp against its reciprocal unless its significand is all ones;
+// both 0 for x = 0.  first[0] keeps the smallest mismatching pattern.
 __global__ __launch_bounds__(256) void k_check_sqrt(uint32_t lo, uint32_t hi,
                                                     unsigned long long* bad, uint32_t* first)
 {
@@ -39,8 +39,10 @@ __global__ __launch_bounds__(256) void k_check_sqrt(uint32_t lo, uint32_t hi,
   for (uint64_t b = (uint64_t)lo + blockIdx.x * blockDim.x + threadIdx.x; b < hi; b += stride) {
     const float x = __uint_as_float((uint32_t)b);
     const float r = sqrt_general(x);
-    const bool rcp = b >= 0x25800000u && b < 0x7f800000u && !ones_significand(r);
-    if (!same(sqrt_cr(x), r) || (rcp && !same(root_rcp(root_short(x)), div_general(1.0f, r)))) {
+    const Root q = root_pair(x);
+    const bool pair = !root_near(x) && b < 0x7f800000u, rcp = pair && !ones_significand(r);
+    if (!same(sqrt_cr(x), r) || (pair && !same(q.r, r)) || (rcp && !same(root_rcp(q), div_general(1.0f, r))) ||
+        (b == 0u && (q.r != 0.0f || root_rcp(q) != 0.0f))) {
       ++nbad;
       atomicMin(first, (uint32_t)b);
     }

@@ -261,6 +261,28 @@ def test_small_grids_wrap_in_x_and_z_bit_exact(res, n):
 
 
 @pytest.mark.parametrize("quad", [True, False])
+def test_pairs_whose_squared_distance_underflows_bit_exact(quad):
+    """Particles apart by less than 2^-75, as they can be near coordinate 0: the squared distance is
+    0 and the reference's gradient with it, though the differences are not."""
+    rng = np.random.default_rng(7)
+    n = 90
+    box, res = (2.0, 2.0, 2.0), (6, 6, 6)
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :3] = np.float32(0.5) * rng.random((n, 3), dtype=np.float32) - np.float32(0.25)
+    for k, d in enumerate([(1e-24, 0, 0), (2e-23, 0, 0), (0, 0, -1e-24), (1e-30, 0, 2e-23), (1e-38, 0, 1e-40)]):
+        pos[2 * k, 0] = pos[2 * k, 2] = 0.0
+        pos[2 * k + 1, :3] = pos[2 * k, :3] + np.array(d, np.float32)
+    sc = scenes.CloudScene("", box, res, n, 1024, pos, np.zeros_like(pos))
+    gpu, orc = make_pair(sc, iters=2, quad=quad)
+    for step in range(1, 4):
+        gpu.update(1)
+        orc.step(1)
+        log(f"clouds, underflowing pairs, step {step}")
+        compare(gpu, orc, n, f"step {step}")
+    gpu.close()
+
+
+@pytest.mark.parametrize("quad", [True, False])
 def test_infinite_velocity_spreads_nan_bit_exact(quad):
     """One particle with an infinite velocity: its predicted position is infinite, so the
     gradient terms of its neighbours turn NaN and so do the lambda, vorticity and confined

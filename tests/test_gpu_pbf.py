@@ -446,6 +446,30 @@ def test_checked_pairs_in_lists_keep_bits(flags, queue, n):
         gpu.close()
 
 
+@pytest.mark.parametrize("flags", [0, 2, 8, 13, 64, 72])
+@pytest.mark.parametrize("mapping", ["stable", "literal"])
+def test_pairs_whose_squared_distance_underflows(flags, mapping):
+    """Particles apart by less than 2^-75, as they can be near coordinate 0: the squared distance is
+    0 and the reference's gradient with it, though the differences are not; walked and replayed."""
+    rng = np.random.default_rng(7)
+    n = 60
+    pos = np.zeros((n, 4), np.float32)
+    pos[:, :3] = 0.25 * rng.random((n, 3), dtype=np.float32) - np.float32(0.1)
+    for k, d in enumerate([(1e-24, 0, 0), (2e-23, 0, 0), (0, 0, -1e-24), (1e-30, 0, 2e-23), (1e-38, 0, 1e-40)]):
+        pos[2 * k, 0] = pos[2 * k, 2] = 0.0
+        pos[2 * k + 1, :3] = pos[2 * k, :3] + np.array(d, np.float32)
+    sc = scenes.dam_break((4, 4, 4), (4, 2, 2), (40, 20, 20), seed=1)
+    sc.pos, sc.vel, sc.n, sc.max_n = pos, np.zeros_like(pos), n, 1024
+    gpu, orc = make_pbf_pair(sc, iters=2, **sc.params(mapping))
+    gpu.set_tuning(64, flags, 0, 16)
+    for step in range(1, 4):
+        log(f"underflowing pairs, flags {flags}, {mapping}, step {step}")
+        gpu.update(1)
+        orc.step(1)
+        compare_pbf(gpu, orc, sc.n, step)
+    gpu.close()
+
+
 @pytest.mark.parametrize("res", [(2, 2, 2), (5, 3, 2), (4, 2, 3), (3, 4, 5)])
 @pytest.mark.parametrize("flags", [0, 2, 8, 13, 64, 72])
 def test_grids_that_wrap_in_every_column(flags, res):
