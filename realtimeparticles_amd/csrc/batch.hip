@@ -28,6 +28,7 @@ using namespace rtp;
 struct rtp_batch {
   int device = 0;
   hipStream_t stream = nullptr;
+  DevBlock buffers;  // the buffers of creation
   std::vector<SceneHost> scenes;
   uint32_t total = 0;     // particles of all scenes
   uint32_t keySpace = 0;  // cell keys (and cell-table entries) of all scenes
@@ -96,35 +97,11 @@ struct rtp_batch {
   {
     drop_graph();
     prof.destroy();
-    for (int k = 0; k < 2; ++k) {
-      dev_free(pos[k]);
-      dev_free(vel[k]);
-      dev_free(pred[k]);
-      dev_free(key[k]);
-      dev_free(idx[k]);
-    }
-    dev_free(vort);
-    dev_free(velTmp);
-    dev_free(density);
-    dev_free(lambda);
-    dev_free(counts);
-    dev_free(startEnd);
-    dev_free(dSlots);
-    dev_free(dConsts);
-    dev_free(dBlocks);
+    buffers.release();
     dev_free(ckPos);
     dev_free(ckVel);
-    dev_free(okey);
-    dev_free(orank);
-    dev_free(oorder[0]);
-    dev_free(oorder[1]);
-    dev_free(ocount.table[0]);
-    dev_free(ocount.table[1]);
-    dev_free(opart);
     dev_free(nbList);
     dev_free(nbCount);
-    dev_free(cols);
-    dev_free(packed);
     if (stream)
       (void)hipStreamDestroy(stream);
     stream = nullptr;
@@ -392,28 +369,36 @@ int rtp_batch_create(int device, const rtp_batch_scene* sc, uint32_t count, rtp_
   const uint32_t N = h->total;
   // ceil(n / b) * b < n + 256 for every block size b <= 256
   h->nbThreads = N + 255u * (uint32_t)h->scenes.size();
-  if ((rc = dev_alloc(&h->pos[0], N)) || (rc = dev_alloc(&h->pos[1], N)) ||
-      (rc = dev_alloc(&h->vel[0], N)) || (rc = dev_alloc(&h->vel[1], N)) ||
-      (rc = dev_alloc(&h->pred[0], N + kPosPad)) || (rc = dev_alloc(&h->pred[1], N + kPosPad)) ||
-      (rc = dev_alloc(&h->vort, N)) || (rc = dev_alloc(&h->velTmp, N)) ||
-      (rc = dev_alloc(&h->density, N)) || (rc = dev_alloc(&h->lambda, N)) ||
-      (rc = dev_alloc(&h->key[0], N)) || (rc = dev_alloc(&h->key[1], N)) ||
-      (rc = dev_alloc(&h->idx[0], N)) || (rc = dev_alloc(&h->idx[1], N)) ||
-      (rc = dev_alloc(&h->counts, count_capacity(N))) ||
-      (rc = dev_alloc(&h->startEnd, h->keySpace)) || (rc = dev_alloc(&h->cols, h->keySpace)) ||
-      (rc = dev_alloc(&h->packed, N)) ||
-      (rc = dev_alloc(&h->dSlots, count)) || (rc = dev_alloc(&h->dConsts, count)) ||
-      (rc = dev_alloc(&h->dBlocks, maxBlocks)) || (rc = dev_alloc(&h->okey, N)) ||
-      (rc = dev_alloc(&h->orank, N)) || (rc = dev_alloc(&h->oorder[0], N)) ||
-      (rc = dev_alloc(&h->oorder[1], N)) ||
-      (rc = dev_alloc(&h->ocount.table[0], (h->keySpace + 15u) & ~15u)) ||
-      (rc = dev_alloc(&h->ocount.table[1], (h->keySpace + 15u) & ~15u)) ||
-      (rc = dev_alloc(&h->opart, scan_partials_needed((h->keySpace + 15u) & ~15u)))) {
+  const uint32_t orderWords = (h->keySpace + 15u) & ~15u;
+  for (int k = 0; k < 2; ++k) {
+    h->buffers.add(&h->pos[k], N);
+    h->buffers.add(&h->vel[k], N);
+    h->buffers.add(&h->pred[k], N + kPosPad);
+    h->buffers.add(&h->key[k], N);
+    h->buffers.add(&h->idx[k], N);
+    h->buffers.add(&h->oorder[k], N);
+    h->buffers.add(&h->ocount.table[k], orderWords);
+  }
+  h->buffers.add(&h->vort, N);
+  h->buffers.add(&h->velTmp, N);
+  h->buffers.add(&h->density, N);
+  h->buffers.add(&h->lambda, N);
+  h->buffers.add(&h->counts, count_capacity(N));
+  h->buffers.add(&h->startEnd, h->keySpace);
+  h->buffers.add(&h->cols, h->keySpace);
+  h->buffers.add(&h->packed, N);
+  h->buffers.add(&h->dSlots, count);
+  h->buffers.add(&h->dConsts, count);
+  h->buffers.add(&h->dBlocks, maxBlocks);
+  h->buffers.add(&h->okey, N);
+  h->buffers.add(&h->orank, N);
+  h->buffers.add(&h->opart, scan_partials_needed(orderWords));
+  if ((rc = h->buffers.alloc())) {
     h->release();
     delete h;
     return rc;
   }
-  h->ocount.words = (h->keySpace + 15u) & ~15u;
+  h->ocount.words = orderWords;
   if (hipMemset(h->ocount.table[0], 0, sizeof(uint32_t) * h->ocount.words) != hipSuccess ||
       hipMemset(h->ocount.table[1], 0, sizeof(uint32_t) * h->ocount.words) != hipSuccess) {
     h->release();

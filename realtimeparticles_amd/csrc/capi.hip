@@ -216,6 +216,7 @@ struct rtp_mlp {
 struct rtp_fluids {
   int device = 0;
   hipStream_t stream = nullptr;
+  DevBlock buffers;  // the buffers of creation
   GridState grid;
   PbfConsts c{};
   uint32_t n = 0;
@@ -574,17 +575,7 @@ struct rtp_fluids {
       (void)hipStreamSynchronize(stream);
     drop_graph();
     prof.destroy();
-    grid.release();
-    for (int k = 0; k < 2; ++k) {
-      dev_free(pos[k]);
-      dev_free(vel[k]);
-      dev_free(pred[k]);
-    }
-    dev_free(vort);
-    dev_free(velTmp);
-    dev_free(density);
-    dev_free(lambda);
-    dev_free(metric);
+    buffers.release();
     dev_free(ckPos);
     dev_free(ckVel);
     dev_free(ckPred);
@@ -592,26 +583,13 @@ struct rtp_fluids {
     dev_free(ckCol);
     dev_free(ckCam);
     render.release();
-    dev_free(feat);
     dev_free(fb.act);
     dev_free(fb.seeds);
     dev_free(fb.list);
     dev_free(fb.halo);
     dev_free(fb.count);
-    dev_free(lamAcc);
-    dev_free(resDensity);
-    dev_free(resMetric);
-    dev_free(okey);
-    dev_free(orank);
-    dev_free(oorder[0]);
-    dev_free(oorder[1]);
-    dev_free(ocount.table[0]);
-    dev_free(ocount.table[1]);
-    dev_free(opart);
     dev_free(nbList);
     dev_free(nbCount);
-    dev_free(cols);
-    dev_free(packed);
     if (stream)
       (void)hipStreamDestroy(stream);
     stream = nullptr;
@@ -623,6 +601,7 @@ struct rtp_fluids {
 struct rtp_boids {
   int device = 0;
   hipStream_t stream = nullptr;
+  DevBlock buffers;  // the buffers of creation but p_acc, which changes places with accAlt
   GridState grid;
   BoidsConsts c{};
   uint32_t n = 0;
@@ -801,14 +780,9 @@ struct rtp_boids {
     if (stream)
       (void)hipStreamSynchronize(stream);
     prof.destroy();
-    grid.release();
-    for (int k = 0; k < 2; ++k) {
-      dev_free(pos[k]);
-      dev_free(vel[k]);
-    }
+    buffers.release();
     dev_free(acc);
     dev_free(accAlt);
-    dev_free(unitVel);
     dev_free(bar);
     if (barHost)
       (void)hipHostFree(barHost);
@@ -901,26 +875,35 @@ int rtp_fluids_create(const rtp_model_desc* d, rtp_fluids** out)
     return fail(RTP_ERR_HIP, "hipStreamCreate failed");
   }
   const uint32_t maxN = d->maxNbParticles;
-  if ((rc = h->grid.alloc(maxN)) || (rc = dev_alloc(&h->pos[0], maxN)) ||
-      (rc = dev_alloc(&h->pos[1], maxN)) || (rc = dev_alloc(&h->vel[0], maxN)) ||
-      (rc = dev_alloc(&h->vel[1], maxN)) || (rc = dev_alloc(&h->pred[0], maxN + kPosPad)) ||
-      (rc = dev_alloc(&h->pred[1], maxN + kPosPad)) || (rc = dev_alloc(&h->vort, maxN)) ||
-      (rc = dev_alloc(&h->velTmp, maxN)) || (rc = dev_alloc(&h->density, maxN)) ||
-      (rc = dev_alloc(&h->lambda, maxN)) || (rc = dev_alloc(&h->metric, kMetricFloats)) ||
-      (rc = dev_alloc(&h->feat, (size_t)maxN * 8)) ||
-      (rc = dev_alloc(&h->lamAcc, maxN)) || (rc = dev_alloc(&h->resDensity, maxN)) ||
-      (rc = dev_alloc(&h->resMetric, kMetricFloats)) || (rc = dev_alloc(&h->okey, maxN)) ||
-      (rc = dev_alloc(&h->orank, maxN)) || (rc = dev_alloc(&h->oorder[0], maxN)) ||
-      (rc = dev_alloc(&h->oorder[1], maxN)) || (rc = dev_alloc(&h->cols, h->grid.g.numCells)) ||
-      (rc = dev_alloc(&h->packed, maxN)) ||
-      (rc = dev_alloc(&h->ocount.table[0], order_count_words(h->grid.g))) ||
-      (rc = dev_alloc(&h->ocount.table[1], order_count_words(h->grid.g))) ||
-      (rc = dev_alloc(&h->opart, scan_partials_needed(order_count_words(h->grid.g))))) {
+  const uint32_t orderWords = order_count_words(h->grid.g);
+  h->grid.add_to(h->buffers, maxN);
+  for (int k = 0; k < 2; ++k) {
+    h->buffers.add(&h->pos[k], maxN);
+    h->buffers.add(&h->vel[k], maxN);
+    h->buffers.add(&h->pred[k], maxN + kPosPad);
+    h->buffers.add(&h->oorder[k], maxN);
+    h->buffers.add(&h->ocount.table[k], orderWords);
+  }
+  h->buffers.add(&h->vort, maxN);
+  h->buffers.add(&h->velTmp, maxN);
+  h->buffers.add(&h->density, maxN);
+  h->buffers.add(&h->lambda, maxN);
+  h->buffers.add(&h->metric, kMetricFloats);
+  h->buffers.add(&h->feat, (size_t)maxN * 8);
+  h->buffers.add(&h->lamAcc, maxN);
+  h->buffers.add(&h->resDensity, maxN);
+  h->buffers.add(&h->resMetric, kMetricFloats);
+  h->buffers.add(&h->okey, maxN);
+  h->buffers.add(&h->orank, maxN);
+  h->buffers.add(&h->cols, h->grid.g.numCells);
+  h->buffers.add(&h->packed, maxN);
+  h->buffers.add(&h->opart, scan_partials_needed(orderWords));
+  if ((rc = h->buffers.alloc())) {
     h->release();
     delete h;
     return rc;
   }
-  h->ocount.words = order_count_words(h->grid.g);
+  h->ocount.words = orderWords;
   if (hipMemset(h->ocount.table[0], 0, sizeof(uint32_t) * h->ocount.words) != hipSuccess ||
       hipMemset(h->ocount.table[1], 0, sizeof(uint32_t) * h->ocount.words) != hipSuccess) {
     h->release();
@@ -1414,10 +1397,13 @@ int rtp_boids_create(const rtp_model_desc* d, rtp_boids** out)
     return fail(RTP_ERR_HIP, "hipStreamCreate failed");
   }
   const uint32_t maxN = d->maxNbParticles;
-  if ((rc = h->grid.alloc(maxN)) || (rc = dev_alloc(&h->pos[0], maxN + kPosPad)) ||
-      (rc = dev_alloc(&h->pos[1], maxN + kPosPad)) || (rc = dev_alloc(&h->vel[0], maxN)) ||
-      (rc = dev_alloc(&h->vel[1], maxN)) || (rc = dev_alloc(&h->acc, maxN)) ||
-      (rc = dev_alloc(&h->unitVel, maxN))) {
+  h->grid.add_to(h->buffers, maxN);
+  for (int k = 0; k < 2; ++k) {
+    h->buffers.add(&h->pos[k], maxN + kPosPad);
+    h->buffers.add(&h->vel[k], maxN);
+  }
+  h->buffers.add(&h->unitVel, maxN);
+  if ((rc = h->buffers.alloc()) || (rc = dev_alloc(&h->acc, maxN))) {
     h->release();
     delete h;
     return rc;
@@ -2083,9 +2069,10 @@ int rtp_grid_build(const rtp_model_desc* d, const float* pos4, uint32_t* keys, u
   RTP_HIP_TRY(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
   float4* pos = nullptr;
   Profiler prof;
-  rc = G.alloc(maxN);
-  if (!rc)
-    rc = dev_alloc(&pos, maxN);
+  DevBlock block;
+  G.add_to(block, maxN);
+  block.add(&pos, maxN);
+  rc = block.alloc();
   if (!rc)
     rc = upload_f4(pos, pos4, n, maxN, make_float4(INFINITY, INFINITY, INFINITY, 0.0f), s);
   if (!rc) {
@@ -2109,8 +2096,7 @@ int rtp_grid_build(const rtp_model_desc* d, const float* pos4, uint32_t* keys, u
   if (!rc)
     rc = G.read(keys, idx, startEnd, s);
   (void)hipStreamSynchronize(s);
-  G.release();
-  dev_free(pos);
+  block.release();
   prof.destroy();
   (void)hipStreamDestroy(s);
   return rc;

@@ -1477,6 +1477,7 @@ using namespace rtp;
 struct rtp_clouds {
   int device = 0;
   hipStream_t stream = nullptr;
+  DevBlock buffers;  // the buffers of creation
   // the temperature passes run on a second stream beside the density iterations: neither
   // reads what the other writes, until XSPH rewrites the positions the temperature walks
   hipStream_t side = nullptr;
@@ -1488,7 +1489,6 @@ struct rtp_clouds {
   bool paused = false;
   // state: ping-pong partners of the cell sort's gather (the partners hold the same data
   // outside the sorted range); predicted positions also ping-pong between Jacobi iterations
-  float4* posBlock = nullptr;  // pos and pred; kPosPad behind the last, the next behind the others
   float4* pos[2] = {};
   float4* vel[2] = {};
   float4* tot[2] = {};
@@ -1514,29 +1514,7 @@ struct rtp_clouds {
 
   void release()
   {
-    grid.release();
-    dev_free(posBlock);
-    for (int k = 0; k < 2; ++k) {
-      pos[k] = pred[k] = nullptr;
-      dev_free(vel[k]);
-      dev_free(tot[k]);
-      dev_free(temp[k]);
-      dev_free(buoy[k]);
-      dev_free(vapor[k]);
-      dev_free(cloud[k]);
-      dev_free(pid[k]);
-    }
-    dev_free(vort);
-    dev_free(velTmp);
-    dev_free(density);
-    dev_free(lambda);
-    dev_free(lap);
-    dev_free(lambdaT);
-    dev_free(list.entry);
-    dev_free(list.count);
-    dev_free(listT.entry);
-    dev_free(listT.count);
-    dev_free(flags);
+    buffers.release();
     prof.destroy();
     if (fork)
       (void)hipEventDestroy(fork);
@@ -1714,28 +1692,30 @@ int rtp_clouds_create(const rtp_model_desc* d, rtp_clouds** out)
     return fail(RTP_ERR_HIP, "hipStreamCreate failed");
   }
   const uint32_t maxN = d->maxNbParticles;
-  // One allocation for the four position buffers, each 256-byte aligned: with a pad behind each,
-  // a model of 131,072 particles took 3.4 ms to create against 2.9 ms without the pads.
-  const size_t posStride = ((size_t)maxN + 15u) / 16u * 16u;
-  if (!(rc = h->grid.alloc(maxN)))
-    rc = dev_alloc(&h->posBlock, 4u * posStride + kPosPad);
-  for (int k = 0; k < 2 && !rc; ++k) {
-    h->pos[k] = h->posBlock + k * posStride;
-    h->pred[k] = h->posBlock + (2 + k) * posStride;
-    if ((rc = dev_alloc(&h->vel[k], maxN)) || (rc = dev_alloc(&h->tot[k], maxN)) ||
-        (rc = dev_alloc(&h->temp[k], maxN)) || (rc = dev_alloc(&h->buoy[k], maxN)) ||
-        (rc = dev_alloc(&h->vapor[k], maxN)) || (rc = dev_alloc(&h->cloud[k], maxN)) ||
-        (rc = dev_alloc(&h->pid[k], maxN)))
-      break;
+  h->grid.add_to(h->buffers, maxN);
+  for (int k = 0; k < 2; ++k) {
+    h->buffers.add(&h->pos[k], maxN + kPosPad);
+    h->buffers.add(&h->pred[k], maxN + kPosPad);
+    h->buffers.add(&h->vel[k], maxN);
+    h->buffers.add(&h->tot[k], maxN);
+    h->buffers.add(&h->temp[k], maxN);
+    h->buffers.add(&h->buoy[k], maxN);
+    h->buffers.add(&h->vapor[k], maxN);
+    h->buffers.add(&h->cloud[k], maxN);
+    h->buffers.add(&h->pid[k], maxN);
   }
-  if (!rc)
-    (void)((rc = dev_alloc(&h->vort, maxN)) || (rc = dev_alloc(&h->velTmp, maxN)) ||
-           (rc = dev_alloc(&h->density, maxN)) || (rc = dev_alloc(&h->lambda, maxN)) ||
-           (rc = dev_alloc(&h->lap, maxN)) || (rc = dev_alloc(&h->lambdaT, maxN)) ||
-           (rc = dev_alloc(&h->list.entry, (size_t)kCldListCap * maxN)) ||
-           (rc = dev_alloc(&h->list.count, maxN)) || (rc = dev_alloc(&h->flags, kCldFlagWords)) ||
-           (rc = dev_alloc(&h->listT.entry, (size_t)kCldListCap * maxN)) ||
-           (rc = dev_alloc(&h->listT.count, maxN)));
+  h->buffers.add(&h->vort, maxN);
+  h->buffers.add(&h->velTmp, maxN);
+  h->buffers.add(&h->density, maxN);
+  h->buffers.add(&h->lambda, maxN);
+  h->buffers.add(&h->lap, maxN);
+  h->buffers.add(&h->lambdaT, maxN);
+  h->buffers.add(&h->flags, kCldFlagWords);
+  for (CldList* l : { &h->list, &h->listT }) {
+    h->buffers.add(&l->entry, (size_t)kCldListCap * maxN);
+    h->buffers.add(&l->count, maxN);
+  }
+  rc = h->buffers.alloc();
   h->list.stride = maxN;
   h->listT.stride = maxN;
   h->quad = maxN <= kQuadDefaultMaxN;
