@@ -119,8 +119,9 @@ typedef struct {
                                   The default shape of a model of at most 262,144 particles
                                   (maxNbParticles) has it, and a fluids model's also
                                   RTP_LAUNCH_NB_LIST when more than half of the device's
-                                  memory is free as it is created;
-                                  set_tuning / autotune replace it */
+                                  memory is free as it is created and such default lists of
+                                  all models hold at most a 64th of it; set_tuning / autotune
+                                  replace it (and free default lists that they don't use) */
 
 /* Which buffers rtp_fluids_read_field copies. */
 typedef enum {

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -213,6 +214,31 @@ struct rtp_mlp {
 
 // ================================================================================ fluids
 
+namespace {
+// Survivor lists that fluids models hold without a tuning that asked for them, per device.  They
+// are four times a model's other buffers, so all models together hold at most a 64th of the
+// device's memory in them (4.5 of 288 GB: 18 models of 262,144 particles, 140 of 32,768), and a
+// model gets none while less than half of the memory is free; it walks then, with the same bits.
+constexpr int kMaxDevices = 64;
+constexpr size_t kDefaultListShare = 64;
+std::atomic<size_t> g_defaultListBytes[kMaxDevices];
+
+bool take_default_lists(int device, size_t bytes)
+{
+  size_t unused = 0, all = 0;
+  if (device < 0 || device >= kMaxDevices || hipMemGetInfo(&unused, &all) != hipSuccess ||
+      unused <= all / 2u)
+    return false;
+  std::atomic<size_t>& held = g_defaultListBytes[device];
+  if (held.fetch_add(bytes) + bytes <= all / kDefaultListShare)
+    return true;
+  held.fetch_sub(bytes);
+  return false;
+}
+
+void give_back_default_lists(int device, size_t bytes) { g_defaultListBytes[device].fetch_sub(bytes); }
+}  // namespace
+
 struct rtp_fluids {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -251,8 +277,10 @@ struct rtp_fluids {
   CountTables ocount;  // the thread order's count tables
   uint32_t* opart = nullptr;
   // survivor lists (RTP_LAUNCH_NB_LIST), allocated when first enabled
+  DevBlock lists;
   uint4* nbList = nullptr;      // kNbCap / 4 x maxN granules
   uint32_t* nbCount = nullptr;  // maxN
+  size_t defaultBytes = 0;      // of lists that no tuning asked for (take_default_lists)
   uint2* cols = nullptr;        // the one-lane walks' column ranges, one per cell
   float4* packed = nullptr;     // PassOrder::packed, maxN
   float* resDensity = nullptr;
@@ -284,17 +312,19 @@ struct rtp_fluids {
     graphValid = false;
   }
 
-  int alloc_lists()
+  int alloc_lists() { return nbList ? RTP_OK : lists.alloc(); }
+
+  // The default lists are given back, or belong to the tuning that asks for lists from here on.
+  void end_default_lists(bool keep)
   {
-    if (nbList)
-      return RTP_OK;
-    int rc = 0;
-    if ((rc = dev_alloc(&nbList, (size_t)(kNbCap / 4u) * grid.maxN)) ||
-        (rc = dev_alloc(&nbCount, grid.maxN))) {
-      dev_free(nbList);
-      nbList = nullptr;
+    if (defaultBytes == 0)
+      return;
+    if (!keep) {
+      (void)hipStreamSynchronize(stream);
+      lists.release();
     }
-    return rc;
+    give_back_default_lists(device, defaultBytes);
+    defaultBytes = 0;
   }
 
   void refresh_consts()
@@ -588,8 +618,8 @@ struct rtp_fluids {
     dev_free(fb.list);
     dev_free(fb.halo);
     dev_free(fb.count);
-    dev_free(nbList);
-    dev_free(nbCount);
+    end_default_lists(false);
+    lists.release();
     if (stream)
       (void)hipStreamDestroy(stream);
     stream = nullptr;
@@ -910,17 +940,20 @@ int rtp_fluids_create(const rtp_model_desc* d, rtp_fluids** out)
     delete h;
     return fail(RTP_ERR_HIP, "hipMemset failed");
   }
+  h->lists.add(&h->nbList, (size_t)(kNbCap / 4u) * maxN);
+  h->lists.add(&h->nbCount, maxN);
   // The default shape of a small model replays survivor lists (1 KiB per particle, at most
   // 256 MiB), which takes the walk out of half its passes: 131,072 particles with the app's
   // parameters and rendering steps 236 -> 181 us a frame, 8,192 particles 191 -> 155 us until done.
-  // With less than half of the device's memory free it walks: the lists are four times a model's
-  // other buffers, so that half is left to further models' and the program's own.
-  size_t freeBytes = 0, allBytes = 0;
-  if (h->L.quad && hipMemGetInfo(&freeBytes, &allBytes) == hipSuccess && freeBytes > allBytes / 2u)
+  const size_t listBytes = (size_t)maxN * (kNbCap + 1u) * 4u;
+  if (h->L.quad && take_default_lists(h->device, listBytes)) {
+    h->defaultBytes = listBytes;
     h->L.nbList = h->alloc_lists() == RTP_OK ? 1 : 0;
-  if (h->L.quad && !h->L.nbList) {
-    (void)hipGetLastError();
-    fail(RTP_OK, "");
+    if (!h->L.nbList) {
+      h->end_default_lists(false);
+      (void)hipGetLastError();
+      fail(RTP_OK, "");
+    }
   }
   h->refresh_consts();
   // Zero state and the reset key tail, like the constructor's reset() (Fluids.cpp:91).
@@ -1298,11 +1331,11 @@ int rtp_fluids_set_tuning(rtp_fluids* h, const rtp_tuning* t)
   int rc = check_tuning(*t, kFluidsLaunchFlags);
   if (rc)
     return rc;
-  if (t->flags & RTP_LAUNCH_NB_LIST) {
-    RTP_HIP_TRY(hipSetDevice(h->device));
-    if ((rc = h->alloc_lists()))
-      return rc;
-  }
+  const bool lists = (t->flags & RTP_LAUNCH_NB_LIST) != 0;
+  RTP_HIP_TRY(hipSetDevice(h->device));
+  if (lists && (rc = h->alloc_lists()))
+    return rc;
+  h->end_default_lists(lists);
   h->L.block = t->blockSize;
   h->L.xcdRemap = t->flags & RTP_LAUNCH_XCD_MAP;
   h->L.tile = (t->flags & RTP_LAUNCH_LDS_TILES) ? 1 : 0;

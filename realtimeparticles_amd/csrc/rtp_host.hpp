@@ -159,7 +159,12 @@ public:
       *k.p = rc ? nullptr : base + k.at;
     return rc;
   }
-  void release() { dev_free(base); }
+  void release()
+  {
+    dev_free(base);
+    for (const Part& k : parts)
+      *k.p = nullptr;
+  }
 
 private:
   struct Part {

@@ -5,9 +5,11 @@ summation order, so positions, velocities, densities, lambdas, predicted positio
 grid are compared for exact equality after every step.  The bar of the task is 1e-5
 relative over 10 steps; exact equality is stricter.
 """
+import ctypes
 import hashlib
 import json
 import os
+import time
 
 import numpy as np
 import pytest
@@ -539,3 +541,82 @@ def test_bad_state_matches_oracle(flags):
             orc.step(1)
             compare_pbf(gpu, orc, sc.n, step)
         gpu.close()
+
+
+def _hip():
+    """The HIP runtime that the library runs on."""
+    capi.lib()
+    with open("/proc/self/maps") as f:
+        return ctypes.CDLL(next(line.split()[-1] for line in f if "libamdhip64.so" in line))
+
+
+def _memory():
+    """Free and total device memory in bytes."""
+    free, every = ctypes.c_size_t(), ctypes.c_size_t()
+    assert _hip().hipMemGetInfo(ctypes.byref(free), ctypes.byref(every)) == 0
+    return free.value, every.value
+
+
+def _used(make):
+    """A new model and the device memory its creation took."""
+    free = _memory()[0]
+    m = make()
+    return m, free - _memory()[0]
+
+
+def test_default_lists_are_bounded_and_given_back():
+    """The survivor lists of the default shape (1 KiB a particle): freed by a tuning without them and
+    with the model, a 64th of the device's memory at most over all models."""
+    n, lists = 1 << 18, 1 << 28
+
+    def make():
+        return capi.Fluids(n, 1000, (2.0, 1.0, 1.0), (20, 10, 10))
+    m, took = _used(make)
+    assert took > lists
+    free = _memory()[0]
+    m.set_tuning(64, capi.LAUNCH_QUAD, 0, 16)
+    t = time.monotonic()  # freed memory may count as free a little later
+    while _memory()[0] - free < lists and time.monotonic() - t < 2.0:
+        time.sleep(0.01)
+    assert _memory()[0] - free >= lists
+    m.close()
+    models = []
+    while len(models) < 64:
+        m, took = _used(make)
+        models.append(m)
+        if took < lists:
+            break
+    log(f"{len(models) - 1} models with default lists")
+    assert took < lists and 1 < len(models) and (len(models) - 1) * lists <= _memory()[1] // 64
+    models.pop(0).close()
+    m, took = _used(make)
+    assert took > lists
+    for k in models + [m]:
+        k.close()
+
+
+def test_models_created_with_little_memory_free_walk_with_the_same_bits():
+    sc = small_scene(seed=9)
+    sc.max_n = 1 << 17
+    free, every = _memory()
+    if free < 0.6 * every:
+        pytest.skip("another program holds the device's memory")
+
+    def make():
+        m = capi.Fluids(sc.max_n, sc.n, sc.box, sc.res, gravity=sc.gravity)
+        m.set_params(**sc.params("stable"))
+        return m
+    with_lists, took = _used(make)
+    assert took > sc.max_n * 1024
+    hold = ctypes.c_void_p()
+    assert _hip().hipMalloc(ctypes.byref(hold), ctypes.c_size_t(int(free - 0.49 * every))) == 0
+    walks, took = _used(make)
+    assert took < sc.max_n * 1024
+    for m in (with_lists, walks):
+        m.load_state(sc.pos, sc.vel)
+        m.update(3)
+    for a, b in zip(with_lists.read_state(), walks.read_state()):
+        _eq(a, b, "state without lists")
+    with_lists.close()
+    walks.close()
+    assert _hip().hipFree(hold) == 0
