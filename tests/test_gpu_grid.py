@@ -40,11 +40,13 @@ def test_sort_pairs_every_digit_width(n, bits):
     _eq(out, keys[ref], "keys")
 
 
-@pytest.mark.parametrize("n, bits", [(1023, 8), (1024, 9), (1025, 10), ((1 << 18) - 1, 8), ((1 << 18) - 1, 9),
-                                     (1 << 17, 10), ((1 << 17) + 1, 10), (1 << 16, 11), ((1 << 16) + 1, 11)])
+@pytest.mark.parametrize("n, bits", [(1023, 8), (1024, 9), (1025, 10), ((1 << 18) - 1, 8), (1 << 18, 8),
+                                     ((1 << 18) - 1, 9), (1 << 18, 9), (1 << 17, 10), ((1 << 17) + 1, 10),
+                                     (1 << 16, 11), ((1 << 16) + 1, 11)])
 def test_sort_pairs_at_the_row_sum_limits(n, bits):
-    """The largest two-launch passes of each width (512 row words a thread) and the smallest sorts past
-    them; half of the keys in one cell, so one digit's column holds most of the count."""
+    """The largest two-launch passes of each width and the smallest sorts past them: of 8 and 9 bits up to
+    2^18 keys (four keys a lane), of 10 and 11 up to 512 row words a thread; half of the keys in one
+    cell, so one digit's column holds most of the count."""
     log(f"sort_pairs n={n} bits={bits}")
     rng = np.random.default_rng(n + bits)
     keys = rng.integers(0, 1 << (2 * bits), n, dtype=np.uint64).astype(np.uint32)
