@@ -200,7 +200,7 @@ struct rtp_batch {
       RTP_PROF(prof, "pbf_density_lambda", s,
                launch_pbf_density_lambda_batch(nb, pred[in], startEnd, density, lambda, s, rec));
       RTP_PROF(prof, "pbf_correct", s,
-               launch_pbf_correct_batch(cb, pred[in], lambda, startEnd, pred[1 - in], pos[cur], vel[cur],
+               launch_pbf_correct_batch(cb, pred[in], startEnd, pred[1 - in], pos[cur], vel[cur],
                                         (last == kLastVel && !vortOn) ? pos[cur] : nullptr, last, s,
                                         rep));
       in = 1 - in;

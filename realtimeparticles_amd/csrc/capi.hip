@@ -2,10 +2,11 @@
 // hipGraph replay and per-kernel profiling.
 //
 // The launch sequence of one PBF substep (Fluids.cpp:400-471 without rendering):
-//   k_predict -> radix sort (passes x {upsweep, scan, downsweep}) -> k_reorder
+//   k_predict -> radix sort (passes x {rows, scatter_rows} of a short sort, else passes x
+//   {upsweep, scan, downsweep}) -> k_reorder -> [k_columns]
 //   -> iters x {k_density_lambda, k_correct} -> [k_vorticity, k_confinement, k_xsph]
 // and of one boids step (Boids.cpp:323-384):
-//   k_boids_hash -> radix sort -> k_reorder -> k_boids_step
+//   k_boids_hash -> radix sort -> k_reorder -> k_boids_unit_vel -> k_boids_step
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -431,9 +432,9 @@ struct rtp_fluids {
         RTP_PROF(prof, "mlp_warm_start", s, launch_mlp_forward(feat, n, mlp->dev, lambda, s, packed));
       const int last = !lastIt ? kNextIter : (learned ? kLastOnly : kLastVel);
       RTP_PROF(prof, "pbf_correct", s,
-               launch_pbf_correct(pred[in], lambda, G.startEnd, pred[1 - in], pos[cur], vel[cur],
+               launch_pbf_correct(pred[in], G.startEnd, pred[1 - in], pos[cur], vel[cur],
                                   (last == kLastVel && !vortOn) ? pos[cur] : nullptr, n, last, c, L, s,
-                                  replay ? kNbReplay : 0, LearnArgs(), pc));
+                                  replay ? kNbReplay : 0, pc));
       in = 1 - in;
       if ((rc = order_threads()))
         return rc;

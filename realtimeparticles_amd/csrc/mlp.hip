@@ -277,7 +277,7 @@ __global__ __launch_bounds__(64 * kTrainWaves) void k_mlp_train(const float* __r
       db2[u] += dz;
       d2[u] = to_bf16(dz);
     }
-      bf16x4 hT[4];
+    bf16x4 hT[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
       hT[t] = transpose16(h[t], identity);

@@ -1015,16 +1015,13 @@ struct CorrectBody {
 
 template <int MODE>
 __device__ __forceinline__ void correct_body(uint32_t i, const float4* __restrict__ pred,
-                                             const float* __restrict__ lambda,
                                              const uint2* __restrict__ se,
                                              float4* __restrict__ predOut,
                                              const float4* __restrict__ pos,
                                              float4* __restrict__ vel, float4* __restrict__ posOut,
-                                             int last, const PbfConsts& c, const LearnArgs& la,
-                                             const WalkCtx& T, const PassOrder& po)
+                                             int last, const PbfConsts& c, const WalkCtx& T,
+                                             const PassOrder& po)
 {
-  (void)la;
-  (void)lambda;
   const float4 p = pred[i];
   const float ywdq = (c.shortMath & kShortArtDiv) ? rcp_refined(c.wdq) : 0.0f;
   CorrectBody<true> b{ c, T.packed, nullptr, (c.shortMath & kShortSqrtGrad) != 0, T.packed[i].w, ywdq };
@@ -1034,20 +1031,19 @@ __device__ __forceinline__ void correct_body(uint32_t i, const float4* __restric
 
 template <int MODE>
 __global__ __launch_bounds__(256) void k_correct(const float4* __restrict__ pred,
-                                                 const float* __restrict__ lambda,
                                                  const uint2* __restrict__ se,
                                                  float4* __restrict__ predOut,
                                                  const float4* __restrict__ pos,
                                                  float4* __restrict__ vel,
                                                  float4* __restrict__ posOut, uint32_t n,
-                                                 int last, PbfConsts c, int remap, LearnArgs la, uint32_t qdepth,
-                     PassOrder po)
+                                                 int last, PbfConsts c, int remap, uint32_t qdepth,
+                                                 PassOrder po)
 {
   const uint32_t t = particle_index(remap);
   RTP_PLAIN_CTX(qdepth)
   RTP_NB_CTX
   if (t < n)
-    correct_body<MODE>(po.particle(t), pred, lambda, se, predOut, pos, vel, posOut, last, c, la, W, po);
+    correct_body<MODE>(po.particle(t), pred, se, predOut, pos, vel, posOut, last, c, W, po);
 }
 
 // ------------------------------------------------- learned substep: per-particle fallback
@@ -1830,7 +1826,6 @@ __global__ __launch_bounds__(kQuadBlock) void k_density_lambda_q(const float4* _
 // k_correct (MODE 0 or kNbReplay) with a quad per particle.
 template <int NB>
 __global__ __launch_bounds__(kQuadBlock) void k_correct_q(const float4* __restrict__ pred,
-                                                          const float* __restrict__ lambda,
                                                           const uint2* __restrict__ se,
                                                           float4* __restrict__ predOut,
                                                           const float4* __restrict__ pos,
@@ -1937,18 +1932,17 @@ __global__ __launch_bounds__(256) void k_density_lambda_t(const float4* __restri
 
 template <int MODE>
 __global__ __launch_bounds__(256) void k_correct_t(const float4* __restrict__ pred,
-                                                   const float* __restrict__ lambda,
                                                    const uint2* __restrict__ se,
                                                    float4* __restrict__ predOut,
                                                    const float4* __restrict__ pos,
                                                    float4* __restrict__ vel,
                                                    float4* __restrict__ posOut, uint32_t n,
-                                                   int last, PbfConsts c, int remap, LearnArgs la, uint32_t qdepth,
-                     PassOrder po)
+                                                   int last, PbfConsts c, int remap, uint32_t qdepth,
+                                                   PassOrder po)
 {
   RTP_TILED_PROLOGUE
   if (active)
-    correct_body<MODE>(i, pred, lambda, se, predOut, pos, vel, posOut, last, c, la, T, po);
+    correct_body<MODE>(i, pred, se, predOut, pos, vel, posOut, last, c, T, po);
 }
 
 __global__ __launch_bounds__(256) void k_vorticity_t(const float4* __restrict__ pred,
@@ -2082,7 +2076,6 @@ __global__ __launch_bounds__(256) void k_density_lambda_batch(BatchView bv,
 
 template <int NB>
 __global__ __launch_bounds__(256) void k_correct_batch(BatchView bv, const float4* __restrict__ pred,
-                                                       const float* __restrict__ lambda,
                                                        const uint2* __restrict__ se,
                                                        float4* __restrict__ predOut,
                                                        const float4* __restrict__ pos,
@@ -2096,8 +2089,8 @@ __global__ __launch_bounds__(256) void k_correct_batch(BatchView bv, const float
   const uint32_t o = b.slot.pbase;
   RTP_PLAIN_CTX(bv.qdepth)
   RTP_BATCH_NB_CTX
-  correct_body<NB>(b.i, pred + o, lambda + o, se + b.slot.kbase, predOut + o, pos + o, vel + o,
-                  posOut ? posOut + o : nullptr, last, c, LearnArgs(), W, batch_order(bv, b));
+  correct_body<NB>(b.i, pred + o, se + b.slot.kbase, predOut + o, pos + o, vel + o,
+                   posOut ? posOut + o : nullptr, last, c, W, batch_order(bv, b));
 }
 
 __global__ __launch_bounds__(256) void k_update_vel_batch(BatchView bv, const float4* __restrict__ pred,
@@ -2310,10 +2303,10 @@ void launch_pbf_density_lambda(const float4* pred, const uint2* startEnd, float*
 #undef RTP_DL
 }
 
-void launch_pbf_correct(const float4* pred, const float* lambda, const uint2* startEnd,
-                        float4* predOut, const float4* pos, float4* vel, float4* posOut,
-                        uint32_t n, int last, const PbfConsts& c, const Launch& L, hipStream_t s,
-                        int mode, const LearnArgs& la, const PassOrder& po)
+void launch_pbf_correct(const float4* pred, const uint2* startEnd, float4* predOut,
+                        const float4* pos, float4* vel, float4* posOut, uint32_t n, int last,
+                        const PbfConsts& c, const Launch& L, hipStream_t s, int mode,
+                        const PassOrder& po)
 {
   if (n == 0)
     return;
@@ -2321,8 +2314,8 @@ void launch_pbf_correct(const float4* pred, const float* lambda, const uint2* st
     mode &= ~(kNbRecord | kNbReplay);
   if (L.quad && !L.tile && (mode & ~kNbReplay) == 0) {
     hipLaunchKernelGGL(mode ? k_correct_q<kNbReplay> : k_correct_q<0>, quad_grid(n),
-                       dim3(kQuadBlock), 0, s, pred, lambda, startEnd, predOut, pos, vel, posOut,
-                       n, last, c, po);
+                       dim3(kQuadBlock), 0, s, pred, startEnd, predOut, pos, vel, posOut, n, last,
+                       c, po);
     return;
   }
   const dim3 g(blocks_for(n, L.block)), b(L.block);
@@ -2330,11 +2323,11 @@ void launch_pbf_correct(const float4* pred, const float* lambda, const uint2* st
 #define RTP_CO(M)                                                                              \
   case M:                                                                                    \
     if (L.tile)                                                                              \
-      hipLaunchKernelGGL(k_correct_t<M>, g, b, lds, s, pred, lambda, startEnd, predOut, pos,   \
-                         vel, posOut, n, last, c, L.xcdRemap, la, q, po);                    \
+      hipLaunchKernelGGL(k_correct_t<M>, g, b, lds, s, pred, startEnd, predOut, pos, vel,      \
+                         posOut, n, last, c, L.xcdRemap, q, po);                             \
     else                                                                                     \
-      hipLaunchKernelGGL(k_correct<M>, g, b, lds, s, pred, lambda, startEnd, predOut, pos,     \
-                         vel, posOut, n, last, c, L.xcdRemap, la, q, po);                    \
+      hipLaunchKernelGGL(k_correct<M>, g, b, lds, s, pred, startEnd, predOut, pos, vel,        \
+                         posOut, n, last, c, L.xcdRemap, q, po);                             \
     break;
   switch (mode) {
     RTP_CO(0)
@@ -2534,12 +2527,11 @@ void launch_pbf_density_lambda_batch(const BatchView& bv, const float4* pred, co
   RTP_BATCH_LAUNCH(RTP_BATCH_NB(k_density_lambda_batch), pred, startEnd, density, lambda);
 }
 
-void launch_pbf_correct_batch(const BatchView& bv, const float4* pred, const float* lambda,
-                              const uint2* startEnd, float4* predOut, const float4* pos,
-                              float4* vel, float4* posOut, int last, hipStream_t s, int nb)
+void launch_pbf_correct_batch(const BatchView& bv, const float4* pred, const uint2* startEnd,
+                              float4* predOut, const float4* pos, float4* vel, float4* posOut,
+                              int last, hipStream_t s, int nb)
 {
-  RTP_BATCH_LAUNCH(RTP_BATCH_NB(k_correct_batch), pred, lambda, startEnd, predOut, pos, vel, posOut,
-                   last);
+  RTP_BATCH_LAUNCH(RTP_BATCH_NB(k_correct_batch), pred, startEnd, predOut, pos, vel, posOut, last);
 }
 
 void launch_pbf_update_vel_batch(const BatchView& bv, const float4* pred, const float4* pos,

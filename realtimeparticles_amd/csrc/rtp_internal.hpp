@@ -347,9 +347,9 @@ void launch_pbf_predict_batch(const BatchView& bv, const float4* pos, const floa
 void launch_reorder_batch(const BatchView& bv, const ReorderArgs& a, hipStream_t s);
 void launch_pbf_density_lambda_batch(const BatchView& bv, const float4* pred, const uint2* startEnd,
                                      float* density, float* lambda, hipStream_t s, int nb = 0);
-void launch_pbf_correct_batch(const BatchView& bv, const float4* pred, const float* lambda,
-                              const uint2* startEnd, float4* predOut, const float4* pos,
-                              float4* vel, float4* posOut, int last, hipStream_t s, int nb = 0);
+void launch_pbf_correct_batch(const BatchView& bv, const float4* pred, const uint2* startEnd,
+                              float4* predOut, const float4* pos, float4* vel, float4* posOut,
+                              int last, hipStream_t s, int nb = 0);
 void launch_pbf_update_vel_batch(const BatchView& bv, const float4* pred, const float4* pos,
                                  float4* vel, float4* posOut, hipStream_t s);
 void launch_pbf_vorticity_batch(const BatchView& bv, const float4* pred, const uint2* startEnd,
@@ -364,13 +364,13 @@ void launch_pbf_density_lambda(const float4* pred, const uint2* startEnd, float*
                                float* lambda, uint32_t n, const PbfConsts& c, const Launch& L,
                                hipStream_t s, int mode = 0, const LearnArgs& la = LearnArgs(),
                         const PassOrder& po = PassOrder());
-// Constraint correction + correctPosition, then per `last` (LastMode) the next iteration's
-// boundary clamp, or updateVel (+ updatePosition when posOut), or nothing.
-void launch_pbf_correct(const float4* pred, const float* lambda, const uint2* startEnd,
-                        float4* predOut, const float4* pos, float4* vel, float4* posOut,
-                        uint32_t n, int last, const PbfConsts& c, const Launch& L, hipStream_t s,
-                        int mode = 0, const LearnArgs& la = LearnArgs(),
-                        const PassOrder& po = PassOrder());
+// Constraint correction + correctPosition (the lambdas come with the positions,
+// PassOrder::packed), then per `last` (LastMode) the next iteration's boundary clamp, or
+// updateVel (+ updatePosition when posOut), or nothing.
+void launch_pbf_correct(const float4* pred, const uint2* startEnd, float4* predOut,
+                        const float4* pos, float4* vel, float4* posOut, uint32_t n, int last,
+                        const PbfConsts& c, const Launch& L, hipStream_t s, int mode,
+                        const PassOrder& po);
 // The learned substep's per-particle fallback (no reference counterpart).  The set: the
 // particles whose post-correction |rho/rho0 - 1| (resDensity) exceeds tau, and every
 // particle within h of one of them.  The halo: every other particle within h of the set;
