@@ -534,10 +534,11 @@ __global__ __launch_bounds__(256) void k_order_scatter(const uint32_t* __restric
 inline uint32_t blocks_for(uint32_t n, uint32_t b) { return (n + b - 1u) / b; }
 
 // Several buffers in one launch: buffer blockIdx.y, 16 KiB a workgroup (the last, partial granule
-// word by word).  A checkpoint's runtime copies keep the host for 8 us each: with one launch for
-// all a restored substep of 8,192 particles takes 55 us among others, 86 before.  From
-// kCopyRuntimeWords words (1,048,576 positions) on the runtime's copies are faster: 27 us
-// against 29 there, 86 against 135 at 4,194,304 particles.
+// word by word).  A checkpoint's runtime copies keep the host for 8 us each, and a substep of a few
+// thousand particles is bound by the host's enqueueing: with one launch for all, a loop of restores
+// and substeps of 8,192 particles took 55 us a turn, 86 before.  From kCopyRuntimeWords words
+// (1,048,576 positions) on the runtime's copies are faster: 27 us against 29 there, 86 against 135
+// at 4,194,304 particles.
 constexpr uint32_t kCopyGranules = 1024;
 constexpr size_t kCopyRuntimeWords = (size_t)1 << 22;
 __global__ __launch_bounds__(256) void k_copy_buffers(CopyList l)

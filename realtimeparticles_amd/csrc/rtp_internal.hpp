@@ -201,7 +201,7 @@ struct ReorderArgs {
   GridConsts g;
 };
 void launch_reorder(const ReorderArgs& a, hipStream_t s);
-// Whole-buffer device copies of one launch (hipMalloc'd buffers: 16-byte aligned).
+// Whole-buffer device copies of one launch (16-byte aligned buffers).
 struct CopyList {
   static constexpr int kMax = 12;
   void* dst[kMax];
