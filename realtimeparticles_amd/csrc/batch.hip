@@ -63,7 +63,7 @@ struct rtp_batch {
   uint32_t nbThreads = 0;
   uint4* nbList = nullptr;
   uint32_t* nbCount = nullptr;
-  uint2* cols = nullptr;  // the walks' column ranges, laid out like startEnd
+  uint2* cols = nullptr;  // the walks' column ranges, laid out like startEnd (columns_pay)
   uint32_t maxCells = 0;  // of a scene
   float4* packed = nullptr;  // PassOrder::packed
   bool constsDirty = true;
@@ -184,8 +184,9 @@ struct rtp_batch {
     // neighbour passes: threads in the grid's order first, then (resort) by current cell;
     // with lists the density / vorticity passes record survivors and the correction,
     // confinement and XSPH passes replay them
-    RTP_PROF(prof, "pbf_columns", s,
-             launch_pbf_columns_batch(bv, startEnd, cols, (uint32_t)scenes.size(), maxCells, s));
+    if (cols)
+      RTP_PROF(prof, "pbf_columns", s,
+               launch_pbf_columns_batch(bv, startEnd, cols, (uint32_t)scenes.size(), maxCells, s));
     BatchView nb = bv;
     nb.cols = cols;
     nb.packed = packed;
@@ -385,7 +386,8 @@ int rtp_batch_create(int device, const rtp_batch_scene* sc, uint32_t count, rtp_
   h->buffers.add(&h->lambda, N);
   h->buffers.add(&h->counts, count_capacity(N));
   h->buffers.add(&h->startEnd, h->keySpace);
-  h->buffers.add(&h->cols, h->keySpace);
+  if (columns_pay(h->keySpace, N))
+    h->buffers.add(&h->cols, h->keySpace);
   h->buffers.add(&h->packed, N);
   h->buffers.add(&h->dSlots, count);
   h->buffers.add(&h->dConsts, count);

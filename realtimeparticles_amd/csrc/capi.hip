@@ -282,7 +282,7 @@ struct rtp_fluids {
   uint4* nbList = nullptr;      // kNbCap / 4 x maxN granules
   uint32_t* nbCount = nullptr;  // maxN
   size_t defaultBytes = 0;      // of lists that no tuning asked for (take_default_lists)
-  uint2* cols = nullptr;        // the one-lane walks' column ranges, one per cell
+  uint2* cols = nullptr;        // the one-lane walks' column ranges, one per cell (columns_pay)
   float4* packed = nullptr;     // PassOrder::packed, maxN
   float* resDensity = nullptr;
   float* resMetric = nullptr; // max, sum, max compression of the residual pass + partials
@@ -392,7 +392,7 @@ struct rtp_fluids {
     po.packed = packed;
     pc.packed = packed;
     // every pass but the plain solver's quad passes walks with one lane
-    if (n > 0 && (L.quad == 0 || L.tile != 0 || wantFeatures || residualPass)) {
+    if (columns_pay(c.g.numCells, n) && (L.quad == 0 || L.tile != 0 || wantFeatures || residualPass)) {
       RTP_PROF(prof, "pbf_columns", s, launch_pbf_columns(G.startEnd, cols, c.g, s));
       po.cols = cols;
       pc.cols = cols;
@@ -926,7 +926,8 @@ int rtp_fluids_create(const rtp_model_desc* d, rtp_fluids** out)
   h->buffers.add(&h->resMetric, kMetricFloats);
   h->buffers.add(&h->okey, maxN);
   h->buffers.add(&h->orank, maxN);
-  h->buffers.add(&h->cols, h->grid.g.numCells);
+  if (columns_pay(h->grid.g.numCells, maxN))
+    h->buffers.add(&h->cols, h->grid.g.numCells);
   h->buffers.add(&h->packed, maxN);
   h->buffers.add(&h->opart, scan_partials_needed(orderWords));
   if ((rc = h->buffers.alloc())) {

@@ -50,6 +50,28 @@ __device__ __forceinline__ float4 ldn(const float4* __restrict__ pred, uint32_t 
 // The first index of a column without one range (indices are below it).
 constexpr uint32_t kSplitColumn = 0xffffffffu;
 
+// The index range of a column from its three cells, z order: their non-empty ranges as one when
+// back to back, (1, 0) when all are empty, else kSplitColumn first.
+__device__ __forceinline__ uint2 merge_column(const uint2 cells[3])
+{
+  uint2 out = make_uint2(1u, 0u);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const uint2 r = cells[k];
+    if (r.x > r.y)
+      continue;
+    if (out.x == kSplitColumn)
+      continue;
+    if (out.x > out.y)
+      out = r;
+    else if (r.x == out.y + 1u)
+      out.y = r.y;
+    else
+      out = make_uint2(kSplitColumn, 0u);
+  }
+  return out;
+}
+
 // A lane's survivor queue: entries slot[0], slot[64], ... (a wave's lanes side by side, so the
 // entries of one lane lie at constant distances), the next free one at wp.  Candidates are
 // written unconditionally and kept by advancing wp, and the queue is drained whenever a lane has
@@ -221,7 +243,7 @@ struct WalkCtx {
   const float* x = nullptr;
   const float* y = nullptr;
   const float* z = nullptr;
-  const uint2* cols = nullptr;             // the columns' ranges (k_columns)
+  const uint2* cols = nullptr;             // the columns' ranges (k_columns), or null
   float4* packed = nullptr;                // PassOrder::packed
   NbList nb;                               // survivor lists of a kNbRecord / kNbReplay pass
   uint32_t slot = 0;                       // this thread's column in them
@@ -370,8 +392,9 @@ __device__ __forceinline__ void scan_any(uint32_t lo, uint32_t hi, const WalkCtx
 // outer and z inner with periodic wrap (fluids.cl:101-123), each cell from start to end.
 // The three cells of one z-column are one index range whenever their non-empty ranges are back
 // to back (always, unless a cell was capped or the column wraps) -- the same candidates in the
-// same order with one loop instead of three.  k_columns has found that range for every cell;
-// the next column's loads while this one is scanned.
+// same order with one loop instead of three.  k_columns has found that range for every cell, and
+// the next column's loads while this one is scanned; on a grid too large for it (columns_pay) a
+// lane merges its own.
 template <class B, class R>
 __device__ __forceinline__ void walk_cells(const float4 p, const float4* __restrict__ pred,
                                            const uint2* __restrict__ se, const PbfConsts& c, B& b,
@@ -386,14 +409,20 @@ __device__ __forceinline__ void walk_cells(const float4 p, const float4* __restr
   const auto row = [&](int k) {  // of column (k / 3 - 1, k % 3 - 1)
     return (wrap((int32_t)cx + k / 3 - 1, rx) * ry + wrap((int32_t)cy + k % 3 - 1, ry)) * rz;
   };
+  const auto column = [&](int32_t first) {
+    if (T.cols)
+      return T.cols[first + z1];
+    const uint2 cells[3] = { se[first + wrap(z1 - 1, rz)], se[first + z1], se[first + wrap(z1 + 1, rz)] };
+    return merge_column(cells);
+  };
   int32_t at = row(0);
-  uint2 r = T.cols[at + z1];
+  uint2 r = column(at);
   for (int k = 0; k < 9; ++k) {
     const int32_t here = at;
     const uint2 now = r;
     if (k < 8) {
       at = row(k + 1);
-      r = T.cols[at + z1];
+      r = column(at);
     }
     int32_t staged = -1;  // the column's place in the tile, if any
     if (T.on) {
@@ -711,9 +740,8 @@ __global__ __launch_bounds__(256) void k_predict(const float4* __restrict__ pos,
     startEnd[t] = make_uint2(1u, 0u);  // grid.cl:91-96
 }
 
-// The index range of every cell's column -- the cells z - 1, z, z + 1 (periodic) in that order:
-// their non-empty ranges as one when back to back, (1, 0) when all are empty, else kSplitColumn
-// first.  One small launch a substep for its five walks, each of whose threads would load and
+// The index range of every cell's column (merge_column), the cells z - 1, z, z + 1 (periodic) in
+// that order.  One small launch a substep for its five walks, each of whose threads would load and
 // merge 27 ranges (about 60 VALU instructions and three loads a column, 18 and one this way).
 // 4.6 us at 256,000 cells; the walks of 1,048,576 particles: density 196 -> 184 us, vorticity
 // 180 -> 167 us.
@@ -723,22 +751,7 @@ __device__ __forceinline__ void column_body(uint32_t t, const uint2* __restrict_
   const uint32_t rz = (uint32_t)g.res[2], z = t % rz, base = t - z;
   const uint2 cells[3] = { se[base + (z != 0u ? z : rz) - 1u], se[t],
                            se[base + (z + 1u < rz ? z + 1u : 0u)] };
-  uint2 out = make_uint2(1u, 0u);
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const uint2 r = cells[k];
-    if (r.x > r.y)
-      continue;
-    if (out.x == kSplitColumn)
-      continue;
-    if (out.x > out.y)
-      out = r;
-    else if (r.x == out.y + 1u)
-      out.y = r.y;
-    else
-      out = make_uint2(kSplitColumn, 0u);
-  }
-  cols[t] = out;
+  cols[t] = merge_column(cells);
 }
 
 __global__ __launch_bounds__(256) void k_columns(const uint2* __restrict__ se,
@@ -1994,7 +2007,7 @@ __global__ __launch_bounds__(256) void k_xsph_t(const float4* __restrict__ pred,
 // A batched pass's survivor lists: slot = the thread's launch-wide id.
 #define RTP_BATCH_NB_CTX             \
   W.nb = bv.nb;                      \
-  W.cols = bv.cols + b.slot.kbase;   \
+  W.cols = bv.cols ? bv.cols + b.slot.kbase : nullptr; \
   W.packed = bv.packed ? bv.packed + b.slot.pbase : nullptr; \
   W.slot = blockIdx.x * blockDim.x + threadIdx.x;
 

@@ -280,7 +280,7 @@ struct PassOrder {
   uint32_t keyBase = 0;             //   plus this (a batched scene's key base)
   int bricks = 0;                   //   1: brick_key of the cell instead of its index
   NbList nb;
-  const uint2* cols = nullptr;      // the walks' column ranges (launch_pbf_columns)
+  const uint2* cols = nullptr;      // the walks' column ranges (launch_pbf_columns), or null
   // Per particle its position and, in the w lane, the datum the next pass needs of a neighbour:
   // lambda from the density pass for the correction, |vorticity| (when not null then) for the
   // confinement: one 16-byte gather a survivor instead of 12 and 4 bytes from two arrays.
@@ -333,10 +333,16 @@ struct BatchView {
   const uint32_t* order = nullptr;  // batch-wide thread order (scene slices stay in place)
   uint32_t* keyOut = nullptr;       // correction passes: batch-wide key of each output
   NbList nb;                        // survivor lists; a thread's slot is its launch-wide id
-  const uint2* cols = nullptr;      // the walks' column ranges, scene by scene like the cell table
+  const uint2* cols = nullptr;      // the walks' column ranges, scene by scene like the cell table, or null
   float4* packed = nullptr;         // PassOrder::packed of the whole batch
 };
-// The column ranges of the cell table (one per cell) that the one-lane walks read.
+// The column ranges of the cell table (one per cell) that the one-lane walks read, when n particles
+// repay the table: it takes 3.6 us for a million cells from a few millions on, and saves the walks
+// about 45 us a substep and million particles.  A substep of 307,200 particles with lists takes 568
+// us with it and 569 without at 2 million cells, 635 and 578 at 16 million, 1,085 and 701 at 108
+// million; of 1,048,576 particles 1,441 and 1,481 at 2 million, 1,519 and 1,496 at 16 million.
+constexpr uint32_t kColumnCells = 8;
+constexpr bool columns_pay(uint64_t cells, uint64_t n) { return cells <= kColumnCells * n; }
 void launch_pbf_columns(const uint2* startEnd, uint2* cols, const GridConsts& g, hipStream_t s);
 void launch_pbf_columns_batch(const BatchView& bv, const uint2* startEnd, uint2* cols,
                               uint32_t numScenes, uint32_t maxCells, hipStream_t s);

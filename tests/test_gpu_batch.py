@@ -97,6 +97,27 @@ def test_batch_scene_against_oracle():
     b.close()
 
 
+@pytest.mark.parametrize("flags", [0, capi.LAUNCH_RESORT, capi.LAUNCH_RESORT | capi.LAUNCH_NB_LIST])
+def test_sparse_batch_without_a_column_table(flags):
+    """More than eight cells a particle: no column table, the walks merge the columns' cells."""
+    scs = [scenes.dam_break((8, 6, 5 + k), (2.0 + k, 2.0, 1.0), (20 + 10 * k, 20, 10), seed=k, extra=0) for k in range(3)]
+    models = separate_models(scs, 2, "stable")
+    b = make_batch(scs, 2, "stable")
+    b.set_tuning(64, 0, 16, flags)
+    b.enable_profiling(True)
+    for step in range(1, 4):
+        b.update(1)
+        for k, m in enumerate(models):
+            m.update(1)
+            log(f"sparse batch, flags {flags}, step {step}, scene {k}")
+            compare_scene(b, k, m, f"step {step} scene {k}")
+            m.read_state()
+    assert "pbf_columns" not in b.profile()
+    b.close()
+    for m in models:
+        m.close()
+
+
 def test_batch_graph_replay_and_tuning_do_not_change_bits():
     scs = scenes.batch_scenes(count=24, seed=3, n_lo=500, n_hi=6000)
     b = make_batch(scs, 3, "stable")

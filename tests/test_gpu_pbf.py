@@ -499,6 +499,27 @@ def test_grids_that_wrap_in_every_column(flags, res):
     gpu.close()
 
 
+@pytest.mark.parametrize("flags", [0, 2, 8, 13, 29])
+def test_column_table_only_up_to_eight_cells_a_particle(flags):
+    """2,000 particles on 16,000 cells, the most the column table serves, then 1,999, whose one-lane
+    walks merge the columns' cells themselves."""
+    sc = scenes.dam_break((20, 10, 10), (4, 2, 2), (40, 20, 20), seed=3, extra=48)
+    gpu, orc = make_pbf_pair(sc, iters=2, **sc.params("stable"))
+    gpu.set_tuning(64, flags, 0, 16)
+    gpu.enable_profiling(True)
+    for n in (2000, 1999):
+        gpu.set_nb_particles(n)
+        orc.s.n = n
+        gpu.reset_profile()
+        for step in range(1, 4):
+            log(f"column table, n {n}, flags {flags}, step {step}")
+            gpu.update(1)
+            orc.step(1)
+            compare_pbf(gpu, orc, n, step)
+        assert gpu.profile().get("pbf_columns", (0, 0))[0] == (3 if n == 2000 else 0)
+    gpu.close()
+
+
 @pytest.mark.parametrize("box", [(0.2, 0.1, 0.1), (800.0, 400.0, 400.0)])
 def test_general_forms_outside_short_range(box):
     """Effect radius h = 0.005 and h = 20, outside [2^-7, 2^4] where the short correctly
