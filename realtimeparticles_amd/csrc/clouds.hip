@@ -925,7 +925,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_temp_lambda(const float4* __r
                                                          float* __restrict__ lap,
                                                          float* __restrict__ lambdaT, uint32_t n,
                                                          CloudConsts c, CldList list,
-                                                         uint32_t* __restrict__ flags, int)
+                                                         uint32_t* __restrict__ flags)
 {
   const uint32_t i = logical_block(1) * kCldLanes + threadIdx.x;
   if (i >= n)
@@ -1066,7 +1066,7 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_vorticity(const float4* __res
                                                        const float4* __restrict__ vel,
                                                        float4* __restrict__ vort, uint32_t n,
                                                        CloudConsts c, CldList list,
-                                                       uint32_t* __restrict__ flags, int)
+                                                       uint32_t* __restrict__ flags)
 {
   const uint32_t i = logical_block(1) * kCldLanes + threadIdx.x;
   if (i >= n)
@@ -1324,14 +1324,13 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_temp_lambda_q(const float4* _
                                                                  float* __restrict__ lambdaT,
                                                                  uint32_t n, CloudConsts c,
                                                                  CldList list,
-                                                                 uint32_t* __restrict__ flags,
-                                                                 int useList)
+                                                                 uint32_t* __restrict__ flags)
 {
   RTP_CQ_PROLOGUE
   const float4 pos = posP[i];
   CqTempLambda b{ c, tempP, tempP[i], c.q.restDensity };
   cq_neighbours<kCqRecord>(on, i, true, pos, posP, se, c.f.g, list, lds, b,
-                           !useList || flags[kCldTempWord] != 0u);
+                           flags[kCldTempWord] != 0u);
   float lt = 0.0f;
   if (lead)
     lt = cld_temp_lambda_out(i, b.laplacian, b.sumGradCi, b.sumSqGradC, lap, lambdaT, c);
@@ -1401,13 +1400,14 @@ __global__ __launch_bounds__(kCldLanes) void k_cld_vorticity_q(const float4* __r
                                                                const float4* __restrict__ vel,
                                                                float4* __restrict__ vort, uint32_t n,
                                                                CloudConsts c, CldList list,
-                                                               uint32_t* __restrict__ flags, int useList)
+                                                               uint32_t* __restrict__ flags)
 {
   RTP_CQ_PROLOGUE
   const float4 pos = pred[i];
-  // the velocities of this step's particles are finite: the velocity update clamped them
+  // the velocities of the first n particles, which all cell ranges lie in, are finite: the
+  // velocity update clamped them
   CqVorticity b{ c, vel, vel[i] };
-  cq_neighbours<kCqRecord>(on, i, true, pos, pred, se, c.f.g, list, lds, b, !useList);
+  cq_neighbours<kCqRecord>(on, i, true, pos, pred, se, c.f.g, list, lds, b);
   if (lead)
     vort[i] = b.w;
   cld_flag(!lead | cld_safe(b.w), flags, kFlagVort);
@@ -1587,7 +1587,7 @@ struct rtp_clouds {
       RTP_HIP_TRY(hipStreamWaitEvent(t, fork, 0));
       RTP_PROF(prof, "cld_temp_lambda", t,
                hipLaunchKernelGGL(qd ? k_cld_temp_lambda_q : k_cld_temp_lambda, dim3(bw), dim3(kCldLanes), 0, t, pos[cur], temp[cur],
-                                  G.startEnd, lap, lambdaT, n, c, listT, flags, useList));
+                                  G.startEnd, lap, lambdaT, n, c, listT, flags));
       RTP_PROF(prof, "cld_temp_correct", t,
                hipLaunchKernelGGL(qd ? k_cld_temp_correct_q : k_cld_temp_correct, dim3(bw), dim3(kCldLanes), 0, t, pos[cur], lambdaT,
                                   G.startEnd, temp[cur], n, c, listT, flags, useList));
@@ -1618,7 +1618,7 @@ struct rtp_clouds {
     if (c.f.p.isVorticityConfEnabled) {
       RTP_PROF(prof, "cld_vorticity", s,
                hipLaunchKernelGGL(qd ? k_cld_vorticity_q : k_cld_vorticity, dim3(bw), dim3(kCldLanes), 0, s, pred[pc], G.startEnd,
-                                  vel[cur], vort, n, c, list, flags, useList));
+                                  vel[cur], vort, n, c, list, flags));
       RTP_PROF(prof, "cld_confinement", s,
                hipLaunchKernelGGL(qd ? k_cld_confinement_q : k_cld_confinement, dim3(bw), dim3(kCldLanes), 0, s, pred[pc],
                                   G.startEnd, vort, vel[cur], velTmp, n, c, list, flags, useList));
