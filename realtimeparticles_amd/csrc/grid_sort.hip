@@ -392,6 +392,16 @@ __global__ __launch_bounds__(256) void k_reorder_batch(ReorderArgs a, BatchView 
   reorder_body(i, l, sc.kbase, o);
 }
 
+__global__ __launch_bounds__(kSmallThreads) void k_sort_small(uint32_t* __restrict__ keyA,
+                                                              uint32_t* __restrict__ keyB,
+                                                              uint32_t* __restrict__ idxA,
+                                                              uint32_t* __restrict__ idxB, uint32_t n,
+                                                              int passes)
+{
+  __shared__ SmallSortLds lds;
+  small_sort_block<8>(keyA, keyB, idxA, idxB, n, passes, lds);
+}
+
 // A sort whose column sums are short -- kRowLoads row words a thread or fewer, with four keys a
 // lane -- takes two launches a pass: the scan's launches cost more than every workgroup's
 // own sums.  A pass took (upsweep, scan launches, downsweep; now) 10.2 (8.3) us at 8,192 keys of
@@ -637,11 +647,22 @@ int small_sort_pass_count(const SortPlan& p)
   return (p.n <= kSmallSortMax && small_sort_fits()) ? small_sort_passes(p) : 0;
 }
 
+// sort_pairs takes one workgroup and one launch up to kSmallSortFaster keys when their passes are
+// three or more, as rtp_sort_pairs has of wide keys: on the device it takes as long as their six
+// launches or more (a 4-bit pass 3 us at 500 keys, 4.5 at 4,000; two launches 4.7 and 6.7), but a
+// call that waits for the sort took 121 to 143 us with one launch and 153 to 165 with six.
+constexpr uint32_t kSmallSortFaster = 4096;  // eight keys a thread
+
+static bool use_small_sort(const SortPlan& p)
+{
+  return p.n <= kSmallSortFaster && p.passes >= 3 && small_sort_fits();
+}
+
 bool sort_result_in_b(const SortPlan& p)
 {
   if (p.n == 0)
     return false;
-  return (p.passes & 1) != 0;
+  return ((use_small_sort(p) ? small_sort_passes(p) : p.passes) & 1) != 0;
 }
 
 int sort_pairs(const SortPlan& p, uint32_t* keyA, uint32_t* keyB, uint32_t* idxA, uint32_t* idxB,
@@ -650,6 +671,12 @@ int sort_pairs(const SortPlan& p, uint32_t* keyA, uint32_t* keyB, uint32_t* idxA
   *resultInB = false;
   if (p.n == 0)
     return RTP_OK;
+  if (use_small_sort(p)) {  // one workgroup, all passes in LDS
+    const int passes = small_sort_passes(p);
+    hipLaunchKernelGGL(k_sort_small, dim3(1), dim3(kSmallThreads), 0, s, keyA, keyB, idxA, idxB, p.n, passes);
+    *resultInB = (passes & 1) != 0;
+    return RTP_OK;
+  }
   uint32_t *kin = keyA, *kout = keyB, *iin = idxA, *iout = idxB;
   bool inB = false;
   for (int pass = 0; pass < p.passes; ++pass) {

@@ -136,7 +136,7 @@ struct SortPlan {
   size_t countWords = 0;   // radix * subtiles
   int keyBits = 0;         // significant bits of the largest key
 };
-// The one-workgroup LDS sort of the persistent boids update takes at most this many keys.
+// The one-workgroup LDS sort takes at most this many keys.
 constexpr uint32_t kSmallSortMax = 8192;
 constexpr int kSortItems = 32;  // keys per lane of a subtile, for 2^22 keys and more
 // Keys per lane of a subtile for a sort of n keys: smaller subtiles below 2^22 keys, so a

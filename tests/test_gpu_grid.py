@@ -57,6 +57,21 @@ def test_sort_pairs_at_the_row_sum_limits(n, bits):
     _eq(out, keys[ref], "keys")
 
 
+@pytest.mark.parametrize("n", [1, 511, 4095, 4096, 4097])
+@pytest.mark.parametrize("bits", [18, 19, 28, 32])
+def test_sort_pairs_of_wide_keys_in_one_workgroup(n, bits):
+    """Up to 4,096 keys of three passes or more (over 18 bits) sort in one workgroup, an odd number of
+    4-bit passes (19 bits) or an even one; narrower keys and 4,097 in launches of their own."""
+    log(f"sort_pairs n={n}, {bits}-bit keys")
+    rng = np.random.default_rng(n + bits)
+    keys = rng.integers(0, 1 << bits, n, dtype=np.uint64).astype(np.uint32)
+    keys[::3] = keys[0]
+    out, perm = capi.sort_pairs(keys, max_key=(1 << bits) - 1)
+    ref = np.argsort(keys, kind="stable")
+    _eq(perm, ref.astype(np.uint32), "perm")
+    _eq(out, keys[ref], "keys")
+
+
 def test_sort_pairs_nearly_sorted_input():
     # the next step's keys are the previous order with a few cells changed
     rng = np.random.default_rng(4)
